@@ -6,6 +6,7 @@
 #include "internal.h"
 #include "mfma_pipe.h"
 #include "w4pk.h"
+#include "w4skinny.h"
 
 #include <type_traits>
 
@@ -653,6 +654,150 @@ __global__ __launch_bounds__(GateUpPk::NT, 2) void moe_down_pk_kernel(
   store_down<T>(acc, m0, n0, H, sorted, R, out + part * part_stride, ldo);
 }
 
+// ---- few routes per expert -----------------------------------------------------
+// Gate/up and down for experts of a handful to 64 routes (decode batches), on
+// the weight-streaming core of w4skinny.h: 16 TB-row blocks; a wave's NB blocks
+// of 16 weight rows are half gate and half up rows of the same features. Bound
+// by the stream of expert weights. The 128-row packed core copies 128 token
+// rows per stage whatever the block holds, twice the bytes of the weights, in
+// 32-byte pieces. E = 8, top-2, H = 4096, F = 14336, whole layer on one box:
+// T = 1 110 -> 67 us, 16 270 -> 172 us (gate/up 165 -> 102, 4.8 TB/s; down
+// 98 -> 66), 40 280 -> 189, 100 290 -> 232, 160 315 -> 262 us. At 16 rows two
+// blocks per wave beat four (186 vs 204 us: 1.2 rounds of workgroups against
+// 2.3); non-temporal weight loads took 205 us.
+template <int TB>
+struct SkinnyCfg {
+  static constexpr int NB = TB == 1 ? 2 : 4;  // 16-row blocks per wave: half gate, half up
+  static constexpr int FT = 32 * NB;           // features of a gate/up workgroup
+  static constexpr int CT = 64 * NB;           // columns of a down workgroup
+  static constexpr int HS = TB <= 2 ? 2 : 1;   // 64 rows of 256 k would leave one workgroup per CU
+  static constexpr int D = TB <= 2 ? 2 : 3;    // stages in flight
+  static constexpr int lds(int groups) { return sk::lds_bytes<NB, TB, HS>(groups); }
+};
+
+template <int TB, class WRow, class TRow>
+INTENT_DEVICE void skinny_mainloop(char* lds, const void* x, const TRow& trow, const sk::W4Src& w, const WRow& wrow,
+                                   int nh, int used, f32x4 (&acc)[SkinnyCfg<TB>::NB][TB]) {
+  using C = SkinnyCfg<TB>;
+  if constexpr (TB == 1) {
+    sk::w4_mainloop<C::NB, TB, 1, C::HS, C::D>(lds, x, trow, w, wrow, nh, acc);
+  } else if constexpr (TB == 2) {
+    if (used <= 1)
+      sk::w4_mainloop<C::NB, TB, 1, C::HS, C::D>(lds, x, trow, w, wrow, nh, acc);
+    else
+      sk::w4_mainloop<C::NB, TB, 2, C::HS, C::D>(lds, x, trow, w, wrow, nh, acc);
+  } else {
+    if (used <= 2)
+      sk::w4_mainloop<C::NB, TB, 2, C::HS, C::D>(lds, x, trow, w, wrow, nh, acc);
+    else if (used == 3)
+      sk::w4_mainloop<C::NB, TB, 3, C::HS, C::D>(lds, x, trow, w, wrow, nh, acc);
+    else
+      sk::w4_mainloop<C::NB, TB, 4, C::HS, C::D>(lds, x, trow, w, wrow, nh, acc);
+  }
+}
+
+// 16-row blocks of the aligned rows m0 .. that hold a route (padding rows,
+// sentinel R, sit at the end of an expert's last block).
+template <int TB>
+INTENT_DEVICE int skinny_used(const int32_t* __restrict__ sorted, int m0, int R) {
+  int u = 0;
+#pragma unroll
+  for (int t = 0; t < TB; ++t) u += sorted[m0 + 16 * t] < R ? 1 : 0;
+  return __builtin_amdgcn_readfirstlane(u);
+}
+
+template <int TB>
+__global__ __launch_bounds__(sk::kThreads, 2) void moe_gate_up_skinny_kernel(
+    const f16* __restrict__ x, int64_t ldx, int H, const int32_t* __restrict__ sorted,
+    const int32_t* __restrict__ blocks, int mblocks, int R, int top_k, const uint8_t* __restrict__ wq,
+    const f16* __restrict__ ws, const uint8_t* __restrict__ wz, int F, int gs, sk::GroupDiv div, int vec,
+    f16* __restrict__ act, int64_t ld_act) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  // Row block outermost: the blocks past the last expert's exit at once, and
+  // interleaved with the working ones they would leave CUs idle (the dispatcher
+  // places workgroups by position).
+  const int ctiles = (int)gridDim.x / mblocks;
+  const int mb = blockIdx.x / ctiles, ct = blockIdx.x % ctiles;
+  const int e = blocks[mb];
+  if (e < 0) return;
+  const int m0 = mb * 16 * TB;
+  using C = SkinnyCfg<TB>;
+  constexpr int NB = C::NB;
+  const int f0 = ct * C::FT;
+  const int64_t ldq = H / 2, ldp = H / gs;
+  const GateUpRowMap<mp::Tile<128, 64 * NB, 1, 4>> rows{f0, F};
+  const mp::GatherRows trows{x, ldx * 2, sorted, R, top_k};
+  const sk::W4Src w{wq + (int64_t)e * 2 * F * ldq, ldq, ws + (int64_t)e * 2 * F * ldp, wz + (int64_t)e * 2 * F * ldp,
+                    ldp, (int)ldp, vec != 0, div};
+  f32x4 acc[NB][TB];
+  const int used = skinny_used<TB>(sorted, m0, R);
+  skinny_mainloop<TB>(lds, x, [&](int p) { return trows.off(m0, p); }, w, rows, H / 128, used, acc);
+
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int t = 0; t < TB; ++t) {
+    if (t >= used) break;
+    const int row = m0 + 16 * t + (lane & 15);
+    const bool valid = sorted[row] < R;
+#pragma unroll
+    for (int b = 0; b < NB / 2; ++b) {
+      const int f = f0 + wave * 8 * NB + b * 16 + 4 * (lane >> 4);
+      float o[4];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) o[c] = valid ? silu_mul(acc[b][t][c], acc[b + NB / 2][t][c]) : 0.f;
+      const f16x2 lo = __builtin_convertvector(f32x2{o[0], o[1]}, f16x2);
+      const f16x2 hi = __builtin_convertvector(f32x2{o[2], o[3]}, f16x2);
+      if (f + 3 < F)
+        *reinterpret_cast<u32x2*>(act + (int64_t)row * ld_act + f) =
+            u32x2{bit_cast<uint32_t>(lo), bit_cast<uint32_t>(hi)};
+    }
+  }
+}
+
+// K (= F) is split into `splits` runs of whole units of `unit` k (run p:
+// units p * n / splits ..), each a partial f32 result that the combine adds in order.
+template <int TB>
+__global__ __launch_bounds__(sk::kThreads, 2) void moe_down_skinny_kernel(
+    const f16* __restrict__ act, int64_t ld_act, const int32_t* __restrict__ sorted,
+    const int32_t* __restrict__ blocks, int mblocks, int ntiles, int R, const uint8_t* __restrict__ wq,
+    const f16* __restrict__ ws, const uint8_t* __restrict__ wz, int H, int F, int gs, sk::GroupDiv div, int vec,
+    int unit, int splits, float* __restrict__ out, int64_t ldo, int64_t part_stride) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  const int mb = blockIdx.x / (ntiles * splits), rest = blockIdx.x % (ntiles * splits);
+  const int ct = rest % ntiles, part = rest / ntiles;
+  const int e = blocks[mb];
+  if (e < 0) return;
+  const int m0 = mb * 16 * TB;
+  constexpr int NB = SkinnyCfg<TB>::NB;
+  const int n0 = ct * SkinnyCfg<TB>::CT;
+  const int units = F / unit;
+  const int k0 = part * units / splits * unit, k1 = (part + 1) * units / splits * unit;
+  const int64_t ldq = F / 2, ldp = F / gs;
+  const int groups = splits == 1 ? (int)ldp : (k1 - k0) / gs;
+  const int64_t g0 = splits == 1 ? 0 : k0 / gs;
+  const sk::W4Src w{wq + (int64_t)e * H * ldq + k0 / 2, ldq, ws + (int64_t)e * H * ldp + g0,
+                    wz + (int64_t)e * H * ldp + g0, ldp, groups, vec != 0 && g0 % 4 == 0 && groups % 4 == 0, div};
+  const ClampRows rows{n0, H};
+  f32x4 acc[NB][TB];
+  const int used = skinny_used<TB>(sorted, m0, R);
+  skinny_mainloop<TB>(lds, act + (int64_t)m0 * ld_act + k0, [&](int p) { return (uint32_t)(p * ld_act * 2); }, w, rows,
+                      (k1 - k0) / 128, used, acc);
+
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  float* dst = out + part * part_stride;
+#pragma unroll
+  for (int t = 0; t < TB; ++t) {
+    if (t >= used) break;
+    const int r = sorted[m0 + 16 * t + (lane & 15)];
+    if (r >= R) continue;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      const int col = n0 + wave * 16 * NB + b * 16 + 4 * (lane >> 4);
+      if (col + 3 < H) *reinterpret_cast<f32x4*>(dst + (int64_t)r * ldo + col) = acc[b][t];
+    }
+  }
+}
+
 // y[t, d] += w[t, s] * out[t*k + s, d], slot by slot (mul then add, no fma).
 // With splits > 1 the route's output is the in-order sum of its K parts
 // (part p at route_out + p * part_stride).
@@ -1098,6 +1243,92 @@ size_t composite_workspace(int64_t T, int64_t top_k, int64_t E, int64_t H, int64
   return big > base ? big : base;
 }
 
+// Row block of the weight-streaming kernels (moe_*_skinny_kernel) for experts
+// of R / E routes on average, or 0: the 128- and 160-row tiles. A block holds
+// up to three times the average, so that few experts need a second pass over
+// their weights; from 44 on many overflow 64 rows (E = 8, H = 4096, F = 14336,
+// average 50: 285 vs 321 us, 64: 379 vs 345 us; E = 32, H = 2048, F = 1408,
+// average 50: 120 vs 115 us for the 128-row tiles).
+int64_t skinny_block(int64_t R, int64_t E) {
+  if (R <= 5 * E) return 16;
+  if (R <= 18 * E) return 32;
+  if (R <= 44 * E) return 64;
+  return 0;
+}
+
+struct SkinnyPlan {
+  int64_t block;       // 0: not taken
+  int splits, unit;    // down projection: K parts of whole units of `unit` k
+  int up_lds, down_lds;
+};
+
+// Taken when both projections have whole 128-k steps of 16-byte aligned rows,
+// groups of whole 32 k, and group parameters that fit LDS beside the token
+// stages with two workgroups per CU.
+SkinnyPlan skinny_plan(const void* x, int64_t T, int64_t top_k, int64_t E, int64_t H, int64_t F, int64_t gs,
+                       const uint8_t* wgu, const uint8_t* wd) {
+  SkinnyPlan p{};
+  const int64_t block = skinny_block(T * top_k, E);
+  if (block == 0 || H % 128 != 0 || F % 128 != 0 || gs % 32 != 0 || H % gs != 0 || F % gs != 0 ||
+      !intent::aligned16(x) || !intent::aligned16(wgu) || !intent::aligned16(wd) || !intent::fits_offset(2 * F, H / 2) ||
+      !intent::fits_offset(H, F / 2) || !intent::fits_offset(T, H * 2) || H / 32 >= 65536 || F / 32 >= 65536)
+    return p;
+  // units of whole 128-k steps and groups; of four groups where that divides F (vector parameter loads)
+  int64_t unit = gs % 128 == 0 ? gs : 128 % gs == 0 ? 128 : F;
+  if (F % (4 * unit) == 0) unit *= 4;
+  const int64_t units = F / unit;
+  const int splits = units >= 4 ? 4 : units >= 2 ? 2 : 1;
+  const int64_t longest = (units + splits - 1) / splits * unit;
+  const auto lds = [&](int groups) {
+    return block == 16 ? SkinnyCfg<1>::lds(groups) : block == 32 ? SkinnyCfg<2>::lds(groups) : SkinnyCfg<4>::lds(groups);
+  };
+  if (H / gs > 256 || longest / gs > 256) return p;
+  p.up_lds = lds((int)(H / gs));
+  p.down_lds = lds((int)(longest / gs));
+  if (p.up_lds > 81920 || p.down_lds > 81920) return p;
+  p.block = block;
+  p.splits = splits;
+  p.unit = (int)unit;
+  return p;
+}
+
+int skinny_lds(const void* kernel, int bytes) {
+  if (bytes <= 65536) return INTENT_OK;
+  const hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  INTENT_REQUIRE(e == hipSuccess, INTENT_ERR_LAUNCH, "moe: %d bytes of LDS refused (%s)", bytes, hipGetErrorString(e));
+  return INTENT_OK;
+}
+
+template <int TB>
+int skinny_launch(const SkinnyPlan& p, const void* x, int64_t H, const int32_t* sorted, const int32_t* blocks,
+                  int64_t nblocks, int64_t R, int64_t top_k, const uint8_t* wgu, const void* sgu, const uint8_t* zgu,
+                  const uint8_t* wd, const void* sd, const uint8_t* zd, int64_t F, int64_t gs, void* act, float* out,
+                  void* stream) {
+  const sk::GroupDiv div = sk::group_div(gs);
+  // vector parameter loads: 4-group runs, 8-byte aligned scales and 4-byte aligned zeros
+  const auto vec = [&](const void* s, const uint8_t* z, int64_t ldp) {
+    return ldp % 4 == 0 && (reinterpret_cast<uintptr_t>(s) & 7) == 0 && intent::aligned4(z) ? 1 : 0;
+  };
+  const int64_t up_grid = nblocks * ((F + SkinnyCfg<TB>::FT - 1) / SkinnyCfg<TB>::FT);
+  const int64_t ntiles = (H + SkinnyCfg<TB>::CT - 1) / SkinnyCfg<TB>::CT;
+  const int64_t down_grid = nblocks * ntiles * p.splits;
+  INTENT_REQUIRE(up_grid < (1ll << 31) && down_grid < (1ll << 31), INTENT_ERR_UNSUPPORTED, "grid too large");
+  int st = skinny_lds((const void*)moe_gate_up_skinny_kernel<TB>, p.up_lds);
+  if (st != INTENT_OK) return st;
+  st = skinny_lds((const void*)moe_down_skinny_kernel<TB>, p.down_lds);
+  if (st != INTENT_OK) return st;
+  hipLaunchKernelGGL((moe_gate_up_skinny_kernel<TB>), dim3((unsigned)up_grid), dim3(sk::kThreads), p.up_lds,
+                     (hipStream_t)stream, (const f16*)x, H, (int)H, sorted, blocks, (int)nblocks, (int)R, (int)top_k,
+                     wgu, (const f16*)sgu, zgu, (int)F, (int)gs, div, vec(sgu, zgu, H / gs), (f16*)act, F);
+  st = intent::launch_status("moe_gate_up_skinny");
+  if (st != INTENT_OK) return st;
+  hipLaunchKernelGGL((moe_down_skinny_kernel<TB>), dim3((unsigned)down_grid), dim3(sk::kThreads), p.down_lds,
+                     (hipStream_t)stream, (const f16*)act, F, sorted, blocks, (int)nblocks, (int)ntiles, (int)R, wd,
+                     (const f16*)sd, zd, (int)H, (int)F, (int)gs, div, vec(sd, zd, F / gs), p.unit, p.splits, out, H,
+                     R * H);
+  return intent::launch_status("moe_down_skinny");
+}
+
 }  // namespace
 
 extern "C" size_t intent_moe_workspace_size(int64_t T, int64_t top_k, int64_t E, int64_t H, int64_t F,
@@ -1118,7 +1349,8 @@ extern "C" int intent_moe_expert_ffn_w4(const float* router_logits, const void* 
   INTENT_REQUIRE(group_size > 0, INTENT_ERR_INVALID_ARGUMENT, "group_size must be positive");
   const bool big = composite_wants_pk160(T, top_k, E) && pk160_ok(H, group_size, wgu_scales, wgu_zeros) &&
                    pk160_ok(F, group_size, wd_scales, wd_zeros) && F % (down_splits(F, group_size) * 4 * group_size) == 0;
-  const int64_t B = big ? Pk160::BM : kCompositeBlock;
+  const SkinnyPlan skinny = skinny_plan(x, T, top_k, E, H, F, group_size, wgu_packed, wd_packed);
+  const int64_t B = skinny.block > 0 ? skinny.block : big ? Pk160::BM : kCompositeBlock;
   const MoEWorkspace L = moe_layout(T, top_k, E, H, F, B);
   const size_t need = composite_workspace(T, top_k, E, H, F);
   INTENT_REQUIRE(workspace && workspace_bytes >= need, INTENT_ERR_WORKSPACE, "workspace needs %zu bytes, got %zu", need,
@@ -1138,6 +1370,16 @@ extern "C" int intent_moe_expert_ffn_w4(const float* router_logits, const void* 
   if (st != INTENT_OK) return st;
   st = intent_moe_align(ids, T, top_k, E, B, sorted, L.capacity, blocks, L.nblocks, offsets, total, stream);
   if (st != INTENT_OK) return st;
+  if (skinny.block > 0) {
+    INTENT_REQUIRE(x && wgu_packed && wgu_scales && wgu_zeros && wd_packed && wd_scales && wd_zeros,
+                   INTENT_ERR_INVALID_ARGUMENT, "null pointer argument");
+    const auto launch = B == 16 ? skinny_launch<1> : B == 32 ? skinny_launch<2> : skinny_launch<4>;
+    st = launch(skinny, x, H, sorted, blocks, L.nblocks, T * top_k, top_k, wgu_packed, wgu_scales, wgu_zeros, wd_packed,
+                wd_scales, wd_zeros, F, group_size, act, out, stream);
+    if (st != INTENT_OK) return st;
+    launch_combine(out, H, wts, T, top_k, y, H, H, skinny.splits, T * top_k * H, (hipStream_t)stream);
+    return intent::launch_status("moe_combine");
+  }
   st = intent_moe_gate_up_w4(x, T, H, H, sorted, blocks, L.nblocks, B, top_k, wgu_packed, wgu_scales, wgu_zeros, E, F,
                              group_size, act, F, stream);
   if (st != INTENT_OK) return st;

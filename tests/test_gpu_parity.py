@@ -395,6 +395,25 @@ def test_moe_ffn_many_routes(gpu, threads, T, H, E, k, F, group):
     assert_close_rms(got, ref, what=f"moe ffn many routes T {T} H {H} E {E} F {F} group {group}")
 
 
+# Few routes per expert: the weight-streaming kernels at 16-, 32- and 64-row blocks (R / E up to 5, 18 and
+# 44), with an odd number of 128-k steps, K parts of unequal length, group sizes from one 32-k chunk to a
+# whole row, widths off the workgroup tiles, and (skew) an expert whose routes need several blocks.
+@pytest.mark.parametrize("T,H,E,k,F,group,skew", [
+    (1, 128, 4, 2, 128, 128, 0.0), (7, 384, 8, 2, 1408, 128, 0.0), (16, 640, 8, 2, 640, 64, 0.0),
+    (20, 256, 16, 2, 384, 32, 4.0), (33, 384, 8, 2, 896, 128, 0.0), (60, 256, 8, 2, 2304, 128, 0.0),
+    (50, 512, 8, 2, 512, 256, 6.0), (90, 384, 8, 2, 384, 96, 0.0), (160, 256, 8, 2, 640, 128, 0.0),
+    (100, 640, 8, 3, 768, 32, 3.0), (170, 384, 8, 2, 384, 384, 0.0)])
+def test_moe_ffn_few_routes(gpu, threads, T, H, E, k, F, group, skew):
+    d = moe_small(11 + T, T, H, E, k, F, group=group)
+    d["logits"][:, 1] += skew
+    y0 = np.random.default_rng(2).standard_normal((T, H), dtype=np.float32)
+    got = run_ffn(d, y0)
+    ids, wts = oracle.moe_route(d["logits"], k, True)
+    ref = oracle.moe_ffn_w4(d["x"], ids, wts, d["wgu"], d["sgu"], d["zgu"], d["wd"], d["sd"], d["zd"],
+                            y=y0.copy(), threads=threads)
+    assert_close_rms(got - y0, ref - y0, what=f"moe few routes T {T} H {H} E {E} F {F} group {group}")
+
+
 # More than 64 row blocks of 160 rows (64 experts of ~128 routes): the
 # heavy-first block order of gate/up takes several wave-wide passes.
 def test_moe_ffn_many_blocks(gpu, threads):
