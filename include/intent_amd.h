@@ -75,6 +75,19 @@ int intent_w8a16_matmul(const void* x, int64_t M, int64_t K, int64_t x_ld,
                         const int8_t* w, int64_t N, int64_t w_ld,
                         const void* scales,
                         void* y, int64_t y_ld, void* stream);
+/*
+ * The same product with a workspace: where the tiles of the output leave most
+ * of the GPU idle, K is split over workgroups and the f32 partial sums pass
+ * through it. _workspace_size gives the bytes a call of these extents can use
+ * (0: none); with less, or null, the call runs without a split. 16-byte
+ * aligned, free for reuse when the stream has passed the call.
+ */
+size_t intent_w8a16_matmul_workspace_size(int64_t M, int64_t K, int64_t N);
+int intent_w8a16_matmul_ws(const void* x, int64_t M, int64_t K, int64_t x_ld,
+                           const int8_t* w, int64_t N, int64_t w_ld,
+                           const void* scales,
+                           void* y, int64_t y_ld,
+                           void* workspace, size_t workspace_bytes, void* stream);
 
 /*
  * W4A16 asymmetric group-dequant contraction:
@@ -105,6 +118,14 @@ int intent_w4a16_gemm(const void* x, int64_t M, int64_t K, int64_t x_ld,
                       const void* scales, const uint8_t* zeros, int64_t qparam_ld,
                       int64_t group_size,
                       void* y, int64_t y_ld, void* stream);
+/* The GEMM with a workspace for a K split (see intent_w8a16_matmul_ws). */
+size_t intent_w4a16_gemm_workspace_size(int64_t M, int64_t K, int64_t N, int64_t group_size);
+int intent_w4a16_gemm_ws(const void* x, int64_t M, int64_t K, int64_t x_ld,
+                         const uint8_t* packed, int64_t N, int64_t packed_ld,
+                         const void* scales, const uint8_t* zeros, int64_t qparam_ld,
+                         int64_t group_size,
+                         void* y, int64_t y_ld,
+                         void* workspace, size_t workspace_bytes, void* stream);
 
 /*
  * W8A8: out[m,n] = bf16( f32(acc[m,n]) * a_scale[m] * w_scale[n] ), with

@@ -27,10 +27,13 @@ struct W4Args {
   const uint8_t* z;
   int64_t ldp;
   int gs;
+  // The same rows from column k0 on (a whole number of groups).
+  INTENT_DEVICE W4Args at(int k0) const { return {q + k0 / 2, ldq, s + k0 / gs, z + k0 / gs, ldp, gs}; }
 };
 struct W8Args {
   const int8_t* q;
   int64_t ldq;
+  INTENT_DEVICE W8Args at(int k0) const { return {q + k0, ldq}; }
 };
 
 template <class T, class WArgs>
@@ -44,7 +47,9 @@ struct WeightOp<T, W4Args> {
 };
 // W4 with windowed group parameters (W4Operand kWin): group sizes that are
 // multiples of 64, scale and zero rows in whole dwords.
-struct W4WinArgs : W4Args {};
+struct W4WinArgs : W4Args {
+  INTENT_DEVICE W4WinArgs at(int k0) const { return {W4Args::at(k0)}; }  // k0: whole runs of four groups
+};
 template <class T>
 struct WeightOp<T, W4WinArgs> {
   using Op = mp::W4Operand<T::BN, T::NT, true>;
@@ -58,6 +63,7 @@ struct W4SymArgs {
   int64_t ldq;
   const f16* s;
   int64_t lds;
+  INTENT_DEVICE W4SymArgs at(int k0) const { return {q + (int64_t)(k0 / 8) * ldq, ldq, s + (int64_t)(k0 / 64) * lds, lds}; }
 };
 template <class T>
 struct WeightOp<T, W4SymArgs> {
@@ -786,6 +792,102 @@ __global__ __launch_bounds__(T::NT_WS, 1) void dense_gemm_kernel(const f16* __re
   store_dense<T, kColScale>(acc, m0, n0, M, N, y, ldy, colscale);
 }
 
+// ---- K split over workgroups ----------------------------------------------------
+// Few output tiles leave most CUs without work; blockIdx.y then takes one run
+// of the K stages and writes f32 partial sums, which dense_combine_kernel adds
+// in order. Run p covers units [p n / S, (p + 1) n / S) of `unit` k.
+template <class T, class WArgs>
+__global__ __launch_bounds__(T::NT_WS, 1) void dense_split_kernel(const f16* __restrict__ x, int64_t ldx, int M,
+                                                                  WArgs w, int N, int K, int unit,
+                                                                  float* __restrict__ part, int mblocks) {
+  __shared__ __attribute__((aligned(16))) char buf0[T::STAGE_BYTES];
+  __shared__ __attribute__((aligned(16))) char buf1[T::STAGE_BYTES];
+  char* const bufs[2] = {buf0, buf1};
+  int tmb, tnb;
+  grid_tile(mblocks, 4, tmb, tnb);
+  const int m0 = tmb * T::BM;
+  const int n0 = tnb * T::BN;
+  const int p = blockIdx.y, S = gridDim.y, units = K / unit;
+  const int k0 = (int)((int64_t)p * units / S) * unit, k1 = (int)((int64_t)(p + 1) * units / S) * unit;
+  typename WeightOp<T, WArgs>::Op bop;
+  WeightOp<T, WArgs>::init(bop, w.at(k0), n0, N);
+  f32x16 acc[T::TI][T::TJ];
+  mp::DmaRowsOperand<T::BM, mp::DenseRows, T::NW> aop;
+  aop.init(mp::DenseRows{x + k0, ldx * 2, M}, m0, T::wave() % T::NW);
+  if (!mp::mainloop_ws<T, mp::F16Math, 2>(aop, bop, (k1 - k0) / 64, bufs, acc)) return;
+  // Partial sums keep the register layout: 16 bytes per lane, 1 KB contiguous
+  // per store, block (tile, wave, i, j, g) of run p.
+  constexpr int BLK = T::TI * T::TJ * 4;
+  float* out = part + (((int64_t)p * gridDim.x + blockIdx.x) * T::NW + T::wave()) * (BLK * 256) + (threadIdx.x & 63) * 4;
+#pragma unroll
+  for (int i = 0; i < T::TI; ++i) {
+    if (m0 + T::row(i) >= M) continue;
+#pragma unroll
+    for (int j = 0; j < T::TJ; ++j)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<f32x4*>(out + ((i * T::TJ + j) * 4 + g) * 256) =
+            f32x4{acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
+  }
+}
+
+// y = f16(part 0 + part 1 + .. (* colscale[n])) over the tiles of
+// dense_split_kernel: workgroup (tile, wave) of the split grid, one wave per
+// 32-row block, so that a wave's stores cover 32 rows x 8 bytes of TJ * 4
+// neighbouring pieces.
+template <class T, bool kColScale>
+__global__ __launch_bounds__(64) void dense_combine_kernel(const float* __restrict__ part, int S, int tiles, int M,
+                                                           int N, f16* __restrict__ y, int64_t ldy,
+                                                           const f16* __restrict__ colscale, int vec, int mblocks) {
+  constexpr int BLK = T::TI * T::TJ * 4;
+  // blockIdx.x: ((tile * NW + wave) * TI + i) * TJ + j
+  int id = blockIdx.x;
+  const int j = id % T::TJ;
+  id /= T::TJ;
+  const int i = id % T::TI;
+  id /= T::TI;
+  const int wave = id % T::NW;
+  const int tile = id / T::NW;
+  int tmb, tnb;
+  grouped_tile(xcd_swizzle(tile, tiles), mblocks, tiles / mblocks, 4, tmb, tnb);
+  const int lane = threadIdx.x;
+  const int m = tmb * T::BM + (wave % T::WM) * T::WTM + i * 32 + (lane & 31);
+  const int n0 = tnb * T::BN + (wave / T::WM) * T::WTN + j * 32 + (lane >> 5) * 4;
+  if (m >= M) return;
+  const float* src = part + ((int64_t)tile * T::NW + wave) * (BLK * 256) + (i * T::TJ + j) * 1024 + lane * 4;
+  const int64_t stride = (int64_t)tiles * T::NW * (BLK * 256);
+  f32x4 v[4];
+#pragma unroll
+  for (int g = 0; g < 4; ++g) v[g] = *reinterpret_cast<const f32x4*>(src + g * 256);
+  for (int p = 1; p < S; ++p) {
+    src += stride;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const f32x4 o = *reinterpret_cast<const f32x4*>(src + g * 256);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) v[g][c] += o[c];
+    }
+  }
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    const int n = n0 + g * 8;
+    if constexpr (kColScale) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) v[g][c] *= n + c < N ? (float)colscale[n + c] : 0.f;
+    }
+    f16* dst = y + (int64_t)m * ldy + n;
+    if (vec && n + 3 < N) {
+      *reinterpret_cast<u32x2*>(dst) =
+          u32x2{bit_cast<uint32_t>(__builtin_convertvector(f32x2{v[g][0], v[g][1]}, f16x2)),
+                bit_cast<uint32_t>(__builtin_convertvector(f32x2{v[g][2], v[g][3]}, f16x2))};
+    } else {
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        if (n + c < N) dst[c] = (f16)v[g][c];
+    }
+  }
+}
+
 template <class T, class WArgs, bool kColScale>
 int launch_tile(const f16* x, int64_t ldx, int M, int N, int K, const WArgs& w, f16* y, int64_t ldy,
                 const f16* colscale, hipStream_t st, const char* name) {
@@ -800,17 +902,121 @@ int launch_tile(const f16* x, int64_t ldx, int M, int N, int K, const WArgs& w, 
   return intent::launch_status(name);
 }
 
-// Tiles: 256 x 192 (4 consumer waves of 128 x 96) once M fills it, else
-// 128 x 128 (consumers of 64 x 64); each with 4 producer waves that copy the
-// activations by LDS DMA and decode the weights (mainloop_ws). 192 columns:
-// N = 11008 gives 58 column tiles; with 8 row tiles that is 464 workgroups,
-// 1.8 rounds of 256 CUs (256-wide tiles would give 344, 1.34).
+// Tile and K split of an M x N x K product whose K can be cut at multiples of
+// `unit`. Few tiles leave CUs idle (256 x 192 tiles of M = 512, N = 4096: 44
+// workgroups on 256 CUs), so smaller tiles and K runs are weighed against the
+// stages each workgroup then walks and the partial sums' round trip, in
+// microseconds measured on this kernel: a stage costs a + b L while the L =
+// workgroups / 256 per CU do not exceed one, then (a + b) times the rounds; a
+// split adds 3 us and 0.27 us per MB of partial sums. Fitted to 60 shapes (M
+// 17..2048, N 1024..14336, K 2048..11008, W4): the choice is within 2% of the
+// best of all twelve plans on average. N = K = 4096, M = 77: 36 -> 18 us, 256:
+// 66 -> 23, 512: 66 -> 32, 1024: 68 -> 43 us; K = 11008, M = 256: 166 -> 40 us.
+struct DensePlan {
+  int tile;    // rows of the tile: 256 (256 x 192), 128 (128 x 128), 64 (64 x 128)
+  int splits;  // K runs (1: no workspace)
+};
+constexpr int64_t kMaxSplitBytes = 64 << 20;
+
+int64_t dense_tiles(int64_t M, int64_t N, int tile) {
+  const int64_t bn = tile == 256 ? 192 : 128;
+  return ((M + tile - 1) / tile) * ((N + bn - 1) / bn);
+}
+int64_t dense_split_bytes(const DensePlan& p, int64_t M, int64_t N) {
+  return p.splits > 1 ? p.splits * dense_tiles(M, N, p.tile) * p.tile * (p.tile == 256 ? 192 : 128) * 4 : 0;
+}
+
+// stage_scale: the 64- and 128-row tiles' stage cost relative to the fit (1.1
+// for W4 without windowed group parameters, whose producers load them every stage).
+DensePlan dense_plan(int64_t M, int64_t N, int64_t K, int64_t unit, bool may_split, double stage_scale) {
+  DensePlan best{M > 128 ? 256 : 128, 1};
+  if (dense_tiles(M, N, 256) >= 512) return best;  // two rounds of the large tile: nothing idles
+  const auto cost = [&](const DensePlan& p) {
+    const double a = p.tile == 256 ? 0.95 : p.tile == 128 ? 0.48 : 0.40;
+    const double b = p.tile == 256 ? 0.42 : p.tile == 128 ? 0.14 : 0.05;
+    const double L = (double)(dense_tiles(M, N, p.tile) * p.splits) / 256;
+    const double up = (double)((dense_tiles(M, N, p.tile) * p.splits + 255) / 256);
+    const double stage = (L <= 1 ? a + b * L : (a + b) * (L + up) / 2) * (p.tile == 256 ? 1.0 : stage_scale);
+    const double split = p.splits > 1 ? 3 + 0.27e-6 * (double)dense_split_bytes(p, M, N) : 0;
+    return (p.tile == 64 ? 5 : 4) + (double)K / 64 / p.splits * stage + split;
+  };
+  const double keep = 0.95 * cost(best);  // the plain plan unless another is clearly faster
+  double least = keep;
+  for (int tile = 256; tile >= 64; tile /= 2)
+    for (int splits = 1; splits <= (may_split ? 16 : 1); splits *= 2) {
+      const DensePlan p{tile, splits};
+      if (splits > K / unit || dense_split_bytes(p, M, N) > kMaxSplitBytes) break;
+      const double c = cost(p);
+      if (c < least) {
+        least = c;
+        best = p;
+      }
+    }
+  return best;
+}
+
+// K cuts of a W4 product: whole groups and stages; runs of four groups where
+// they divide K (windowed parameters), W4Cut::win.
+struct W4Cut {
+  int64_t unit;
+  bool win;
+};
+W4Cut w4_cut(int64_t K, int64_t gs) {
+  const bool win = gs % 64 == 0 && K % (4 * gs) == 0;
+  return {win ? 4 * gs : gs % 64 == 0 ? gs : 64, win};
+}
+DensePlan w4_plan(int64_t M, int64_t N, int64_t K, int64_t gs, bool may_split) {
+  const W4Cut c = w4_cut(K, gs);
+  return dense_plan(M, N, K, c.unit, may_split, c.win ? 1.0 : 1.1);
+}
+DensePlan w8_plan(int64_t M, int64_t N, int64_t K, bool may_split) { return dense_plan(M, N, K, 64, may_split, 1.0); }
+
+template <class T, class WArgs, bool kColScale>
+int launch_split(const f16* x, int64_t ldx, int M, int N, int K, const WArgs& w, f16* y, int64_t ldy,
+                 const f16* colscale, int splits, int unit, float* part, hipStream_t st, const char* name) {
+  const int mblocks = (M + T::BM - 1) / T::BM;
+  const int64_t grid = (int64_t)mblocks * ((N + T::BN - 1) / T::BN);
+  const int64_t cgrid = grid * T::NW * T::TI * T::TJ;
+  INTENT_REQUIRE(cgrid < (1ll << 31), INTENT_ERR_UNSUPPORTED, "%s: grid too large", name);
+  INTENT_REQUIRE(intent::fits_offset(M, ldx * 2), INTENT_ERR_UNSUPPORTED,
+                 "%s: activations too large for 31-bit buffer offsets", name);
+  hipLaunchKernelGGL((dense_split_kernel<T, WArgs>), dim3((unsigned)grid, splits), dim3(T::NT_WS), 0, st, x, ldx, M, w,
+                     N, K, unit, part, mblocks);
+  const int s = intent::launch_status(name);
+  if (s != INTENT_OK) return s;
+  const int vec = ldy % 4 == 0 && (reinterpret_cast<uintptr_t>(y) & 7) == 0;
+  hipLaunchKernelGGL((dense_combine_kernel<T, kColScale>), dim3((unsigned)cgrid), dim3(64), 0, st, part, splits,
+                     (int)grid, M, N, y, ldy, colscale, vec, mblocks);
+  return intent::launch_status(name);
+}
+
 template <class WArgs, bool kColScale>
 int launch_dense(const f16* x, int64_t ldx, int M, int N, int K, const WArgs& w, f16* y, int64_t ldy,
-                 const f16* colscale, hipStream_t st, const char* name) {
-  if (M > 128)
+                 const f16* colscale, hipStream_t st, const char* name, const DensePlan& p) {
+  if (p.tile == 256)
     return launch_tile<mp::Tile<256, 192, 2, 2>, WArgs, kColScale>(x, ldx, M, N, K, w, y, ldy, colscale, st, name);
-  return launch_tile<mp::Tile<128, 128, 2, 2>, WArgs, kColScale>(x, ldx, M, N, K, w, y, ldy, colscale, st, name);
+  if (p.tile == 128)
+    return launch_tile<mp::Tile<128, 128, 2, 2>, WArgs, kColScale>(x, ldx, M, N, K, w, y, ldy, colscale, st, name);
+  return launch_tile<mp::Tile<64, 128, 2, 2>, WArgs, kColScale>(x, ldx, M, N, K, w, y, ldy, colscale, st, name);
+}
+
+template <class WArgs, bool kColScale>
+int launch_dense_split(const f16* x, int64_t ldx, int M, int N, int K, const WArgs& w, f16* y, int64_t ldy,
+                       const f16* colscale, hipStream_t st, const char* name, const DensePlan& p, int64_t unit,
+                       float* part) {
+  if (p.tile == 256)
+    return launch_split<mp::Tile<256, 192, 2, 2>, WArgs, kColScale>(x, ldx, M, N, K, w, y, ldy, colscale, p.splits,
+                                                                    (int)unit, part, st, name);
+  if (p.tile == 128)
+    return launch_split<mp::Tile<128, 128, 2, 2>, WArgs, kColScale>(x, ldx, M, N, K, w, y, ldy, colscale, p.splits,
+                                                                    (int)unit, part, st, name);
+  return launch_split<mp::Tile<64, 128, 2, 2>, WArgs, kColScale>(x, ldx, M, N, K, w, y, ldy, colscale, p.splits,
+                                                                 (int)unit, part, st, name);
+}
+
+// A workspace the plan can use: 16-byte aligned and large enough.
+bool split_ready(const DensePlan& p, int64_t M, int64_t N, const void* ws, size_t bytes) {
+  return p.splits > 1 && ws && intent::aligned16(ws) && bytes >= (size_t)dense_split_bytes(p, M, N);
 }
 
 }  // namespace
@@ -835,7 +1041,7 @@ int w8a16_gemv_launch(const void* x, int64_t M, int64_t K, int64_t x_ld, const i
 
 int w4a16_gemm_launch(const void* x, int64_t M, int64_t K, int64_t x_ld, const uint8_t* packed, int64_t N,
                       int64_t packed_ld, const void* scales, const uint8_t* zeros, int64_t qparam_ld, int64_t gs,
-                      void* y, int64_t y_ld, void* stream) {
+                      void* y, int64_t y_ld, void* ws, size_t ws_bytes, void* stream) {
   if (M == 0 || N == 0) return INTENT_OK;
   if (!w4a16_fast(x, K, x_ld, packed, packed_ld, gs) || !(gs == 32 || gs % 64 == 0))
     return w4a16_generic_launch(x, M, K, x_ld, packed, N, packed_ld, scales, zeros, qparam_ld, gs, y, y_ld, stream);
@@ -843,11 +1049,24 @@ int w4a16_gemm_launch(const void* x, int64_t M, int64_t K, int64_t x_ld, const u
                      intent::fits_offset(256 + 1, x_ld * 2),
                  INTENT_ERR_UNSUPPORTED, "w4a16_gemm: operand too large for 31-bit buffer offsets");
   W4Args w{packed, packed_ld, (const f16*)scales, zeros, qparam_ld, (int)gs};
-  if (gs % 64 == 0 && qparam_ld % 4 == 0 && intent::aligned4(scales) && intent::aligned4(zeros) && M > 128)
-    return launch_dense<W4WinArgs, false>((const f16*)x, x_ld, (int)M, (int)N, (int)K, W4WinArgs{w}, (f16*)y, y_ld,
-                                          nullptr, (hipStream_t)stream, "w4a16_gemm");
-  return launch_dense<W4Args, false>((const f16*)x, x_ld, (int)M, (int)N, (int)K, w, (f16*)y, y_ld, nullptr,
-                                       (hipStream_t)stream, "w4a16_gemm");
+  const f16* xx = (const f16*)x;
+  f16* yy = (f16*)y;
+  hipStream_t st = (hipStream_t)stream;
+  const bool win = gs % 64 == 0 && qparam_ld % 4 == 0 && intent::aligned4(scales) && intent::aligned4(zeros);
+  const W4Cut cut = w4_cut(K, gs);
+  const DensePlan split = w4_plan(M, N, K, gs, true);
+  if (split_ready(split, M, N, ws, ws_bytes)) {
+    if (win && cut.win)
+      return launch_dense_split<W4WinArgs, false>(xx, x_ld, (int)M, (int)N, (int)K, W4WinArgs{w}, yy, y_ld, nullptr, st,
+                                                  "w4a16_gemm", split, cut.unit, (float*)ws);
+    return launch_dense_split<W4Args, false>(xx, x_ld, (int)M, (int)N, (int)K, w, yy, y_ld, nullptr, st, "w4a16_gemm",
+                                             split, cut.unit, (float*)ws);
+  }
+  const DensePlan p = w4_plan(M, N, K, gs, false);
+  if (win)
+    return launch_dense<W4WinArgs, false>(xx, x_ld, (int)M, (int)N, (int)K, W4WinArgs{w}, yy, y_ld, nullptr, st,
+                                          "w4a16_gemm", p);
+  return launch_dense<W4Args, false>(xx, x_ld, (int)M, (int)N, (int)K, w, yy, y_ld, nullptr, st, "w4a16_gemm", p);
 }
 
 }  // namespace intent
@@ -915,7 +1134,7 @@ extern "C" int intent_w4a16_matmul(const void* x, int64_t M, int64_t K, int64_t 
     return intent::w4a16_gemv_launch(x, M, K, x_ld, packed, N, packed_ld, scales, zeros, qparam_ld, group_size, y,
                                      y_ld, stream);
   return intent::w4a16_gemm_launch(x, M, K, x_ld, packed, N, packed_ld, scales, zeros, qparam_ld, group_size, y, y_ld,
-                                   stream);
+                                   nullptr, 0, stream);
 }
 
 extern "C" int intent_w4a16_gemv(const void* x, int64_t M, int64_t K, int64_t x_ld, const uint8_t* packed, int64_t N,
@@ -940,11 +1159,31 @@ extern "C" int intent_w4a16_gemm(const void* x, int64_t M, int64_t K, int64_t x_
   int st = intent::w4a16_check(x, M, K, x_ld, packed, N, packed_ld, scales, zeros, qparam_ld, group_size, y, y_ld);
   if (st != INTENT_OK) return st;
   return intent::w4a16_gemm_launch(x, M, K, x_ld, packed, N, packed_ld, scales, zeros, qparam_ld, group_size, y, y_ld,
-                                   stream);
+                                   nullptr, 0, stream);
 }
 
-extern "C" int intent_w8a16_matmul(const void* x, int64_t M, int64_t K, int64_t x_ld, const int8_t* w, int64_t N,
-                                   int64_t w_ld, const void* scales, void* y, int64_t y_ld, void* stream) {
+extern "C" size_t intent_w4a16_gemm_workspace_size(int64_t M, int64_t K, int64_t N, int64_t group_size) {
+  if (M <= 0 || N <= 0 || K <= 0 || K % 128 != 0 || !(group_size == 32 || (group_size > 0 && group_size % 64 == 0)) ||
+      K % group_size != 0)
+    return 0;
+  return (size_t)dense_split_bytes(w4_plan(M, N, K, group_size, true), M, N);
+}
+
+extern "C" int intent_w4a16_gemm_ws(const void* x, int64_t M, int64_t K, int64_t x_ld, const uint8_t* packed, int64_t N,
+                                    int64_t packed_ld, const void* scales, const uint8_t* zeros, int64_t qparam_ld,
+                                    int64_t group_size, void* y, int64_t y_ld, void* workspace, size_t workspace_bytes,
+                                    void* stream) {
+  intent::clear_error();
+  int st = intent::w4a16_check(x, M, K, x_ld, packed, N, packed_ld, scales, zeros, qparam_ld, group_size, y, y_ld);
+  if (st != INTENT_OK) return st;
+  return intent::w4a16_gemm_launch(x, M, K, x_ld, packed, N, packed_ld, scales, zeros, qparam_ld, group_size, y, y_ld,
+                                   workspace, workspace_bytes, stream);
+}
+
+namespace {
+
+int w8a16_launch(const void* x, int64_t M, int64_t K, int64_t x_ld, const int8_t* w, int64_t N, int64_t w_ld,
+                 const void* scales, void* y, int64_t y_ld, void* workspace, size_t workspace_bytes, void* stream) {
   intent::clear_error();
   INTENT_REQUIRE(M >= 0 && N >= 0 && K >= 0, INTENT_ERR_INVALID_ARGUMENT, "negative extent");
   INTENT_REQUIRE(M <= INT32_MAX && N <= INT32_MAX && K <= INT32_MAX, INTENT_ERR_UNSUPPORTED, "extent exceeds int32");
@@ -959,8 +1198,33 @@ extern "C" int intent_w8a16_matmul(const void* x, int64_t M, int64_t K, int64_t 
   INTENT_REQUIRE(intent::fits_offset(N, w_ld) && intent::fits_offset(256 + 1, x_ld * 2), INTENT_ERR_UNSUPPORTED,
                  "w8a16_matmul: operand too large for 31-bit buffer offsets");
   W8Args ws{w, w_ld};
-  return launch_dense<W8Args, true>((const f16*)x, x_ld, (int)M, (int)N, (int)K, ws, (f16*)y, y_ld,
-                                      (const f16*)scales, (hipStream_t)stream, "w8a16_matmul");
+  const f16* xx = (const f16*)x;
+  f16* yy = (f16*)y;
+  hipStream_t st = (hipStream_t)stream;
+  const DensePlan split = w8_plan(M, N, K, true);
+  if (split_ready(split, M, N, workspace, workspace_bytes))
+    return launch_dense_split<W8Args, true>(xx, x_ld, (int)M, (int)N, (int)K, ws, yy, y_ld, (const f16*)scales, st,
+                                            "w8a16_matmul", split, 64, (float*)workspace);
+  return launch_dense<W8Args, true>(xx, x_ld, (int)M, (int)N, (int)K, ws, yy, y_ld, (const f16*)scales, st,
+                                    "w8a16_matmul", w8_plan(M, N, K, false));
+}
+
+}  // namespace
+
+extern "C" int intent_w8a16_matmul(const void* x, int64_t M, int64_t K, int64_t x_ld, const int8_t* w, int64_t N,
+                                   int64_t w_ld, const void* scales, void* y, int64_t y_ld, void* stream) {
+  return w8a16_launch(x, M, K, x_ld, w, N, w_ld, scales, y, y_ld, nullptr, 0, stream);
+}
+
+extern "C" size_t intent_w8a16_matmul_workspace_size(int64_t M, int64_t K, int64_t N) {
+  if (M <= 16 || N <= 0 || K <= 0 || K % 64 != 0) return 0;
+  return (size_t)dense_split_bytes(w8_plan(M, N, K, true), M, N);
+}
+
+extern "C" int intent_w8a16_matmul_ws(const void* x, int64_t M, int64_t K, int64_t x_ld, const int8_t* w, int64_t N,
+                                      int64_t w_ld, const void* scales, void* y, int64_t y_ld, void* workspace,
+                                      size_t workspace_bytes, void* stream) {
+  return w8a16_launch(x, M, K, x_ld, w, N, w_ld, scales, y, y_ld, workspace, workspace_bytes, stream);
 }
 
 extern "C" int intent_fp4_bf16_matmul(const void* x, int64_t M, int64_t K, int64_t x_ld, const uint8_t* packed,
@@ -1251,5 +1515,5 @@ extern "C" int intent_w4a16_sym_gemm(const void* x, int64_t M, int64_t K, int64_
                  INTENT_ERR_UNSUPPORTED, "w4a16_sym_gemm: operand too large for 31-bit buffer offsets");
   W4SymArgs w{packed, packed_ld, (const f16*)scales, scales_ld};
   return launch_dense<W4SymArgs, false>((const f16*)x, x_ld, (int)M, (int)N, (int)K, w, (f16*)y, y_ld, nullptr,
-                                        (hipStream_t)stream, "w4a16_sym_gemm");
+                                        (hipStream_t)stream, "w4a16_sym_gemm", DensePlan{M > 128 ? 256 : 128, 1});
 }

@@ -103,6 +103,17 @@ def _ld(t) -> int:
     return t.stride(0) if t.dim() >= 2 else t.shape[0]
 
 
+def _split_scratch(nbytes: int, like):
+    """Scratch of a K split for one launch: from torch's allocator on the launch stream (which
+    reuses it only after that stream has passed the launch), so that calls of one artifact on
+    several streams or threads never share it. None when the call needs none."""
+    if nbytes == 0:
+        return None
+    import torch
+
+    return torch.empty(nbytes, dtype=torch.uint8, device=like.device)
+
+
 # ---- W4A16 ------------------------------------------------------------------------
 
 def _w4_check(env: dict) -> None:
@@ -126,6 +137,13 @@ def _w4_launch(v: dict, env: dict, stream: int, workspace) -> str:
     if kernel == "auto":
         kernel = "gemv" if env["M"] <= 16 else "gemm"
     entry = {"gemv": "intent_w4a16_gemv", "gemm": "intent_w4a16_gemm"}[kernel]
+    if kernel == "gemm":
+        scratch = _split_scratch(_native.library().intent_w4a16_gemm_workspace_size(env["M"], env["K"], env["N"],
+                                                                                    env["GROUP"]), y)
+        if scratch is not None:
+            _native.call("intent_w4a16_gemm_ws", _ptr(x), env["M"], env["K"], _ld(x), _ptr(q), env["N"], _ld(q), _ptr(s),
+                         _ptr(z), s.stride(0), env["GROUP"], _ptr(y), _ld(y), _ptr(scratch), scratch.numel(), stream)
+            return entry
     _native.call(entry, _ptr(x), env["M"], env["K"], _ld(x), _ptr(q), env["N"], _ld(q), _ptr(s), _ptr(z),
                  s.stride(0), env["GROUP"], _ptr(y), _ld(y), stream)
     return entry
@@ -152,8 +170,15 @@ weight_only_int4_asym_matmul = KernelDefinition(
 
 def _w8a16_launch(v: dict, env: dict, stream: int, workspace) -> str:
     x, w, s, y = v["activation"], v["weight"], v["scales"], v["output"]
-    _native.call("intent_w8a16_matmul", _ptr(x), env["M"], env["K"], _ld(x), _ptr(w), env["N"], _ld(w), _ptr(s),
-                 _ptr(y), _ld(y), stream)
+    scratch = None
+    if env["M"] > 16:
+        scratch = _split_scratch(_native.library().intent_w8a16_matmul_workspace_size(env["M"], env["K"], env["N"]), y)
+    if scratch is not None:
+        _native.call("intent_w8a16_matmul_ws", _ptr(x), env["M"], env["K"], _ld(x), _ptr(w), env["N"], _ld(w), _ptr(s),
+                     _ptr(y), _ld(y), _ptr(scratch), scratch.numel(), stream)
+    else:
+        _native.call("intent_w8a16_matmul", _ptr(x), env["M"], env["K"], _ld(x), _ptr(w), env["N"], _ld(w), _ptr(s),
+                     _ptr(y), _ld(y), stream)
     return "intent_w8a16_matmul"
 
 

@@ -414,6 +414,30 @@ def test_moe_ffn_few_routes(gpu, threads, T, H, E, k, F, group, skew):
     assert_close_rms(got - y0, ref - y0, what=f"moe few routes T {T} H {H} E {E} F {F} group {group}")
 
 
+# K split over workgroups (partial sums through scratch) and the 64-, 128- and 256-row tiles: rows and
+# columns off the tiles, runs of unequal length (11 or 43 units over 8 runs), every group form the cut takes
+# (windowed, whole groups, 32), and an output whose row stride rules out the vector stores.
+@pytest.mark.parametrize("M,K,N,group,pad", [
+    (17, 1408, 130, 128, 0), (64, 2048, 257, 64, 0), (65, 4096, 128, 128, 3), (129, 5504, 193, 128, 0),
+    (200, 3072, 1001, 32, 0), (300, 8192, 129, 256, 0), (256, 4096, 640, 128, 1), (513, 4096, 200, 64, 0)])
+def test_w4a16_split_k(gpu, threads, M, K, N, group, pad):
+    d = inputs.config1_w4a16_decode(M + N, M=M, K=K, N=N, group=group)
+    assert _native.library().intent_w4a16_gemm_workspace_size(M, K, N, group) > 0
+    y = torch.zeros(M, N + pad, dtype=torch.float16, device="cuda")[:, :N]
+    art(intent.weight_only_int4_asym_matmul)(dev(d["x"]), dev(d["packed"]), dev(d["scales"]), dev(d["zeros"]), y)
+    ref = oracle.w4a16(d["x"], d["packed"], d["scales"], d["zeros"], threads)
+    assert_close_rms(y.cpu().numpy(), ref, what=f"w4a16 split {M}x{K}x{N} g{group}")
+
+
+@pytest.mark.parametrize("M,K,N", [(17, 1088, 130), (65, 4096, 129), (129, 2048, 1001), (300, 8192, 200)])
+def test_w8a16_split_k(gpu, threads, M, K, N):
+    d = inputs.config0_w8a16(M + N, M=M, K=K, N=N)
+    assert _native.library().intent_w8a16_matmul_workspace_size(M, K, N) > 0
+    y = art(intent.weight_only_int8_matmul).run(dev(d["x"]), dev(d["w"]), dev(d["scales"]))
+    ref = oracle.w8a16(d["x"], d["w"], d["scales"], threads)
+    assert_close_rms(host(y), ref, what=f"w8a16 split {M}x{K}x{N}")
+
+
 # More than 64 row blocks of 160 rows (64 experts of ~128 routes): the
 # heavy-first block order of gate/up takes several wave-wide passes.
 def test_moe_ffn_many_blocks(gpu, threads):
