@@ -84,16 +84,35 @@ class CompiledArtifact:
         return self.launch
 
     # ---- invocation ----------------------------------------------------------------
-    @_on_artifact_device
+    # A call whose layout (dtypes, devices, shapes, strides) was bound before goes
+    # straight to its launch; the full binder takes every other one.
     def run(self, *inputs: Any) -> object:
+        bound = self._rebind(inputs, False)
+        return self._run_checked(*inputs) if bound is None else self.runtime.launch_bound(bound)
+
+    def launch(self, *arguments: Any) -> None:
+        bound = self._rebind(arguments, True)
+        if bound is None:
+            self._launch_checked(*arguments)
+        else:
+            self.runtime.launch_bound(bound)
+
+    __call__ = launch
+
+    def _rebind(self, arguments: tuple, supplied_outputs: bool):
+        import torch
+
+        if torch.cuda.current_device() != self.device:
+            return None
+        return self.runtime.rebind(arguments, supplied_outputs)
+
+    @_on_artifact_device
+    def _run_checked(self, *inputs: Any) -> object:
         return self.runtime.run(*inputs)
 
     @_on_artifact_device
-    def launch(self, *arguments: Any) -> None:
+    def _launch_checked(self, *arguments: Any) -> None:
         self.runtime.launch(*arguments)
-
-    def __call__(self, *arguments: Any) -> None:
-        self.launch(*arguments)
 
     @_on_artifact_device
     def prepare(self, *inputs: Any, outputs: tuple | None = None):

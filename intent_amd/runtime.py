@@ -36,12 +36,38 @@ class ConfigurationAssessment:
     reason: str
 
 
-@dataclass
+@dataclass(slots=True)
 class Binding:
     views: dict
     env: dict
     outputs: tuple
     workspace: object = None
+
+
+@dataclass(slots=True)
+class _Layout:
+    """What binding established for one combination of dtypes, devices, shapes and strides.
+
+    Everything the checks of ``_bind`` derive from those alone: a call with the same
+    combination needs only its addresses compared (``pairs``: the views of which one is
+    writable, spans in bytes)."""
+
+    env: dict
+    names: tuple        # the supplied views, in argument order
+    outputs: tuple      # allocated Out buffers: (name, shape, dtype)
+    spans: tuple
+    pairs: tuple
+    workspace: int      # bytes, -1 without one
+
+
+MAX_LAYOUTS = 256  # layouts kept per artifact and calling form; the oldest go first
+
+
+def _current_stream(device: int) -> int:
+    import torch
+
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    return raw(device) if raw is not None else torch.cuda.current_stream(device).cuda_stream
 
 
 class HIPRuntime:
@@ -52,11 +78,107 @@ class HIPRuntime:
         self.arch = arch
         self._interface = definition.interface()
         self._workspace = None
-        self.observation: NativeObservation | None = None
+        self._latest: tuple | None = None  # (entry, kernel name bytes) of the latest launch
+        self._scalars = {p.name for p in definition.params if isinstance(p, Scalar)}
+        self._writable = {p.name for p in definition.params if isinstance(p, Param) and p.access is not ViewKind.IN}
+        self._supplied = tuple(p for p in definition.params if isinstance(p, Scalar) or p.access is not ViewKind.OUT)
+        self._layouts: tuple[dict, dict] = ({}, {})  # by calling form: outputs allocated, outputs supplied
+        self._home = None
 
     @property
     def interface(self) -> PublicInterface:
         return self._interface
+
+    @property
+    def observation(self) -> NativeObservation | None:
+        if self._latest is None:
+            return None
+        entry, kernel = self._latest
+        return NativeObservation(entry, self.definition.name, self.arch, str(_native.LIBRARY_PATH),
+                                 dict(self.constexprs), kernel.decode("utf-8", "replace") if kernel else "")
+
+    # ---- known layouts --------------------------------------------------------
+    def _home_device(self):
+        if self._home is None:
+            import torch
+
+            self._home = torch.device("cuda", self.device)
+        return self._home
+
+    def _layout_key(self, params: tuple, arguments: tuple):
+        """Dtypes, devices, shapes and strides of the arguments; None unless all are plain tensors."""
+        import torch
+
+        key = []
+        for p, a in zip(params, arguments):
+            if p.name in self._scalars:
+                continue
+            if type(a) is not torch.Tensor and type(a) is not torch.nn.Parameter:
+                return None
+            if a.layout is not torch.strided:
+                return None
+            key += (a.dtype, a.device, a.shape, a.stride())
+        return tuple(key)
+
+    def rebind(self, arguments: tuple, supplied_outputs: bool) -> Binding | None:
+        """The binding of a call whose layout has been bound before, or None (then ``_bind`` checks it)."""
+        params = self.definition.params if supplied_outputs else self._supplied
+        if len(arguments) != len(params):
+            return None
+        key = self._layout_key(params, arguments)
+        known = self._layouts[supplied_outputs].get(key) if key is not None else None
+        if known is None:
+            return None
+        env = known.env
+        if self._scalars:
+            env = dict(env)
+            tensors = []
+            for p, a in zip(params, arguments):
+                if p.name in self._scalars:
+                    env[p.name] = a
+                else:
+                    tensors.append(a)
+        else:
+            tensors = arguments
+        if known.pairs:
+            starts = [t.data_ptr() for t in tensors]
+            for i, j in known.pairs:
+                if starts[i] < starts[j] + known.spans[j] and starts[j] < starts[i] + known.spans[i]:
+                    return None  # _bind names the overlap
+        views = dict(zip(known.names, tensors))
+        if known.outputs:
+            import torch
+
+            outputs = []
+            for name, shape, dt in known.outputs:
+                t = torch.empty(shape, dtype=dt, device=self._home_device())
+                views[name] = t
+                outputs.append(t)
+            return Binding(views, env, tuple(outputs), self._workspace_of(known.workspace))
+        outputs = ()
+        if supplied_outputs:
+            outputs = tuple(views[p.name] for p in params if p.name not in self._scalars and p.access is ViewKind.OUT)
+        return Binding(views, env, outputs, self._workspace_of(known.workspace))
+
+    def _remember(self, arguments: tuple, supplied_outputs: bool, binding: Binding) -> None:
+        params = self.definition.params if supplied_outputs else self._supplied
+        key = self._layout_key(params, arguments)
+        if key is None:
+            return
+        views = [(p, a) for p, a in zip(params, arguments) if p.name not in self._scalars]
+        spans = tuple(_span_bytes(t) for _, t in views)
+        pairs = tuple((i, j) for i in range(len(views)) for j in range(i + 1, len(views))
+                      if spans[i] and spans[j]
+                      and (views[i][0].name in self._writable or views[j][0].name in self._writable))
+        made = () if supplied_outputs else tuple((p.name, tuple(binding.views[p.name].shape), binding.views[p.name].dtype)
+                                                 for p in self.definition.params
+                                                 if p.name not in self._scalars and p.access is ViewKind.OUT)
+        known = self._layouts[supplied_outputs]
+        if len(known) >= MAX_LAYOUTS:
+            for old in list(known)[:MAX_LAYOUTS // 2]:
+                known.pop(old, None)
+        need = -1 if self.definition.workspace is None else int(self.definition.workspace(binding.env))
+        known[key] = _Layout(dict(binding.env), tuple(p.name for p, _ in views), made, spans, pairs, need)
 
     # ---- binding ------------------------------------------------------------
     def _bind(self, arguments: tuple, explicit_outputs: tuple | None, abstract: bool = False) -> Binding:
@@ -137,9 +259,7 @@ class HIPRuntime:
         return int(dim(env))
 
     def _check_layout(self, p: Param, t) -> None:
-        import torch
-
-        expected = torch.device("cuda", self.device)
+        expected = self._home_device()
         if t.device != expected:
             raise ValueError(f"compiled artifact is bound to {expected}, but {p.name} is on {t.device}")
         if t.numel() == 0 or p.free_strides:
@@ -154,14 +274,13 @@ class HIPRuntime:
 
     def _check_aliases(self, views: dict) -> None:
         """Writable views may not overlap any other view (noalias contract)."""
-        writable = {p.name for p in self.definition.params if isinstance(p, Param) and p.access is not ViewKind.IN}
+        writable = self._writable
         spans = {}
         for name, t in views.items():
             if t.numel() == 0:
                 continue
             start = t.data_ptr()
-            last = sum((extent - 1) * stride for extent, stride in zip(t.shape, t.stride()))
-            spans[name] = (start, start + (last + 1) * t.element_size())
+            spans[name] = (start, start + _span_bytes(t))
         names = list(spans)
         for i, a in enumerate(names):
             for b in names[i + 1:]:
@@ -172,29 +291,31 @@ class HIPRuntime:
                     raise ValueError(f"{self.definition.name}: {a} and {b} overlap; writable views must not alias")
 
     def _workspace_for(self, env: dict):
-        import torch
+        return self._workspace_of(-1 if self.definition.workspace is None else self.definition.workspace(env))
 
-        if self.definition.workspace is None:
+    def _workspace_of(self, need: int):
+        if need < 0:
             return None
-        need = self.definition.workspace(env)
         if self._workspace is None or self._workspace.numel() < need:
-            self._workspace = torch.empty(max(need, 16), dtype=torch.uint8, device=torch.device("cuda", self.device))
+            import torch
+
+            self._workspace = torch.empty(max(need, 16), dtype=torch.uint8, device=self._home_device())
         return self._workspace
 
     def _launch(self, binding: Binding) -> None:
-        import torch
-
-        stream = torch.cuda.current_stream(self.device).cuda_stream
-        entry = self.definition.launch(binding.views, binding.env, stream, binding.workspace)
-        self.observation = NativeObservation(entry, self.definition.name, self.arch, str(_native.LIBRARY_PATH),
-                                             dict(self.constexprs), _native.last_kernel())
+        entry = self.definition.launch(binding.views, binding.env, _current_stream(self.device), binding.workspace)
+        self._latest = (entry, _native.library().intent_amd_last_kernel())
 
     # ---- provider surface -------------------------------------------------------
-    def run(self, *arguments):
-        binding = self._bind(arguments, None)
-        binding.workspace = self._workspace_for(binding.env)
+    def launch_bound(self, binding: Binding):
         self._launch(binding)
         return _result(binding.outputs)
+
+    def run(self, *arguments):
+        binding = self._bind(arguments, None)
+        self._remember(arguments, False, binding)
+        binding.workspace = self._workspace_for(binding.env)
+        return self.launch_bound(binding)
 
     def launch(self, *arguments):
         interface = self._interface
@@ -206,6 +327,7 @@ class HIPRuntime:
         outs = tuple(a for a, p in zip(arguments, interface.parameters) if getattr(p, "output", False))
         assert len(ins) == n_in
         binding = self._bind(ins, outs)
+        self._remember(arguments, True, binding)
         binding.workspace = self._workspace_for(binding.env)
         self._launch(binding)
         return None
@@ -221,6 +343,13 @@ class HIPRuntime:
 
     def tuning_configurations(self, *arguments):
         return ()
+
+
+def _span_bytes(t) -> int:
+    """Bytes from a strided view's first element to the end of its last; 0 for an empty one."""
+    if t.numel() == 0:
+        return 0
+    return (sum((extent - 1) * stride for extent, stride in zip(t.shape, t.stride())) + 1) * t.element_size()
 
 
 def _result(outputs: tuple):

@@ -167,3 +167,64 @@ def test_bench_refuses_multi_gpu():
     proc = subprocess.run([sys.executable, str(ROOT / "bench.py"), "--gpus", "2"], capture_output=True, text=True,
                           timeout=120)
     assert proc.returncode == 2 and "exactly one GPU" in proc.stdout
+
+
+def _cpu_runtime(defn, monkeypatch, **constexprs):
+    """A runtime that binds CPU tensors and records launches instead of making them."""
+    rt = runtime_for(defn, **constexprs)
+    rt._home = torch.device("cpu")
+    launches = []
+    monkeypatch.setattr(rt, "_launch", launches.append)
+    return rt, launches
+
+
+def test_known_layout_binds_like_the_first_call(monkeypatch):
+    rt, launches = _cpu_runtime(intent.weight_only_int4_asym_matmul, monkeypatch)
+
+    def args(M, stride=0):
+        x = torch.zeros(M, 256 + stride, dtype=torch.float16)[:, :256]
+        return (x, torch.zeros(8, 128, dtype=torch.uint8), torch.zeros(8, 2, dtype=torch.float16),
+                torch.zeros(8, 2, dtype=torch.uint8))
+
+    assert rt.rebind(args(3), False) is None  # nothing bound yet
+    rt.run(*args(3))
+    a = args(3)
+    b = rt.rebind(a, False)
+    first = launches[0]
+    assert b.env == first.env and list(b.views) == list(first.views)
+    assert all(b.views[n] is t for n, t in zip(("activation", "packed_weight", "scales", "zeros"), a))
+    assert b.outputs[0].shape == first.outputs[0].shape and b.outputs[0].dtype == first.outputs[0].dtype
+    assert b.outputs[0] is not first.outputs[0]
+    # any other shape, stride, dtype, count or kind of argument goes to the full binder
+    assert rt.rebind(args(4), False) is None
+    assert rt.rebind(args(3, stride=8), False) is None
+    assert rt.rebind((a[0].float(),) + a[1:], False) is None
+    assert rt.rebind(a[:3], False) is None
+    assert rt.rebind((1.0,) + a[1:], False) is None
+    # supplied outputs are another form, with its own layouts; an overlap is refused on every call
+    y = torch.zeros(3, 8, dtype=torch.float16)
+    assert rt.rebind(a + (y,), True) is None
+    rt.launch(*a, y)
+    assert rt.rebind(a + (y,), True).outputs[0] is y
+    shared = torch.zeros(3 * 256 + 24, dtype=torch.float16)
+    over = (shared[:768].view(3, 256),) + a[1:] + (shared[760:784].view(3, 8),)
+    assert rt.rebind(over, True) is None
+    with pytest.raises(ValueError, match="must not alias"):
+        rt.launch(*over)
+
+
+def test_known_layouts_scalars_and_bound(monkeypatch):
+    from intent_amd import runtime as runtime_module
+
+    rt, launches = _cpu_runtime(intent.scaled_fp8_matmul, monkeypatch)
+    lhs = torch.zeros(2, 128, dtype=torch.float8_e4m3fn)
+    rhs = torch.zeros(128, 16, dtype=torch.float8_e4m3fn)
+    rt.run(lhs, rhs, 0.5, 2.0)
+    b = rt.rebind((lhs, rhs, 0.25, 3.0), False)
+    assert (b.env["lhs_scale"], b.env["rhs_scale"]) == (0.25, 3.0)
+    assert (launches[0].env["lhs_scale"], launches[0].env["rhs_scale"]) == (0.5, 2.0)
+    monkeypatch.setattr(runtime_module, "MAX_LAYOUTS", 4)
+    for m in range(1, 12):
+        rt.run(torch.zeros(m, 128, dtype=torch.float8_e4m3fn), rhs, 1.0, 1.0)
+        assert len(rt._layouts[0]) <= 4
+    assert rt.rebind((torch.zeros(11, 128, dtype=torch.float8_e4m3fn), rhs, 1.0, 1.0), False) is not None
