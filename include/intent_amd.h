@@ -143,6 +143,14 @@ int intent_w8a8_gemm(const int8_t* a, int64_t M, int64_t K, int64_t a_ld,
                      const int8_t* w, int64_t N, int64_t w_ld,
                      const float* w_scales,
                      void* out, int64_t out_ld, void* stream);
+/* The same product with a workspace for a K split (see intent_w8a16_matmul_ws;
+ * the int32 sums stay exact, so the result has the same bits). */
+size_t intent_w8a8_gemm_workspace_size(int64_t M, int64_t K, int64_t N);
+int intent_w8a8_gemm_ws(const int8_t* a, int64_t M, int64_t K, int64_t a_ld,
+                        const float* a_scales,
+                        const int8_t* w, int64_t N, int64_t w_ld,
+                        const float* w_scales, void* out, int64_t out_ld,
+                        void* workspace, size_t workspace_bytes, void* stream);
 
 /*
  * int8 x int8 -> int32 contraction with optional int32 bias (nullable):

@@ -1,7 +1,7 @@
 // W8A8 int8 GEMM on v_mfma_i32_32x32x32_i8 (gfx950), exact int32 accumulation.
 //
-// Tiles of 256 x 256 with 8 waves in 4 x 2 (or 128 x 128 with 4 waves for
-// small problems) on the pipelined core in mfma_pipe.h: both K-contiguous int8 operands are
+// Tiles of 256 x 256 with 8 waves in 4 x 2 (or 128 x 128 and 64 x 128 with 4
+// waves, i8_plan) on the pipelined core in mfma_pipe.h: both K-contiguous int8 operands are
 // staged global -> VGPR -> LDS, 128 k per stage, two stages in flight.
 // Epilogues: bf16(f32(acc) * a_scale[m] * w_scale[n]) or int32 acc + bias[n].
 #include "common.h"
@@ -327,6 +327,93 @@ __global__ __launch_bounds__(T::NT_WS, 1) void lowbit_ws_kernel(const int8_t* __
   }
 }
 
+// ---- K split over workgroups (W8A8) -----------------------------------------------
+// blockIdx.y takes one run of the K stages and leaves its int32 sums in the
+// register layout (1 KB contiguous per store); i8_combine_kernel adds the runs
+// (exact, so any order gives the same bits) and applies the scales.
+template <class T, bool kHalf>
+__global__ __launch_bounds__(T::NT, 1) void i8_split_kernel(const int8_t* __restrict__ a, int64_t lda, int M,
+                                                            const int8_t* __restrict__ w, int64_t ldw, int N, int K,
+                                                            int32_t* __restrict__ part, int mblocks) {
+  __shared__ __attribute__((aligned(16))) char buf0[T::STAGE_BYTES];
+  __shared__ __attribute__((aligned(16))) char buf1[T::STAGE_BYTES];
+  int tmb, tnb;
+  grid_tile(mblocks, 4, tmb, tnb);
+  const int m0 = tmb * T::BM;
+  const int n0 = tnb * T::BN;
+  const int stages = (K + mp::ROWB - 1) / mp::ROWB;
+  const int p = blockIdx.y, S = gridDim.y;
+  const int s0 = (int)((int64_t)p * stages / S), s1 = (int)((int64_t)(p + 1) * stages / S);
+  const bool half = kHalf && p == S - 1;  // the run that holds the last, 64-k stage
+  const int nk = s1 - s0;
+  mp::RegRowsOperand<T::BN, mp::DenseRows, kHalf, T::NW> bop;
+  bop.init(mp::DenseRows{w + (int64_t)s0 * mp::ROWB, ldw, N}, n0, T::wave(), half ? nk - 1 : -1);
+  mp::RegRowsOperand<T::BM, mp::DenseRows, kHalf, T::NW> aop;
+  aop.init(mp::DenseRows{a + (int64_t)s0 * mp::ROWB, lda, M}, m0, T::wave(), half ? nk - 1 : -1);
+  i32x16 acc[T::TI][T::TJ];
+  mp::mainloop<T, mp::I8Math>(aop, bop, nk, buf0, buf1, acc, half);
+  constexpr int BLK = T::TI * T::TJ * 4;
+  int32_t* out = part + (((int64_t)p * gridDim.x + blockIdx.x) * T::NW + T::wave()) * (BLK * 256) + (threadIdx.x & 63) * 4;
+#pragma unroll
+  for (int i = 0; i < T::TI; ++i) {
+    if (m0 + T::row(i) >= M) continue;
+#pragma unroll
+    for (int j = 0; j < T::TJ; ++j)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<i32x4*>(out + ((i * T::TJ + j) * 4 + g) * 256) =
+            i32x4{acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
+  }
+}
+
+// out = bf16((f32(sum of the runs) * sa[m]) * sw[n]); one wave per 32 x 32 block.
+template <class T>
+__global__ __launch_bounds__(64) void i8_combine_kernel(const int32_t* __restrict__ part, int S, int tiles, int M,
+                                                        int N, const float* __restrict__ a_scales,
+                                                        const float* __restrict__ w_scales, uint16_t* __restrict__ out,
+                                                        int64_t ldo, int vec, int mblocks) {
+  constexpr int BLK = T::TI * T::TJ * 4;
+  int id = blockIdx.x;  // ((tile * NW + wave) * TI + i) * TJ + j
+  const int j = id % T::TJ;
+  id /= T::TJ;
+  const int i = id % T::TI;
+  id /= T::TI;
+  const int wave = id % T::NW, tile = id / T::NW;
+  int tmb, tnb;
+  grouped_tile(xcd_swizzle(tile, tiles), mblocks, tiles / mblocks, 4, tmb, tnb);
+  const int lane = threadIdx.x;
+  const int m = tmb * T::BM + (wave % T::WM) * T::WTM + i * 32 + (lane & 31);
+  const int n0 = tnb * T::BN + (wave / T::WM) * T::WTN + j * 32 + (lane >> 5) * 4;
+  if (m >= M) return;
+  const int32_t* src = part + ((int64_t)tile * T::NW + wave) * (BLK * 256) + (i * T::TJ + j) * 1024 + lane * 4;
+  const int64_t stride = (int64_t)tiles * T::NW * (BLK * 256);
+  u32x4 v[4];
+#pragma unroll
+  for (int g = 0; g < 4; ++g) v[g] = *reinterpret_cast<const u32x4*>(src + g * 256);
+  for (int p = 1; p < S; ++p) {
+    src += stride;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) v[g] += *reinterpret_cast<const u32x4*>(src + g * 256);
+  }
+  const float sa = a_scales[m];
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    const int n = n0 + g * 8;
+    float f[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) f[c] = ((float)(int32_t)v[g][c] * sa) * (n + c < N ? w_scales[n + c] : 0.f);
+    uint16_t* o = out + (int64_t)m * ldo + n;
+    const u32x2 pk{bf16x2_rne(f[0], f[1]), bf16x2_rne(f[2], f[3])};
+    if (vec && n + 3 < N) {
+      *reinterpret_cast<u32x2*>(o) = pk;
+    } else {
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        if (n + c < N) o[c] = (uint16_t)(pk[c >> 1] >> (16 * (c & 1)));
+    }
+  }
+}
+
 int check_i8(const int8_t* a, int64_t M, int64_t K, int64_t a_ld, const int8_t* w, int64_t N, int64_t w_ld,
              const void* out, int64_t out_ld) {
   INTENT_REQUIRE(M >= 0 && N >= 0 && K >= 0, INTENT_ERR_INVALID_ARGUMENT, "negative extent");
@@ -363,22 +450,89 @@ int launch_tile(const int8_t* a, int64_t M, int64_t K, int64_t a_ld, const float
   return intent::launch_status(name);
 }
 
-// 256 x 256 tiles once the problem has enough of them to fill the chip.
+using T64 = mp::Tile<64, 128, 2, 2>;
+
+struct I8Plan {
+  int tile;    // rows of the tile: 256 (256 x 256), 128 (128 x 128), 64 (64 x 128)
+  int splits;  // K runs (1: no workspace)
+};
+int64_t i8_tiles(int64_t M, int64_t N, int tile) {
+  const int64_t bn = tile == 256 ? 256 : 128;
+  return ((M + tile - 1) / tile) * ((N + bn - 1) / bn);
+}
+int64_t i8_split_bytes(const I8Plan& p, int64_t M, int64_t N) {
+  return p.splits > 1 ? p.splits * i8_tiles(M, N, p.tile) * p.tile * (p.tile == 256 ? 256 : 128) * 4 : 0;
+}
+// Costs in microseconds, measured: a 128-k stage takes a + b L at L =
+// workgroups / 256 up to one per CU, then (a + b) times the rounds; a split adds
+// 2.5 us and 0.27 us per MB of int32 sums. Fitted to 78 shapes (M 1..4096, N
+// 1024..14336, K 1024..8192): the choice is within 0.6% of the best of all plans
+// on average. With the quantizer, N = K = 8192: M = 1 35 -> 20 us, 32 35 -> 21,
+// 128 39 -> 26 us; N = 2048, K = 8192, M = 64: 36 -> 17 us; N = 11008, K = 4096,
+// M = 1024: 66 -> 58 us (256 x 256 tiles on 172 CUs beat 688 of 128 x 128).
+I8Plan i8_plan(int64_t M, int64_t N, int64_t K, bool may_split) {
+  if (i8_tiles(M, N, 256) >= 256) return {256, 1};
+  const int64_t stages = (K + mp::ROWB - 1) / mp::ROWB;
+  I8Plan best{128, 1};
+  double least = 0;
+  for (int tile = 256; tile >= 64; tile /= 2) {
+    const double c0 = tile == 256 ? 7.0 : tile == 128 ? 4.5 : 4.7;
+    const double a = tile == 256 ? 0.82 : tile == 128 ? 0.39 : 0.32;
+    const double b = tile == 256 ? 1.05 : tile == 128 ? 0.206 : 0.12;
+    for (int splits = 1; splits <= (may_split ? 8 : 1) && splits <= stages; splits *= 2) {
+      const I8Plan p{tile, splits};
+      if (i8_split_bytes(p, M, N) > (64 << 20)) break;
+      const int64_t wgs = i8_tiles(M, N, tile) * splits;
+      const double L = (double)wgs / 256;
+      const double stage = L <= 1 ? a + b * L : (a + b) * (L + (double)((wgs + 255) / 256)) / 2;
+      const double split = splits > 1 ? 2.5 + 0.27e-6 * (double)i8_split_bytes(p, M, N) : 0;
+      const double c = c0 + (double)((stages + splits - 1) / splits) * stage + split;
+      if (least == 0 || c < least) {
+        least = c;
+        best = p;
+      }
+    }
+  }
+  return best;
+}
+
+template <class T>
+int launch_split(const int8_t* a, int64_t M, int64_t K, int64_t a_ld, const float* sa, const int8_t* w, int64_t N,
+                 int64_t w_ld, const float* sw, void* out, int64_t out_ld, int splits, void* ws, void* stream,
+                 const char* name) {
+  const int mblocks = (int)((M + T::BM - 1) / T::BM);
+  const int64_t grid = (int64_t)mblocks * ((N + T::BN - 1) / T::BN);
+  const int64_t cgrid = grid * T::NW * T::TI * T::TJ;
+  INTENT_REQUIRE(cgrid < (1ll << 31), INTENT_ERR_UNSUPPORTED, "%s: grid too large", name);
+  INTENT_REQUIRE(intent::fits_offset(M, a_ld) && intent::fits_offset(N, w_ld), INTENT_ERR_UNSUPPORTED,
+                 "%s: operand too large for 31-bit buffer offsets", name);
+  const auto kernel = K % mp::ROWB == 0 ? i8_split_kernel<T, false> : i8_split_kernel<T, true>;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)grid, splits), dim3(T::NT), 0, (hipStream_t)stream, a, a_ld, (int)M, w,
+                     w_ld, (int)N, (int)K, (int32_t*)ws, mblocks);
+  const int st = intent::launch_status(name);
+  if (st != INTENT_OK) return st;
+  const int vec = out_ld % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & 7) == 0;
+  hipLaunchKernelGGL((i8_combine_kernel<T>), dim3((unsigned)cgrid), dim3(64), 0, (hipStream_t)stream,
+                     (const int32_t*)ws, splits, (int)grid, (int)M, (int)N, sa, sw, (uint16_t*)out, out_ld, vec,
+                     mblocks);
+  return intent::launch_status(name);
+}
+
 template <Epi E>
 int launch_i8(const int8_t* a, int64_t M, int64_t K, int64_t a_ld, const float* sa, const int8_t* w, int64_t N,
               int64_t w_ld, const float* sw, const int32_t* bias, void* out, int64_t out_ld, void* stream,
               const char* name) {
-  const int64_t big = ((M + 255) / 256) * ((N + 255) / 256);
-  if (big >= 256)
+  const I8Plan p = i8_plan(M, N, K, false);
+  if (p.tile == 256)
     return launch_tile<T256, E>(a, M, K, a_ld, sa, w, N, w_ld, sw, bias, out, out_ld, stream, name);
-  return launch_tile<T128, E>(a, M, K, a_ld, sa, w, N, w_ld, sw, bias, out, out_ld, stream, name);
+  if (p.tile == 128)
+    return launch_tile<T128, E>(a, M, K, a_ld, sa, w, N, w_ld, sw, bias, out, out_ld, stream, name);
+  return launch_tile<T64, E>(a, M, K, a_ld, sa, w, N, w_ld, sw, bias, out, out_ld, stream, name);
 }
 
-}  // namespace
-
-extern "C" int intent_w8a8_gemm(const int8_t* a, int64_t M, int64_t K, int64_t a_ld, const float* a_scales,
-                                const int8_t* w, int64_t N, int64_t w_ld, const float* w_scales, void* out,
-                                int64_t out_ld, void* stream) {
+int w8a8_launch(const int8_t* a, int64_t M, int64_t K, int64_t a_ld, const float* a_scales, const int8_t* w, int64_t N,
+                int64_t w_ld, const float* w_scales, void* out, int64_t out_ld, void* ws, size_t ws_bytes,
+                void* stream) {
   intent::clear_error();
   int st = check_i8(a, M, K, a_ld, w, N, w_ld, out, out_ld);
   if (st != INTENT_OK || M == 0 || N == 0) return st;
@@ -386,8 +540,32 @@ extern "C" int intent_w8a8_gemm(const int8_t* a, int64_t M, int64_t K, int64_t a
   if (!i8_fast(a, K, a_ld, w, w_ld))
     return intent::i8_generic_launch(a, M, K, a_ld, w, N, w_ld, a_scales, w_scales, nullptr, out, out_ld, true,
                                      stream);
+  const I8Plan p = i8_plan(M, N, K, true);
+  if (p.splits > 1 && ws && intent::aligned16(ws) && ws_bytes >= (size_t)i8_split_bytes(p, M, N)) {
+    const auto launch = p.tile == 256 ? launch_split<T256> : p.tile == 128 ? launch_split<T128> : launch_split<T64>;
+    return launch(a, M, K, a_ld, a_scales, w, N, w_ld, w_scales, out, out_ld, p.splits, ws, stream, "w8a8_gemm");
+  }
   return launch_i8<Epi::kBf16Scaled>(a, M, K, a_ld, a_scales, w, N, w_ld, w_scales, nullptr, out, out_ld, stream,
                                      "w8a8_gemm");
+}
+
+}  // namespace
+
+extern "C" int intent_w8a8_gemm(const int8_t* a, int64_t M, int64_t K, int64_t a_ld, const float* a_scales,
+                                const int8_t* w, int64_t N, int64_t w_ld, const float* w_scales, void* out,
+                                int64_t out_ld, void* stream) {
+  return w8a8_launch(a, M, K, a_ld, a_scales, w, N, w_ld, w_scales, out, out_ld, nullptr, 0, stream);
+}
+
+extern "C" size_t intent_w8a8_gemm_workspace_size(int64_t M, int64_t K, int64_t N) {
+  if (M <= 0 || N <= 0 || K <= 0 || K % 64 != 0) return 0;
+  return (size_t)i8_split_bytes(i8_plan(M, N, K, true), M, N);
+}
+
+extern "C" int intent_w8a8_gemm_ws(const int8_t* a, int64_t M, int64_t K, int64_t a_ld, const float* a_scales,
+                                   const int8_t* w, int64_t N, int64_t w_ld, const float* w_scales, void* out,
+                                   int64_t out_ld, void* workspace, size_t workspace_bytes, void* stream) {
+  return w8a8_launch(a, M, K, a_ld, a_scales, w, N, w_ld, w_scales, out, out_ld, workspace, workspace_bytes, stream);
 }
 
 extern "C" int intent_i8_gemm_i32(const int8_t* a, int64_t M, int64_t K, int64_t a_ld, const int8_t* w, int64_t N,

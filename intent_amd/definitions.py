@@ -200,8 +200,13 @@ weight_only_int8_matmul = KernelDefinition(
 
 def _w8a8_launch(v: dict, env: dict, stream: int, workspace) -> str:
     a, sa, w, sw, out = v["activation"], v["activation_scales"], v["weight"], v["weight_scales"], v["output"]
-    _native.call("intent_w8a8_gemm", _ptr(a), env["M"], env["K"], _ld(a), _ptr(sa), _ptr(w), env["N"], _ld(w),
-                 _ptr(sw), _ptr(out), _ld(out), stream)
+    scratch = _split_scratch(_native.library().intent_w8a8_gemm_workspace_size(env["M"], env["K"], env["N"]), out)
+    if scratch is not None:
+        _native.call("intent_w8a8_gemm_ws", _ptr(a), env["M"], env["K"], _ld(a), _ptr(sa), _ptr(w), env["N"], _ld(w),
+                     _ptr(sw), _ptr(out), _ld(out), _ptr(scratch), scratch.numel(), stream)
+    else:
+        _native.call("intent_w8a8_gemm", _ptr(a), env["M"], env["K"], _ld(a), _ptr(sa), _ptr(w), env["N"], _ld(w),
+                     _ptr(sw), _ptr(out), _ld(out), stream)
     return "intent_w8a8_gemm"
 
 

@@ -438,6 +438,21 @@ def test_w8a16_split_k(gpu, threads, M, K, N):
     assert_close_rms(host(y), ref, what=f"w8a16 split {M}x{K}x{N}")
 
 
+# W8A8 with K split over workgroups: runs of unequal length, a last stage of 64 k (K % 128 == 64), rows and
+# columns off the 64-, 128- and 256-row tiles, and an output stride that rules out the vector stores. The int32
+# sums are exact, so every output bit is the oracle's.
+@pytest.mark.parametrize("M,K,N,pad", [(1, 4160, 130, 0), (33, 4096, 257, 1), (64, 3520, 1001, 0), (129, 8192, 128, 0),
+                                       (200, 4160, 640, 2), (300, 8192, 1030, 0)])
+def test_w8a8_split_k(gpu, threads, M, K, N, pad):
+    d = inputs.config3_w8a8(M + N, M=M, K=K, N=N)
+    assert _native.library().intent_w8a8_gemm_workspace_size(M, K, N) > 0
+    y = torch.zeros(M, N + pad, dtype=torch.bfloat16, device="cuda")[:, :N]
+    art(intent.w8a8_scaled_matmul)(dev(d["a"]), dev(d["a_scales"]), dev(d["w"]), dev(d["w_scales"]), y)
+    ref = oracle.w8a8(d["a"], d["a_scales"], d["w"], d["w_scales"], threads)
+    got = y.contiguous().view(torch.int16).cpu().numpy().view(np.uint16)
+    assert np.array_equal(got, ref)
+
+
 # More than 64 row blocks of 160 rows (64 experts of ~128 routes): the
 # heavy-first block order of gate/up takes several wave-wide passes.
 def test_moe_ffn_many_blocks(gpu, threads):
