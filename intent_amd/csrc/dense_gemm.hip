@@ -821,7 +821,7 @@ __global__ __launch_bounds__(T::NT_WS, 1) void dense_split_kernel(const f16* __r
   float* out = part + (((int64_t)p * gridDim.x + blockIdx.x) * T::NW + T::wave()) * (BLK * 256) + (threadIdx.x & 63) * 4;
 #pragma unroll
   for (int i = 0; i < T::TI; ++i) {
-    if (m0 + T::row(i) >= M) continue;
+    if (m0 + T::wave_m() * T::WTM + i * 32 >= M) continue;  // wave-uniform: a per-lane test lets the last MFMAs' operand reads sink under it
 #pragma unroll
     for (int j = 0; j < T::TJ; ++j)
 #pragma unroll
@@ -905,10 +905,8 @@ int launch_tile(const f16* x, int64_t ldx, int M, int N, int K, const WArgs& w, 
 // Tile and K split of an M x N x K product whose K can be cut at multiples of
 // `unit`. Few tiles leave CUs idle (256 x 192 tiles of M = 512, N = 4096: 44
 // workgroups on 256 CUs), so smaller tiles and K runs are weighed against the
-// stages each workgroup then walks and the partial sums' round trip, in
-// microseconds measured on this kernel: a stage costs a + b L while the L =
-// workgroups / 256 per CU do not exceed one, then (a + b) times the rounds; a
-// split adds 3 us and 0.27 us per MB of partial sums. Fitted to 60 shapes (M
+// stages each workgroup then walks and the partial sums' round trip (GridCost,
+// measured on this kernel); a split adds 3 us and 0.27 us per MB. Fitted to 60 shapes (M
 // 17..2048, N 1024..14336, K 2048..11008, W4): the choice is within 2% of the
 // best of all twelve plans on average. N = K = 4096, M = 77: 36 -> 18 us, 256:
 // 66 -> 23, 512: 66 -> 32, 1024: 68 -> 43 us; K = 11008, M = 256: 166 -> 40 us.
@@ -932,13 +930,12 @@ DensePlan dense_plan(int64_t M, int64_t N, int64_t K, int64_t unit, bool may_spl
   DensePlan best{M > 128 ? 256 : 128, 1};
   if (dense_tiles(M, N, 256) >= 512) return best;  // two rounds of the large tile: nothing idles
   const auto cost = [&](const DensePlan& p) {
-    const double a = p.tile == 256 ? 0.95 : p.tile == 128 ? 0.48 : 0.40;
-    const double b = p.tile == 256 ? 0.42 : p.tile == 128 ? 0.14 : 0.05;
-    const double L = (double)(dense_tiles(M, N, p.tile) * p.splits) / 256;
-    const double up = (double)((dense_tiles(M, N, p.tile) * p.splits + 255) / 256);
-    const double stage = (L <= 1 ? a + b * L : (a + b) * (L + up) / 2) * (p.tile == 256 ? 1.0 : stage_scale);
-    const double split = p.splits > 1 ? 3 + 0.27e-6 * (double)dense_split_bytes(p, M, N) : 0;
-    return (p.tile == 64 ? 5 : 4) + (double)K / 64 / p.splits * stage + split;
+    const double k = p.tile == 256 ? 1.0 : stage_scale;
+    const intent::GridCost c = p.tile == 256   ? intent::GridCost{4, 0.95, 0.42}
+                               : p.tile == 128 ? intent::GridCost{4, 0.48 * k, 0.14 * k}
+                                               : intent::GridCost{5, 0.40 * k, 0.05 * k};
+    return c.us(dense_tiles(M, N, p.tile) * p.splits, (double)K / 64 / p.splits) +
+           (p.splits > 1 ? 3 + 0.27e-6 * (double)dense_split_bytes(p, M, N) : 0);
   };
   const double keep = 0.95 * cost(best);  // the plain plan unless another is clearly faster
   double least = keep;

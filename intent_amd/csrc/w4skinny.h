@@ -262,6 +262,13 @@ INTENT_DEVICE void w4_mainloop(char* lds, const void* x, const TRow& trow, const
 #pragma unroll
   for (int d = 0; d + 1 < D; ++d)
     if (whole + d < nst) stage(whole + d, xr[d], wr[d], false);
+  // The sums are complete here, under the whole wave: without this the compiler
+  // may move a last stage's fragment reads below a caller's per-lane branch,
+  // where masked lanes would not load their part of an MFMA operand.
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int t = 0; t < TU; ++t) asm volatile("" : "+v"(acc[b][t]));
 }
 
 }  // namespace sk

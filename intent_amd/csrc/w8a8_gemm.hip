@@ -356,7 +356,7 @@ __global__ __launch_bounds__(T::NT, 1) void i8_split_kernel(const int8_t* __rest
   int32_t* out = part + (((int64_t)p * gridDim.x + blockIdx.x) * T::NW + T::wave()) * (BLK * 256) + (threadIdx.x & 63) * 4;
 #pragma unroll
   for (int i = 0; i < T::TI; ++i) {
-    if (m0 + T::row(i) >= M) continue;
+    if (m0 + T::wave_m() * T::WTM + i * 32 >= M) continue;  // wave-uniform: a per-lane test lets the last MFMAs' operand reads sink under it
 #pragma unroll
     for (int j = 0; j < T::TJ; ++j)
 #pragma unroll
@@ -463,9 +463,8 @@ int64_t i8_tiles(int64_t M, int64_t N, int tile) {
 int64_t i8_split_bytes(const I8Plan& p, int64_t M, int64_t N) {
   return p.splits > 1 ? p.splits * i8_tiles(M, N, p.tile) * p.tile * (p.tile == 256 ? 256 : 128) * 4 : 0;
 }
-// Costs in microseconds, measured: a 128-k stage takes a + b L at L =
-// workgroups / 256 up to one per CU, then (a + b) times the rounds; a split adds
-// 2.5 us and 0.27 us per MB of int32 sums. Fitted to 78 shapes (M 1..4096, N
+// The cheapest tile and number of K runs by GridCost over 128-k stages (measured
+// on this kernel); a split adds 2.5 us and 0.27 us per MB of int32 sums. Fitted to 78 shapes (M 1..4096, N
 // 1024..14336, K 1024..8192): the choice is within 0.6% of the best of all plans
 // on average. With the quantizer, N = K = 8192: M = 1 35 -> 20 us, 32 35 -> 21,
 // 128 39 -> 26 us; N = 2048, K = 8192, M = 64: 36 -> 17 us; N = 11008, K = 4096,
@@ -476,17 +475,14 @@ I8Plan i8_plan(int64_t M, int64_t N, int64_t K, bool may_split) {
   I8Plan best{128, 1};
   double least = 0;
   for (int tile = 256; tile >= 64; tile /= 2) {
-    const double c0 = tile == 256 ? 7.0 : tile == 128 ? 4.5 : 4.7;
-    const double a = tile == 256 ? 0.82 : tile == 128 ? 0.39 : 0.32;
-    const double b = tile == 256 ? 1.05 : tile == 128 ? 0.206 : 0.12;
+    const intent::GridCost cost = tile == 256   ? intent::GridCost{7.0, 0.82, 1.05}
+                                  : tile == 128 ? intent::GridCost{4.5, 0.39, 0.206}
+                                                : intent::GridCost{4.7, 0.32, 0.12};
     for (int splits = 1; splits <= (may_split ? 8 : 1) && splits <= stages; splits *= 2) {
       const I8Plan p{tile, splits};
       if (i8_split_bytes(p, M, N) > (64 << 20)) break;
-      const int64_t wgs = i8_tiles(M, N, tile) * splits;
-      const double L = (double)wgs / 256;
-      const double stage = L <= 1 ? a + b * L : (a + b) * (L + (double)((wgs + 255) / 256)) / 2;
-      const double split = splits > 1 ? 2.5 + 0.27e-6 * (double)i8_split_bytes(p, M, N) : 0;
-      const double c = c0 + (double)((stages + splits - 1) / splits) * stage + split;
+      const double c = cost.us(i8_tiles(M, N, tile) * splits, (double)((stages + splits - 1) / splits)) +
+                       (splits > 1 ? 2.5 + 0.27e-6 * (double)i8_split_bytes(p, M, N) : 0);
       if (least == 0 || c < least) {
         least = c;
         best = p;
