@@ -460,6 +460,14 @@ int intent_deepgemm_fp8(const uint8_t* a, int64_t M, int64_t K, int64_t a_ld,
                         const uint8_t* b, int64_t N, int64_t b_ld,
                         const float* b_scales, int64_t b_scales_ld,
                         void* out, int64_t out_ld, void* stream);
+/* The same product with a workspace for a K split (see intent_w8a16_matmul_ws). */
+size_t intent_deepgemm_fp8_workspace_size(int64_t M, int64_t K, int64_t N);
+int intent_deepgemm_fp8_ws(const uint8_t* a, int64_t M, int64_t K, int64_t a_ld,
+                           const float* a_scales, int64_t a_scales_ld,
+                           const uint8_t* b, int64_t N, int64_t b_ld,
+                           const float* b_scales, int64_t b_scales_ld,
+                           void* out, int64_t out_ld,
+                           void* workspace, size_t workspace_bytes, void* stream);
 
 /* FP8 x FP8 -> FP8 GEMM. Replaces fp8_e4m3_matmul (format 0) and
  * fp8_e5m2_matmul (format 1) (examples/kernels/contraction/weight_only_int4.py:

@@ -78,6 +78,8 @@ SIGNATURES: dict[str, tuple[list, object]] = {
     "intent_fp4_bf16_matmul": ([P, I64, I64, I64, P, I64, I64, P, I64, P], INT),
     "intent_fp8_gemm": ([P, I64, I64, I64, P, I64, I64, INT, P, I64, P], INT),
     "intent_deepgemm_fp8": ([P, I64, I64, I64, P, I64, P, I64, I64, P, I64, P, I64, P], INT),
+    "intent_deepgemm_fp8_workspace_size": ([I64, I64, I64], SIZE),
+    "intent_deepgemm_fp8_ws": ([P, I64, I64, I64, P, I64, P, I64, I64, P, I64, P, I64, P, SIZE, P], INT),
     "intent_moe_workspace_size": ([I64, I64, I64, I64, I64, I64], SIZE),
     "intent_moe_expert_ffn_w4": ([P, P, I64, I64, I64, I64, INT, P, P, P, P, P, P, I64, I64, P, P, SIZE, P, P, P],
                                  INT),

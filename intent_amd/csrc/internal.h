@@ -39,6 +39,18 @@ int fill_launch(void* out, int64_t rows, int64_t cols, int64_t ld, int elem_byte
 // query fails, which callers treat as "no round-fitting").
 int cu_count();
 
+// Time of a tiled kernel in microseconds, from measurements of it: base, plus
+// per stage of the K loop a + b L while the L = workgroups / 256 do not exceed
+// one per CU, and (a + b) times the rounds beyond (half a round's cost for a
+// partly filled one, since its workgroups share a CU with those before them).
+struct GridCost {
+  double base, a, b;
+  double us(int64_t workgroups, double stages) const {
+    const double L = (double)workgroups / 256;
+    return base + stages * (L <= 1 ? a + b * L : (a + b) * (L + (double)((workgroups + 255) / 256)) / 2);
+  }
+};
+
 }  // namespace intent
 
 #define INTENT_REQUIRE(cond, code, ...)            \

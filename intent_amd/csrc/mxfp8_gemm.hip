@@ -1012,26 +1012,33 @@ __global__ __launch_bounds__(256, 1) void i8_gemm_kn_kernel(const uint8_t* __res
 // (sum_k lhs*rhs) * lhs_scale * rhs_scale). The f32 scales cannot ride the
 // MFMA's E8M0 scale operand, so each 128-k stage is summed into a fresh
 // accumulator and folded into the main one with one fma per element
-// ("2xacc"): main += fresh * (lhs_scale * rhs_scale). Tiles of 256 x 128, four
-// waves of 128 x 64; the per-row scales of a stage travel with it by DMA.
-using TDg = mp::Tile<256, 128, 2, 2>;
-
-__global__ __launch_bounds__(256, 1) void deepgemm_fp8_kernel(const uint8_t* __restrict__ a, int64_t lda, int M,
-                                                              const float* __restrict__ sa, int64_t ld_sa,
-                                                              const uint8_t* __restrict__ b, int64_t ldb, int N,
-                                                              const float* __restrict__ sb, int64_t ld_sb, int K,
-                                                              uint16_t* __restrict__ out, int64_t ldo, int mblocks) {
-  using T = TDg;
+// ("2xacc"): main += fresh * (lhs_scale * rhs_scale). Tiles of 128 x 128 or 64 x
+// 128 with four waves; two (three) workgroups per CU hide each other's stage
+// barrier and folds, which one 256 x 128 workgroup (one wave per SIMD) could not:
+// 4096^3 116 -> 96 us for the kernel. The per-row scales of a stage travel with it
+// by DMA.
+//
+// kSplit: blockIdx.y takes one run of the 128-k blocks and leaves its f32 sums
+// in the register layout (1 KB contiguous per store) for deepgemm_combine_kernel.
+template <class T, bool kSplit>
+__global__ __launch_bounds__(256, 2) void deepgemm_fp8_kernel(
+    const uint8_t* __restrict__ a, int64_t lda, int M, const float* __restrict__ sa, int64_t ld_sa,
+    const uint8_t* __restrict__ b, int64_t ldb, int N, const float* __restrict__ sb, int64_t ld_sb, int K,
+    void* __restrict__ out, int64_t ldo, int mblocks) {
   constexpr int SB = (T::BM + T::BN) * (mp::ROWB + 4);
   __shared__ __attribute__((aligned(1024))) char smem[2 * SB];
   int tmb, tnb;
   grid_tile(mblocks, 4, tmb, tnb);
   const int m0 = tmb * T::BM;
   const int n0 = tnb * T::BN;
+  const int blocks = K / mp::ROWB;
+  const int b0 = kSplit ? (int)((int64_t)blockIdx.y * blocks / gridDim.y) : 0;
+  const int b1 = kSplit ? (int)((int64_t)(blockIdx.y + 1) * blocks / gridDim.y) : blocks;
   mxdma::Rows<T::BM, T::NW, true> aop;
   mxdma::Rows<T::BN, T::NW, true> bop;
-  aop.init(a, lda, M, reinterpret_cast<const uint8_t*>(sa), ld_sa * 4, m0, T::wave(), 1);
-  bop.init(b, ldb, N, reinterpret_cast<const uint8_t*>(sb), ld_sb * 4, n0, T::wave(), 128);
+  aop.init(a + (int64_t)b0 * mp::ROWB, lda, M, reinterpret_cast<const uint8_t*>(sa + b0), ld_sa * 4, m0, T::wave(), 1);
+  bop.init(b + (int64_t)b0 * mp::ROWB, ldb, N, reinterpret_cast<const uint8_t*>(sb + b0), ld_sb * 4, n0, T::wave(),
+           128);
   i32x16 fresh[T::TI][T::TJ];
   f32x16 acc[T::TI][T::TJ];
 #pragma unroll
@@ -1046,13 +1053,75 @@ __global__ __launch_bounds__(256, 1) void deepgemm_fp8_kernel(const uint8_t* __r
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[i][j][e] = __builtin_fmaf(v[e], w, acc[i][j][e]);
   };
-  mxdma::dma_mainloop<T, mxdma::ScaleMode::kPromote>(smem, aop, bop, K / mp::ROWB, mxdma::SplitK{1, 0}, fresh,
-                                                     promote);
+  mxdma::dma_mainloop<T, mxdma::ScaleMode::kPromote>(smem, aop, bop, b1 - b0, mxdma::SplitK{1, 0}, fresh, promote);
+  if constexpr (kSplit) {
+    constexpr int BLK = T::TI * T::TJ * 4;
+    float* part = reinterpret_cast<float*>(out) +
+                  (((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * T::NW + T::wave()) * (BLK * 256) +
+                  (threadIdx.x & 63) * 4;
+#pragma unroll
+    for (int i = 0; i < T::TI; ++i) {
+      if (m0 + T::wave_m() * T::WTM + i * 32 >= M) continue;  // wave-uniform: a per-lane test lets the last MFMAs' operand reads sink under it
+#pragma unroll
+      for (int j = 0; j < T::TJ; ++j)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          *reinterpret_cast<f32x4*>(part + ((i * T::TJ + j) * 4 + g) * 256) =
+              f32x4{acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
+    }
+    return;
+  }
   mxdma::store_rows_lds<T, 2>(smem, m0, n0, M, N, reinterpret_cast<char*>(out), ldo * 2, [&](int i, int j, int g) {
     const f32x16& v = acc[i][j];
-    return mxdma::Piece<2>{{f32_to_bf16_rne(v[4 * g]) | ((uint32_t)f32_to_bf16_rne(v[4 * g + 1]) << 16),
-                            f32_to_bf16_rne(v[4 * g + 2]) | ((uint32_t)f32_to_bf16_rne(v[4 * g + 3]) << 16)}};
+    return mxdma::Piece<2>{{bf16x2_rne(v[4 * g], v[4 * g + 1]), bf16x2_rne(v[4 * g + 2], v[4 * g + 3])}};
   });
+}
+
+// out = bf16(the runs' sums added in order); one wave per 32 x 32 block.
+template <class T>
+__global__ __launch_bounds__(64) void deepgemm_combine_kernel(const float* __restrict__ part, int S, int tiles, int M,
+                                                              int N, uint16_t* __restrict__ out, int64_t ldo, int vec,
+                                                              int mblocks) {
+  constexpr int BLK = T::TI * T::TJ * 4;
+  int id = blockIdx.x;  // ((tile * NW + wave) * TI + i) * TJ + j
+  const int j = id % T::TJ;
+  id /= T::TJ;
+  const int i = id % T::TI;
+  id /= T::TI;
+  const int wave = id % T::NW, tile = id / T::NW;
+  int tmb, tnb;
+  grouped_tile(xcd_swizzle(tile, tiles), mblocks, tiles / mblocks, 4, tmb, tnb);
+  const int lane = threadIdx.x;
+  const int m = tmb * T::BM + (wave % T::WM) * T::WTM + i * 32 + (lane & 31);
+  const int n0 = tnb * T::BN + (wave / T::WM) * T::WTN + j * 32 + (lane >> 5) * 4;
+  if (m >= M) return;
+  const float* src = part + ((int64_t)tile * T::NW + wave) * (BLK * 256) + (i * T::TJ + j) * 1024 + lane * 4;
+  const int64_t stride = (int64_t)tiles * T::NW * (BLK * 256);
+  f32x4 v[4];
+#pragma unroll
+  for (int g = 0; g < 4; ++g) v[g] = *reinterpret_cast<const f32x4*>(src + g * 256);
+  for (int p = 1; p < S; ++p) {
+    src += stride;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const f32x4 o = *reinterpret_cast<const f32x4*>(src + g * 256);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) v[g][c] += o[c];
+    }
+  }
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    const int n = n0 + g * 8;
+    uint16_t* o = out + (int64_t)m * ldo + n;
+    const u32x2 pk{bf16x2_rne(v[g][0], v[g][1]), bf16x2_rne(v[g][2], v[g][3])};
+    if (vec && n + 3 < N) {
+      *reinterpret_cast<u32x2*>(o) = pk;
+    } else {
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        if (n + c < N) o[c] = (uint16_t)(pk[c >> 1] >> (16 * (c & 1)));
+    }
+  }
 }
 
 // FP8 x FP8 -> FP8 GEMM (fp8_e4m3_matmul, fp8_e5m2_matmul,
@@ -1333,10 +1402,69 @@ extern "C" int intent_i8_gemm_i32_kn(const int8_t* a, int64_t M, int64_t K, int6
   return intent::launch_status("i8_gemm_i32_kn");
 }
 
-extern "C" int intent_deepgemm_fp8(const uint8_t* a, int64_t M, int64_t K, int64_t a_ld, const float* a_scales,
-                                   int64_t a_scales_ld, const uint8_t* b, int64_t N, int64_t b_ld,
-                                   const float* b_scales, int64_t b_scales_ld, void* out, int64_t out_ld,
-                                   void* stream) {
+namespace {
+
+struct DgPlan {
+  int tile;    // rows of the tile (128 or 64; 128 columns)
+  int splits;  // K runs (1: no workspace)
+};
+int64_t dg_tiles(int64_t M, int64_t N, int tile) { return ((M + tile - 1) / tile) * ((N + 127) / 128); }
+int64_t dg_split_bytes(const DgPlan& p, int64_t M, int64_t N) {
+  return p.splits > 1 ? p.splits * dg_tiles(M, N, p.tile) * p.tile * 128 * 4 : 0;
+}
+// The cheaper of 128- and 64-row tiles and up to eight K runs by GridCost over
+// 128-k stages (measured on this kernel); a split adds 2.2 us and 0.25 us per MB.
+// Fitted to 66 shapes (M 1..4096, N 1024..14336, K 1024..7168): within 2.2% of the
+// best of all plans on average. 256-row tiles (one wave per SIMD) lost at every
+// shape. With the quantizer, N = K = 4096: M = 1 46 -> 14 us, 64 47 -> 17, 256
+// 56 -> 23, 1024 64 -> 42, 4096 142 -> 121 us; N = 14336, K = 4096, M = 384: 62 -> 48.
+DgPlan dg_plan(int64_t M, int64_t N, int64_t K, bool may_split) {
+  const int64_t stages = K / mp::ROWB;
+  DgPlan best{128, 1};
+  double least = 0;
+  for (int tile = 128; tile >= 64; tile /= 2) {
+    const intent::GridCost cost = tile == 128 ? intent::GridCost{4.0, 0.61, 0.20} : intent::GridCost{4.1, 0.48, 0.05};
+    for (int splits = 1; splits <= (may_split ? 8 : 1) && splits <= stages; splits *= 2) {
+      const DgPlan p{tile, splits};
+      if (dg_split_bytes(p, M, N) > (64 << 20)) break;
+      const double c = cost.us(dg_tiles(M, N, tile) * splits, (double)((stages + splits - 1) / splits)) +
+                       (splits > 1 ? 2.2 + 0.25e-6 * (double)dg_split_bytes(p, M, N) : 0);
+      if (least == 0 || c < least) {
+        least = c;
+        best = p;
+      }
+    }
+  }
+  return best;
+}
+
+template <class T>
+int dg_launch(const uint8_t* a, int64_t M, int64_t K, int64_t a_ld, const float* a_scales, int64_t a_scales_ld,
+              const uint8_t* b, int64_t N, int64_t b_ld, const float* b_scales, int64_t b_scales_ld, void* out,
+              int64_t out_ld, int splits, void* ws, void* stream) {
+  const int mblocks = (int)((M + T::BM - 1) / T::BM);
+  const int64_t grid = (int64_t)mblocks * ((N + T::BN - 1) / T::BN);
+  const int64_t cgrid = grid * T::NW * T::TI * T::TJ;
+  INTENT_REQUIRE(cgrid < (1ll << 31), INTENT_ERR_UNSUPPORTED, "deepgemm_fp8: grid too large");
+  hipStream_t st = (hipStream_t)stream;
+  if (splits == 1) {
+    hipLaunchKernelGGL((deepgemm_fp8_kernel<T, false>), dim3((unsigned)grid), dim3(256), 0, st, a, a_ld, (int)M,
+                       a_scales, a_scales_ld, b, b_ld, (int)N, b_scales, b_scales_ld, (int)K, out, out_ld, mblocks);
+    return intent::launch_status("deepgemm_fp8");
+  }
+  hipLaunchKernelGGL((deepgemm_fp8_kernel<T, true>), dim3((unsigned)grid, splits), dim3(256), 0, st, a, a_ld, (int)M,
+                     a_scales, a_scales_ld, b, b_ld, (int)N, b_scales, b_scales_ld, (int)K, ws, 0, mblocks);
+  const int s = intent::launch_status("deepgemm_fp8");
+  if (s != INTENT_OK) return s;
+  const int vec = out_ld % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & 7) == 0;
+  hipLaunchKernelGGL((deepgemm_combine_kernel<T>), dim3((unsigned)cgrid), dim3(64), 0, st, (const float*)ws, splits,
+                     (int)grid, (int)M, (int)N, (uint16_t*)out, out_ld, vec, mblocks);
+  return intent::launch_status("deepgemm_fp8");
+}
+
+int dg_entry(const uint8_t* a, int64_t M, int64_t K, int64_t a_ld, const float* a_scales, int64_t a_scales_ld,
+             const uint8_t* b, int64_t N, int64_t b_ld, const float* b_scales, int64_t b_scales_ld, void* out,
+             int64_t out_ld, void* ws, size_t ws_bytes, void* stream) {
   intent::clear_error();
   INTENT_REQUIRE(M >= 0 && N >= 0 && K >= 0 && M <= INT32_MAX && N <= INT32_MAX && K <= INT32_MAX,
                  INTENT_ERR_INVALID_ARGUMENT, "bad extents");
@@ -1352,13 +1480,35 @@ extern "C" int intent_deepgemm_fp8(const uint8_t* a, int64_t M, int64_t K, int64
   INTENT_REQUIRE(intent::fits_offset(M, a_ld) && intent::fits_offset(N, b_ld) &&
                      intent::fits_offset(M, a_scales_ld * 4) && intent::fits_offset(N / 128 + 1, b_scales_ld * 4),
                  INTENT_ERR_UNSUPPORTED, "deepgemm_fp8: operand too large for 31-bit buffer offsets");
-  const int mblocks = (int)((M + TDg::BM - 1) / TDg::BM);
-  const int64_t grid = (int64_t)mblocks * ((N + TDg::BN - 1) / TDg::BN);
-  INTENT_REQUIRE(grid < (1ll << 31), INTENT_ERR_UNSUPPORTED, "deepgemm_fp8: grid too large");
-  hipLaunchKernelGGL(deepgemm_fp8_kernel, dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, a, a_ld, (int)M,
-                     a_scales, a_scales_ld, b, b_ld, (int)N, b_scales, b_scales_ld, (int)K, (uint16_t*)out, out_ld,
-                     mblocks);
-  return intent::launch_status("deepgemm_fp8");
+  DgPlan p = dg_plan(M, N, K, true);
+  if (p.splits > 1 && !(ws && intent::aligned16(ws) && ws_bytes >= (size_t)dg_split_bytes(p, M, N)))
+    p = dg_plan(M, N, K, false);
+  const auto launch = p.tile == 128 ? dg_launch<mp::Tile<128, 128, 2, 2>> : dg_launch<mp::Tile<64, 128, 2, 2>>;
+  return launch(a, M, K, a_ld, a_scales, a_scales_ld, b, N, b_ld, b_scales, b_scales_ld, out, out_ld, p.splits, ws,
+                stream);
+}
+
+}  // namespace
+
+extern "C" int intent_deepgemm_fp8(const uint8_t* a, int64_t M, int64_t K, int64_t a_ld, const float* a_scales,
+                                   int64_t a_scales_ld, const uint8_t* b, int64_t N, int64_t b_ld,
+                                   const float* b_scales, int64_t b_scales_ld, void* out, int64_t out_ld,
+                                   void* stream) {
+  return dg_entry(a, M, K, a_ld, a_scales, a_scales_ld, b, N, b_ld, b_scales, b_scales_ld, out, out_ld, nullptr, 0,
+                  stream);
+}
+
+extern "C" size_t intent_deepgemm_fp8_workspace_size(int64_t M, int64_t K, int64_t N) {
+  if (M <= 0 || N <= 0 || K <= 0 || K % 128 != 0) return 0;
+  return (size_t)dg_split_bytes(dg_plan(M, N, K, true), M, N);
+}
+
+extern "C" int intent_deepgemm_fp8_ws(const uint8_t* a, int64_t M, int64_t K, int64_t a_ld, const float* a_scales,
+                                      int64_t a_scales_ld, const uint8_t* b, int64_t N, int64_t b_ld,
+                                      const float* b_scales, int64_t b_scales_ld, void* out, int64_t out_ld,
+                                      void* workspace, size_t workspace_bytes, void* stream) {
+  return dg_entry(a, M, K, a_ld, a_scales, a_scales_ld, b, N, b_ld, b_scales, b_scales_ld, out, out_ld, workspace,
+                  workspace_bytes, stream);
 }
 
 extern "C" int intent_fp8_gemm(const uint8_t* a, int64_t M, int64_t K, int64_t a_ld, const uint8_t* bt, int64_t N,

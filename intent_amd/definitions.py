@@ -873,8 +873,13 @@ def _deepgemm_check(env: dict) -> None:
 def _deepgemm_launch(v: dict, env: dict, stream: int, workspace) -> str:
     lhs, rhs, ls, rs, out = v["lhs"], v["rhs"], v["lhs_scale"], v["rhs_scale"], v["output"]
     M, KB, N = env["M"], env["KB"], env["N"]
-    _native.call("intent_deepgemm_fp8", _ptr(lhs), M, KB * 128, KB * 128, _ptr(ls), KB, _ptr(rhs), N, KB * 128,
-                 _ptr(rs), KB, _ptr(out), _ld(out), stream)
+    scratch = _split_scratch(_native.library().intent_deepgemm_fp8_workspace_size(M, KB * 128, N), out)
+    if scratch is not None:
+        _native.call("intent_deepgemm_fp8_ws", _ptr(lhs), M, KB * 128, KB * 128, _ptr(ls), KB, _ptr(rhs), N, KB * 128,
+                     _ptr(rs), KB, _ptr(out), _ld(out), _ptr(scratch), scratch.numel(), stream)
+    else:
+        _native.call("intent_deepgemm_fp8", _ptr(lhs), M, KB * 128, KB * 128, _ptr(ls), KB, _ptr(rhs), N, KB * 128,
+                     _ptr(rs), KB, _ptr(out), _ld(out), stream)
     return "intent_deepgemm_fp8"
 
 

@@ -996,6 +996,23 @@ def test_deepgemm_fp8(gpu, threads, M, KB, N):
     assert np.max(np.abs(_bf16_bits_to_f64(got) - ref)) <= 1e-2 * np.abs(ref).max()
 
 
+# K split over workgroups (block scales of each run) on both tiles, off their rows and columns, with runs of
+# unequal length and an output stride that rules out the vector stores.
+@pytest.mark.parametrize("M,KB,N,pad", [(1, 32, 4096, 0), (17, 9, 130, 0), (65, 32, 257, 3), (129, 56, 130, 0),
+                                        (300, 25, 200, 0)])
+def test_deepgemm_fp8_split_k(gpu, threads, M, KB, N, pad):
+    a, b = _fp8_bits(M + 1, (M, KB * 128)), _fp8_bits(N + 2, (N, KB * 128))
+    g = torch.Generator().manual_seed(M + N)
+    sa, sb = (torch.rand(M, KB, generator=g) + 0.25).numpy(), (torch.rand((N + 127) // 128, KB, generator=g) + 0.25).numpy()
+    assert _native.library().intent_deepgemm_fp8_workspace_size(M, KB * 128, N) > 0
+    out = torch.zeros(M, N + pad, dtype=torch.bfloat16, device="cuda")[:, :N]
+    art(intent.deepgemm_fp8_2xacc)(dev(a).view(torch.float8_e4m3fn).view(M, KB, 128),
+                                   dev(b).view(torch.float8_e4m3fn).view(N, KB, 128), dev(sa), dev(sb), out)
+    ref = _bf16_bits_to_f64(oracle.deepgemm_fp8(a, sa, b, sb, threads))
+    # bf16 output: one rounding of ~2^-8 relative on either side
+    assert np.max(np.abs(out.double().cpu().numpy() - ref)) <= 1e-2 * np.abs(ref).max()
+
+
 def test_deepgemm_fp8_reference_inputs(gpu):
     # The reference's case and input construction (experiments/cpu/providers/mojo/
     # contraction.py:227-236: per-block absmax scaling to 448, M = N = K = 4096),
