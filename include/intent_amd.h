@@ -620,7 +620,9 @@ int intent_grouped_gemm_kn(const void* x, int64_t rows, int64_t K, int64_t x_ld,
  * with f32 accumulation; a token's contributions are added in member order
  * (deterministic). Out-of-range routing entries are clamped, never
  * dereferenced. D and F multiples of 64. workspace: at least
- * intent_moe_expert_ffn_workspace_size(T, R, D, F) bytes, 16-byte aligned.
+ * intent_moe_expert_ffn_workspace_size(T, R, D, F) bytes, 16-byte aligned (the
+ * last 12 R D bytes of it, present for R <= 4096, only let the second projection
+ * split K: a call with less runs without).
  */
 size_t intent_moe_expert_ffn_workspace_size(int64_t T, int64_t R, int64_t D, int64_t F);
 int intent_moe_expert_ffn(const void* x, int64_t T, int64_t D, int64_t x_ld, const int32_t* route_offsets,

@@ -149,18 +149,31 @@ INTENT_DEVICE void grouped_store_lds(const f32x16 (&acc)[T::TI][T::TJ], char* ld
   }
 }
 
-template <class T, class Math, bool kGather, GEpi E>
+// kFew: few rows per group (the time is the weights' stream). Row tiles are
+// then outermost, so that the tiles past the last one, which exit at once, do
+// not take CU slots from between the working ones, and blockIdx.y takes one run
+// of the K stages, whose f32 result goes to out (run 0) or more + (run - 1) * part_stride.
+template <class T, class Math, bool kGather, GEpi E, bool kFew = false>
 __global__ __launch_bounds__(T::NT, 1) void grouped_kn_kernel(
     const uint16_t* __restrict__ x, int64_t ldx, const int32_t* __restrict__ offsets, int G, int rows,
     const int32_t* __restrict__ members, const int32_t* __restrict__ route_token, int nroutes, int ntokens,
     const float* __restrict__ route_weights, const uint16_t* __restrict__ w, int64_t ldw, int64_t gstride, int N, int K,
-    int ntiles, void* __restrict__ out, int64_t ldo) {
+    int ntiles, void* __restrict__ out, int64_t ldo, float* __restrict__ more, int64_t part_stride) {
   __shared__ __attribute__((aligned(16))) char buf0[T::STAGE_BYTES];
   __shared__ __attribute__((aligned(16))) char buf1[T::STAGE_BYTES];
-  const int bid = xcd_swizzle(blockIdx.x, gridDim.x);
-  const GroupTile tile = find_tile(offsets, G, rows, bid % ntiles, T::BM);
+  const int ctiles = (int)gridDim.x / ntiles;
+  const int bid = kFew ? (int)blockIdx.x : xcd_swizzle(blockIdx.x, gridDim.x);
+  const GroupTile tile = find_tile(offsets, G, rows, kFew ? bid / ctiles : bid % ntiles, T::BM);
   if (tile.g < 0) return;  // workgroup-uniform
-  const int n0 = (bid / ntiles) * T::BN;
+  const int n0 = (kFew ? bid % ctiles : bid / ntiles) * T::BN;
+  int nk = K / 64;
+  if constexpr (kFew) {
+    const int s0 = (int)((int64_t)blockIdx.y * nk / gridDim.y), s1 = (int)((int64_t)(blockIdx.y + 1) * nk / gridDim.y);
+    x += s0 * 64;
+    w += (int64_t)s0 * 64 * ldw;
+    nk = s1 - s0;
+    if (blockIdx.y > 0) out = more + (int64_t)(blockIdx.y - 1) * part_stride;
+  }
   const int wave = T::wave();
   mp::DmaKNOperand<T::BN, T::NW> bop;
   bop.init(w + tile.g * gstride + n0, ldw, N - n0, wave);
@@ -174,7 +187,7 @@ __global__ __launch_bounds__(T::NT, 1) void grouped_kn_kernel(
   aop.init(rows_src, tile.start, wave);
   f32x16 acc[T::TI][T::TJ];
   mp::mainloop_kn<T, Math, mp::DmaRowsOperand<T::BM, Rows, T::NW>, mp::DmaKNOperand<T::BN, T::NW>, true>(
-      aop, bop, K / 64, buf0, buf1, acc);
+      aop, bop, nk, buf0, buf1, acc);
   constexpr bool kBf16 = std::is_same<Math, mp::BF16Math>::value;
   grouped_store_lds<T, E, kBf16>(acc, buf0, buf1, tile, n0, N, members, nroutes, route_weights, out, ldo);
 }
@@ -192,17 +205,17 @@ inline int kn_shape_check(int64_t K, int64_t N, int64_t w_ld, const void* w, con
   return INTENT_OK;
 }
 
-template <class Math, bool kGather, GEpi E>
+template <class Math, bool kGather, GEpi E, class T = GTile, bool kFew = false>
 inline void launch_grouped(const void* x, int64_t x_ld, const int32_t* offsets, int64_t G, int64_t rows,
                     const int32_t* members, const int32_t* route_token, int64_t nroutes, int64_t ntokens,
                     const float* route_weights, const void* w, int64_t w_ld, int64_t gstride, int64_t N, int64_t K,
-                    int ntiles, void* out, int64_t out_ld, hipStream_t st) {
-  using T = GTile;
+                    int ntiles, void* out, int64_t out_ld, hipStream_t st, int parts = 1, float* more = nullptr,
+                    int64_t part_stride = 0) {
   const int64_t grid = (int64_t)ntiles * ((N + T::BN - 1) / T::BN);
-  hipLaunchKernelGGL((grouped_kn_kernel<T, Math, kGather, E>), dim3((unsigned)grid), dim3(T::NT), 0, st,
+  hipLaunchKernelGGL((grouped_kn_kernel<T, Math, kGather, E, kFew>), dim3((unsigned)grid, parts), dim3(T::NT), 0, st,
                      (const uint16_t*)x, x_ld, offsets, (int)G, (int)rows, members, route_token, (int)nroutes,
                      (int)ntokens, route_weights, (const uint16_t*)w, w_ld, gstride, (int)N, (int)K, ntiles, out,
-                     out_ld);
+                     out_ld, more, part_stride);
 }
 
 }  // namespace gkn

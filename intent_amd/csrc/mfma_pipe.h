@@ -970,7 +970,7 @@ INTENT_DEVICE Frag kn_frag(const char* b, uint32_t addr0, uint32_t addr1) {
 template <class T>
 struct KNAddr {
   static constexpr int RB = T::BN * 2;
-  static_assert(T::WTN % 32 == 0, "column blocks of 32");
+  static_assert(T::WTN % 64 == 0, "bit 1 of a wave's window index comes from j alone");
   uint32_t base[2];
   INTENT_DEVICE void init() {
     const int lane = threadIdx.x & 63;

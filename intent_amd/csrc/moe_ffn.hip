@@ -198,7 +198,8 @@ __global__ __launch_bounds__(kListThreads) void token_member_list_lds_kernel(
 __global__ __launch_bounds__(256) void token_combine_kernel(const float* __restrict__ contrib, int64_t ldc,
                                                             const int32_t* __restrict__ start,
                                                             const int32_t* __restrict__ list, int T, int D,
-                                                            float* __restrict__ y, int64_t ldy) {
+                                                            float* __restrict__ y, int64_t ldy, int parts,
+                                                            const float* __restrict__ more, int64_t part_stride) {
   const int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int d4 = (D + 3) / 4;
   if (id >= (int64_t)T * d4) return;
@@ -209,14 +210,23 @@ __global__ __launch_bounds__(256) void token_combine_kernel(const float* __restr
   if (d + 3 < D && (ldy & 3) == 0 && (ldc & 3) == 0) {
     f32x4 acc = *reinterpret_cast<const f32x4*>(yo);
     for (int k = b; k < e; ++k) {
-      const f32x4 c = *reinterpret_cast<const f32x4*>(contrib + (int64_t)list[k] * ldc + d);
+      f32x4 c = *reinterpret_cast<const f32x4*>(contrib + (int64_t)list[k] * ldc + d);
+      for (int p = 1; p < parts; ++p) {
+        const f32x4 o = *reinterpret_cast<const f32x4*>(more + (p - 1) * part_stride + (int64_t)list[k] * ldc + d);
+        c = f32x4{__fadd_rn(c[0], o[0]), __fadd_rn(c[1], o[1]), __fadd_rn(c[2], o[2]), __fadd_rn(c[3], o[3])};
+      }
       acc = f32x4{__fadd_rn(acc[0], c[0]), __fadd_rn(acc[1], c[1]), __fadd_rn(acc[2], c[2]), __fadd_rn(acc[3], c[3])};
     }
     *reinterpret_cast<f32x4*>(yo) = acc;
   } else {
     for (int c = 0; c < 4 && d + c < D; ++c) {
       float acc = yo[c];
-      for (int k = b; k < e; ++k) acc = __fadd_rn(acc, contrib[(int64_t)list[k] * ldc + d + c]);
+      for (int k = b; k < e; ++k) {
+        const int64_t o = (int64_t)list[k] * ldc + d + c;
+        float v = contrib[o];
+        for (int p = 1; p < parts; ++p) v = __fadd_rn(v, more[(p - 1) * part_stride + o]);
+        acc = __fadd_rn(acc, v);
+      }
       yo[c] = acc;
     }
   }
@@ -224,8 +234,38 @@ __global__ __launch_bounds__(256) void token_combine_kernel(const float* __restr
 
 size_t round256(size_t v) { return (v + 255) & ~(size_t)255; }
 
+constexpr int kFfnParts = 4;        // K runs of the second projection, at most
+constexpr int64_t kFewRows = 4096;  // routes up to which the workspace has room for them
+
+// Tiles of both projections for R routes over E experts. Few routes per expert:
+// the time is the experts' weights, and a 256 x 256 tile at one workgroup per CU
+// keeps 32 KB of them in flight and copies 256 rows for a handful of routes
+// (and the second projection has D / 256 tiles per expert: 128 workgroups at
+// E = 8, D = 4096). 64-row tiles run two or three workgroups per CU; columns and K
+// runs are chosen for about 512 workgroups. E = 8, D = 4096, F = 14336, whole layer:
+// T = 1 348 -> 152 us, 16 498 -> 320, 200 531 -> 346 (5.5 TB/s), 400 553 -> 412 us.
+// The lines: 50 routes per expert 346 us (64 rows) against 373 (128), 64 383 (128);
+// 100 412 (128) against 553 (256), 125 (E = 32) 522 against 520, 150 622 against 579.
+struct FfnPlan {
+  int rows;      // of a tile
+  int up, down;  // columns of a tile of the first and second projection
+  int parts;     // K runs of the second projection
+};
+FfnPlan ffn_plan(int64_t E, int64_t R, int64_t D, int64_t F) {
+  if (R > 115 * E) return {256, 256, 256, 1};
+  const int64_t busy = R < E ? R : E;  // experts with a route, about
+  FfnPlan p{R > 52 * E ? 128 : 64, 128, 128, 1};
+  if (p.rows == 64) {
+    if (busy * ((F + 255) / 256) >= 320) p.up = 256;
+    if (busy * ((D + 255) / 256) * kFfnParts >= 400) p.down = 256;
+  }
+  const int64_t tiles = busy * ((D + p.down - 1) / p.down);
+  while (p.parts < kFfnParts && tiles * p.parts < 400 && F / 64 >= 2 * p.parts && R <= kFewRows) p.parts *= 2;
+  return p;
+}
+
 struct FfnLayout {
-  size_t hidden, contrib, count, start, list, bytes;
+  size_t hidden, contrib, count, start, list, base, parts, bytes;
 };
 
 FfnLayout ffn_layout(int64_t T, int64_t R, int64_t D, int64_t F) {
@@ -236,6 +276,9 @@ FfnLayout ffn_layout(int64_t T, int64_t R, int64_t D, int64_t F) {
   L.count = o;   o = round256(o + sizeof(int32_t) * (size_t)T);
   L.start = o;   o = round256(o + sizeof(int32_t) * (size_t)(T + 1));
   L.list = o;    o = round256(o + sizeof(int32_t) * (size_t)R);
+  L.base = o;  // enough for a call without K runs
+  L.parts = o;
+  if (R <= kFewRows) o = round256(o + sizeof(float) * (size_t)R * D * (kFfnParts - 1));
   L.bytes = o;
   return L;
 }
@@ -269,7 +312,7 @@ extern "C" int intent_moe_expert_ffn(const void* x, int64_t T, int64_t D, int64_
   INTENT_REQUIRE(intent::fits_offset(T, x_ld * 2) && intent::fits_offset(R, F * 2) && intent::fits_offset(R, D * 4),
                  INTENT_ERR_UNSUPPORTED, "moe_expert_ffn: operands exceed 31-bit buffer offsets");
   const FfnLayout L = ffn_layout(T, R, D, F);
-  INTENT_REQUIRE(workspace && workspace_bytes >= L.bytes, INTENT_ERR_WORKSPACE, "workspace needs %zu bytes, got %zu",
+  INTENT_REQUIRE(workspace && workspace_bytes >= L.base, INTENT_ERR_WORKSPACE, "workspace needs %zu bytes, got %zu",
                  L.bytes, workspace_bytes);
   INTENT_REQUIRE(intent::aligned16(workspace), INTENT_ERR_ALIGNMENT, "workspace must be 16-byte aligned");
   char* ws = (char*)workspace;
@@ -279,18 +322,35 @@ extern "C" int intent_moe_expert_ffn(const void* x, int64_t T, int64_t D, int64_
   int32_t* start = (int32_t*)(ws + L.start);
   int32_t* list = (int32_t*)(ws + L.list);
   hipStream_t s = (hipStream_t)stream;
-  const int64_t ntiles = (R + GTile::BM - 1) / GTile::BM + E;
-  INTENT_REQUIRE(ntiles * ((F + GTile::BN - 1) / GTile::BN) < (1ll << 31), INTENT_ERR_UNSUPPORTED, "grid too large");
+  FfnPlan p = ffn_plan(E, R, D, F);
+  if (p.parts > 1 && workspace_bytes < L.bytes) p.parts = 1;
+  const int64_t ntiles = (R + p.rows - 1) / p.rows + E;
+  const int64_t least = p.up < p.down ? p.up : p.down;
+  INTENT_REQUIRE(ntiles * (((F > D ? F : D) + least - 1) / least) < (1ll << 31), INTENT_ERR_UNSUPPORTED,
+                 "grid too large");
   // hidden[i] = f16(relu(x[token(i)] @ w1[e])) for the members i of expert e
-  launch_grouped<mp::F16Math, true, GEpi::kReluF16>(x, x_ld, route_offsets, E, R, member_routes, route_token, NR, T,
-                                                    nullptr, w1, F, D * F, F, D, (int)ntiles, hidden, F, s);
-  st = intent::launch_status("grouped_kn_kernel<moe w1 relu>");
-  if (st != INTENT_OK) return st;
+  const auto up = [&](auto tile, auto few) {
+    launch_grouped<mp::F16Math, true, GEpi::kReluF16, decltype(tile), decltype(few)::value>(
+        x, x_ld, route_offsets, E, R, member_routes, route_token, NR, T, nullptr, w1, F, D * F, F, D, (int)ntiles, hidden,
+        F, s);
+    return intent::launch_status("grouped_kn_kernel<moe w1 relu>");
+  };
   // contrib[i] = route_weight * (hidden[i] @ w2[e])
-  launch_grouped<mp::F16Math, false, GEpi::kRouteWeight>(hidden, F, route_offsets, E, R, member_routes, nullptr, NR,
-                                                         T, route_weights, w2, D, F * D, D, F, (int)ntiles, contrib,
-                                                         D, s);
-  st = intent::launch_status("grouped_kn_kernel<moe w2 weighted>");
+  const auto down = [&](auto tile, auto few) {
+    launch_grouped<mp::F16Math, false, GEpi::kRouteWeight, decltype(tile), decltype(few)::value>(
+        hidden, F, route_offsets, E, R, member_routes, nullptr, NR, T, route_weights, w2, D, F * D, D, F, (int)ntiles,
+        contrib, D, s, p.parts, (float*)(ws + L.parts), R * D);
+    return intent::launch_status("grouped_kn_kernel<moe w2 weighted>");
+  };
+  const auto pick = [&](auto&& launch, int cols) {
+    if (p.rows == 256) return launch(GTile{}, std::false_type{});
+    if (p.rows == 128) return launch(mp::Tile<128, 128, 2, 2>{}, std::true_type{});
+    if (cols == 256) return launch(mp::Tile<64, 256, 1, 4>{}, std::true_type{});
+    return launch(mp::Tile<64, 128, 2, 2>{}, std::true_type{});
+  };
+  st = pick(up, p.up);
+  if (st != INTENT_OK) return st;
+  st = pick(down, p.down);
   if (st != INTENT_OK) return st;
   if (T <= kListLdsAll && R <= kListLdsAll) {
     const size_t lds = sizeof(int32_t) * (size_t)(2 * T + 1 + 2 * kListLdsAll);
@@ -311,6 +371,6 @@ extern "C" int intent_moe_expert_ffn(const void* x, int64_t T, int64_t D, int64_
   if (st != INTENT_OK) return st;
   const int64_t items = T * ((D + 3) / 4);
   hipLaunchKernelGGL(token_combine_kernel, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, s, contrib, D, start,
-                     list, (int)T, (int)D, y, y_ld);
+                     list, (int)T, (int)D, y, y_ld, p.parts, (const float*)(ws + L.parts), R * D);
   return intent::launch_status("token_combine");
 }

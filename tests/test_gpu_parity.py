@@ -1329,6 +1329,28 @@ def test_moe_expert_ffn_member_list(gpu, T, k):
     assert np.array_equal(lst[:len(order)], order)
 
 
+# Few routes per expert: the 64- and 128-row tiles (R / E up to 52 and 115) with both column widths, widths off
+# them, K runs of the second projection of unequal length, and a workspace without room for the runs.
+@pytest.mark.parametrize("T,D,E,k,F,runs", [(1, 64, 4, 1, 64, True), (3, 192, 8, 2, 320, True), (40, 320, 8, 2, 704, True),
+                                            (90, 128, 2, 1, 1088, True), (200, 576, 4, 2, 448, True),
+                                            (40, 320, 8, 2, 704, False), (300, 64, 3, 1, 1280, True)])
+def test_moe_expert_ffn_few_routes(gpu, threads, T, D, E, k, F, runs):
+    d = inputs.moe_ffn_f16(T + D, T=T, D=D, E=E, top_k=k, F=F, kind="random")
+    y0 = np.random.default_rng(T).standard_normal((T, D), dtype=np.float32)
+    dv = {key: dev(v) for key, v in d.items() if key != "y"}
+    y = dev(y0)
+    R, NR = len(d["member_routes"]), len(d["route_token"])
+    nbytes = int(_native.library().intent_moe_expert_ffn_workspace_size(T, R, D, F)) - (0 if runs else 1)
+    ws = torch.zeros(nbytes + 16, dtype=torch.uint8, device="cuda")
+    _native.call("intent_moe_expert_ffn", dv["x"].data_ptr(), T, D, D, dv["route_offsets"].data_ptr(), E,
+                 dv["member_routes"].data_ptr(), R, dv["route_token"].data_ptr(), dv["route_weights"].data_ptr(), NR,
+                 dv["w1"].data_ptr(), dv["w2"].data_ptr(), F, y.data_ptr(), D, ws.data_ptr(), nbytes,
+                 torch.cuda.current_stream().cuda_stream)
+    ref = oracle.moe_expert_ffn(d["x"], d["route_offsets"], d["member_routes"], d["route_token"], d["route_weights"],
+                                d["w1"], d["w2"], y=y0.copy(), threads=threads)
+    assert_close_rms(host(y) - y0, ref - y0, what=f"moe_expert_ffn few routes {T}x{D}x{F}")
+
+
 @pytest.mark.parametrize("T", [512, 4096])
 def test_moe_expert_ffn_reference_size(gpu, threads, T):
     # moe.py:6-10 (T = 4096, D = 4096, F = 14336, E = 8, top-2) and the config-4 token count,
