@@ -126,6 +126,15 @@ int intent_w4a16_gemm_ws(const void* x, int64_t M, int64_t K, int64_t x_ld,
                          int64_t group_size,
                          void* y, int64_t y_ld,
                          void* workspace, size_t workspace_bytes, void* stream);
+/* The entry that picks by M, with a workspace: as intent_w4a16_gemm_ws above M =
+ * 16; up to 16 rows a K split too where that beats the GEMV (size 0 elsewhere). */
+size_t intent_w4a16_matmul_workspace_size(int64_t M, int64_t K, int64_t N, int64_t group_size);
+int intent_w4a16_matmul_ws(const void* x, int64_t M, int64_t K, int64_t x_ld,
+                           const uint8_t* packed, int64_t N, int64_t packed_ld,
+                           const void* scales, const uint8_t* zeros, int64_t qparam_ld,
+                           int64_t group_size,
+                           void* y, int64_t y_ld,
+                           void* workspace, size_t workspace_bytes, void* stream);
 
 /*
  * W8A8: out[m,n] = bf16( f32(acc[m,n]) * a_scale[m] * w_scale[n] ), with

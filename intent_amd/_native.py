@@ -40,6 +40,8 @@ SIGNATURES: dict[str, tuple[list, object]] = {
     "intent_w8a16_matmul_ws": ([P, I64, I64, I64, P, I64, I64, P, P, I64, P, SIZE, P], INT),
     "intent_w4a16_gemm_workspace_size": ([I64, I64, I64, I64], SIZE),
     "intent_w4a16_gemm_ws": ([P, I64, I64, I64, P, I64, I64, P, P, I64, I64, P, I64, P, SIZE, P], INT),
+    "intent_w4a16_matmul_workspace_size": ([I64, I64, I64, I64], SIZE),
+    "intent_w4a16_matmul_ws": ([P, I64, I64, I64, P, I64, I64, P, P, I64, I64, P, I64, P, SIZE, P], INT),
     "intent_w8a8_gemm": ([P, I64, I64, I64, P, P, I64, I64, P, P, I64, P], INT),
     "intent_w8a8_gemm_workspace_size": ([I64, I64, I64], SIZE),
     "intent_w8a8_gemm_ws": ([P, I64, I64, I64, P, P, I64, I64, P, P, I64, P, SIZE, P], INT),

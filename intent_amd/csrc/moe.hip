@@ -680,19 +680,19 @@ INTENT_DEVICE void skinny_mainloop(char* lds, const void* x, const TRow& trow, c
                                    int nh, int used, f32x4 (&acc)[SkinnyCfg<TB>::NB][TB]) {
   using C = SkinnyCfg<TB>;
   if constexpr (TB == 1) {
-    sk::w4_mainloop<C::NB, TB, 1, C::HS, C::D>(lds, x, trow, w, wrow, nh, acc);
+    sk::w4_mainloop<C::NB, TB, 1, C::HS, C::D, false>(lds, x, trow, w, wrow, nh, acc);
   } else if constexpr (TB == 2) {
     if (used <= 1)
-      sk::w4_mainloop<C::NB, TB, 1, C::HS, C::D>(lds, x, trow, w, wrow, nh, acc);
+      sk::w4_mainloop<C::NB, TB, 1, C::HS, C::D, false>(lds, x, trow, w, wrow, nh, acc);
     else
-      sk::w4_mainloop<C::NB, TB, 2, C::HS, C::D>(lds, x, trow, w, wrow, nh, acc);
+      sk::w4_mainloop<C::NB, TB, 2, C::HS, C::D, false>(lds, x, trow, w, wrow, nh, acc);
   } else {
     if (used <= 2)
-      sk::w4_mainloop<C::NB, TB, 2, C::HS, C::D>(lds, x, trow, w, wrow, nh, acc);
+      sk::w4_mainloop<C::NB, TB, 2, C::HS, C::D, false>(lds, x, trow, w, wrow, nh, acc);
     else if (used == 3)
-      sk::w4_mainloop<C::NB, TB, 3, C::HS, C::D>(lds, x, trow, w, wrow, nh, acc);
+      sk::w4_mainloop<C::NB, TB, 3, C::HS, C::D, false>(lds, x, trow, w, wrow, nh, acc);
     else
-      sk::w4_mainloop<C::NB, TB, 4, C::HS, C::D>(lds, x, trow, w, wrow, nh, acc);
+      sk::w4_mainloop<C::NB, TB, 4, C::HS, C::D, false>(lds, x, trow, w, wrow, nh, acc);
   }
 }
 

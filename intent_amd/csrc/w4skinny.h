@@ -74,21 +74,32 @@ struct W4Src {
 };
 
 // Decodes one dword (8 weights) in the order 0 4 1 5 2 6 3 7.
+template <bool kScale>
 INTENT_DEVICE f16x8 decode8(uint32_t d, uint32_t magic, uint32_t mhi, f16x2 za, f16x2 zb, f16x2 sc) {
   const uint32_t d8 = d >> 8;
-  const f16x2 a = (bit_cast<f16x2>(bfi(0x000F000Fu, d, magic)) - za) * sc;
-  const f16x2 b = (bit_cast<f16x2>(bfi(0x00F000F0u, d, mhi)) - zb) * sc;
-  const f16x2 c = (bit_cast<f16x2>(bfi(0x000F000Fu, d8, magic)) - za) * sc;
-  const f16x2 e = (bit_cast<f16x2>(bfi(0x00F000F0u, d8, mhi)) - zb) * sc;
+  f16x2 a = bit_cast<f16x2>(bfi(0x000F000Fu, d, magic)) - za;
+  f16x2 b = bit_cast<f16x2>(bfi(0x00F000F0u, d, mhi)) - zb;
+  f16x2 c = bit_cast<f16x2>(bfi(0x000F000Fu, d8, magic)) - za;
+  f16x2 e = bit_cast<f16x2>(bfi(0x00F000F0u, d8, mhi)) - zb;
+  if constexpr (kScale) {
+    a *= sc;
+    b *= sc;
+    c *= sc;
+    e *= sc;
+  }
   return f16x8{a[0], a[1], b[0], b[1], c[0], c[1], e[0], e[1]};
 }
 
-// acc[b][t]: lane l holds activation row 16 t + l % 16 and weight rows
-// (of the wave's block b) 4 (l / 16) + 0..3, summed over nh * 128 k.
+// acc[b][t], summed over nh * 128 k. kPost false: lane l holds activation row
+// 16 t + l % 16 and weight rows (of the wave's block b) 4 (l / 16) + 0..3.
+// kPost true (groups of whole 128 k): the weights enter the MFMAs as the exact
+// q - z and each 128-k sum is scaled once in f32, so no weight is rounded to f16;
+// the operands are swapped, so that a lane's sums share one weight row and
+// scale: lane l holds weight row l % 16 and activation rows 16 t + 4 (l / 16) + 0..3.
 // x: activation rows at the range's first k; trow(p): byte offset of row p
 // (< 16 TU, every one readable); wrow(r): weight row of workgroup row r.
 // TU: 16-row blocks computed (<= TB).
-template <int NB, int TB, int TU, int HS, int D, class WRow, class TRow>
+template <int NB, int TB, int TU, int HS, int D, bool kPost, class WRow, class TRow>
 INTENT_DEVICE void w4_mainloop(char* lds, const void* x, const TRow& trow, const W4Src& w, const WRow& wrow, int nh,
                                f32x4 (&acc)[NB][TB]) {
   static_assert(TU >= 1 && TU <= TB, "computed blocks");
@@ -223,6 +234,13 @@ INTENT_DEVICE void w4_mainloop(char* lds, const void* x, const TRow& trow, const
       za[b] = splat2(bit_cast<f16>((uint16_t)(p >> 16)));
       zb[b] = za[b] - splat2((f16)960.f);
     }
+    f32x4 sum[NB][TU];  // kPost: the half's own sums
+    if constexpr (kPost) {
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int t = 0; t < TU; ++t) sum[b][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       f16x8 xf[TU];
@@ -231,9 +249,24 @@ INTENT_DEVICE void w4_mainloop(char* lds, const void* x, const TRow& trow, const
         xf[t] = *reinterpret_cast<const f16x8*>(xb + (t * 16 + n) * XR + hh * 256 + q * 64 + j * 16);
 #pragma unroll
       for (int b = 0; b < NB; ++b) {
-        const f16x8 wf = decode8(r[b][hh][j], magic, mhi, za[b], zb[b], sc[b]);
+        const f16x8 wf = decode8<!kPost>(r[b][hh][j], magic, mhi, za[b], zb[b], sc[b]);
 #pragma unroll
-        for (int t = 0; t < TU; ++t) acc[b][t] = mfma16(wf, xf[t], acc[b][t]);
+        for (int t = 0; t < TU; ++t) {
+          if constexpr (kPost)
+            sum[b][t] = mfma16(xf[t], wf, sum[b][t]);
+          else
+            acc[b][t] = mfma16(wf, xf[t], acc[b][t]);
+        }
+      }
+    }
+    if constexpr (kPost) {
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        const float sf = (float)sc[b][0];
+#pragma unroll
+        for (int t = 0; t < TU; ++t)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[b][t][e] = __builtin_fmaf(sum[b][t][e], sf, acc[b][t][e]);
       }
     }
   };

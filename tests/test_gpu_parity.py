@@ -414,6 +414,27 @@ def test_moe_ffn_few_routes(gpu, threads, T, H, E, k, F, group, skew):
     assert_close_rms(got - y0, ref - y0, what=f"moe few routes T {T} H {H} E {E} F {F} group {group}")
 
 
+# The weight-streaming W4A16 kernel: every instantiated row count (16 .. 96, 128) with rows short of it, groups
+# scaled after the MFMAs (multiples of 128) and before (32, 64), runs of unequal length and of an odd number of
+# 128-k steps, columns off the 64-row workgroups, strided activations and outputs, and (M <= 16) the calls it
+# takes from the GEMV.
+@pytest.mark.parametrize("M,K,N,group,pad", [
+    (17, 1408, 1000, 128, 0), (33, 4096, 130, 128, 0), (48, 2944, 257, 64, 8), (64, 4096, 1001, 32, 0),
+    (77, 3072, 640, 256, 0), (96, 5504, 200, 128, 0), (100, 4096, 129, 128, 16), (128, 4096, 4000, 64, 0),
+    (12, 4096, 11008, 128, 0), (4, 8192, 8200, 128, 0), (2, 14336, 4096, 256, 0), (16, 10240, 4100, 64, 8)])
+def test_w4a16_skinny(gpu, threads, M, K, N, group, pad):
+    d = inputs.config1_w4a16_decode(M + N, M=M, K=K, N=N, group=group)
+    x = torch.zeros(M, K + pad, dtype=torch.float16, device="cuda")
+    x[:, :K] = dev(d["x"])
+    y = torch.zeros(M, N + pad // 8, dtype=torch.float16, device="cuda")[:, :N]
+    a = art(intent.weight_only_int4_asym_matmul)
+    a(x[:, :K], dev(d["packed"]), dev(d["scales"]), dev(d["zeros"]), y)
+    assert a.observation.kernel == "w4a16_skinny", a.observation.kernel
+    cols = np.r_[0:min(N, 700), max(0, N - 70):N]  # the oracle's rows of the weights
+    ref = oracle.w4a16(d["x"], d["packed"][cols], d["scales"][cols], d["zeros"][cols], threads)
+    assert_close_rms(host(y)[:, cols], ref, what=f"w4a16 skinny {M}x{K}x{N} g{group}")
+
+
 # K split over workgroups (partial sums through scratch) and the 64-, 128- and 256-row tiles: rows and
 # columns off the tiles, runs of unequal length (11 or 43 units over 8 runs), every group form the cut takes
 # (windowed, whole groups, 32), and an output whose row stride rules out the vector stores.
