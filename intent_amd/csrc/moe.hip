@@ -26,7 +26,8 @@ constexpr int kMaxAlignExperts = 2048;  // LDS: (3E + 1 + 16E) ints
 // lower index (softmax is monotonic, so raw logits are compared). A run of
 // consecutive experts is summarised by its first untaken candidate and its
 // best non-NaN one, and two adjacent runs merge exactly, so a butterfly over
-// the lanes gives the scan's answer. The max for the softmax is the same
+// the lanes that hold experts gives them the scan's answer (lane 0 writes; six
+// stages whatever E cost 1 us of a layer of 8 experts). The max for the softmax is the same
 // selection over all experts; the softmax denominator is a lane-tree sum.
 struct RouteSel {
   float fv;  // first untaken candidate of the run (fi < 0: none)
@@ -59,6 +60,7 @@ INTENT_DEVICE int route_select(const float (&v)[4], int e0, int E, uint32_t take
   const int lane = threadIdx.x & 63;
 #pragma unroll
   for (int d = 1; d < 64; d <<= 1) {
+    if (4 * d >= E) break;
     RouteSel o;
     o.fv = __shfl_xor(s.fv, d);
     o.fi = __shfl_xor(s.fi, d);
@@ -89,7 +91,10 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const float* __restrict_
   for (int i = 0; i < 4; ++i)
     if (e0 + i < E) part += expf(v[i] - mx);
 #pragma unroll
-  for (int d = 1; d < 64; d <<= 1) part += __shfl_xor(part, d);
+  for (int d = 1; d < 64; d <<= 1) {
+    if (4 * d >= E) break;
+    part += __shfl_xor(part, d);
+  }
   const float sum = part;
   uint32_t taken = 0;
   float p[kMaxTopK];
@@ -161,7 +166,12 @@ __global__ __launch_bounds__(256) void moe_route_seq_kernel(const float* __restr
 // routes are processed in chunks of 1024 in route order; inside a wave the rank
 // of a route among same-expert lanes comes from ballots, across waves from a
 // prefix over per-wave counts, across chunks from a running base per expert.
-// The result equals a stable argsort of the expert ids.
+// The result equals a stable argsort of the expert ids. Bound by its chain of
+// dependent steps: counts are padded and summed by a wave scan (a thread's loop
+// over E = 32 took 2 us), and the first chunk's ids are loaded once. With the
+// router's shorter butterfly, whole layer: E = 32, top-4, H = 2048, F = 1408, T =
+// 16 65 -> 62 us, T = 256 102 -> 99; E = 8, H = 1024, F = 1408, T = 16 29 -> 27.
+// Router and alignment in one launch measured the same at T <= 16, slower above.
 __global__ __launch_bounds__(kAlignThreads) void moe_align_kernel(const int32_t* __restrict__ ids, int R, int E, int B,
                                                                   int32_t* __restrict__ sorted, int capacity,
                                                                   int32_t* __restrict__ blocks, int nblocks,
@@ -183,20 +193,28 @@ __global__ __launch_bounds__(kAlignThreads) void moe_align_kernel(const int32_t*
     cnt[e] = 0;
     base[e] = 0;
   }
+  const int first = tid < R ? ids[tid] : -1;
   __syncthreads();
   for (int r = tid; r < R; r += kAlignThreads) {
-    const int e = ids[r];
+    const int e = r == tid ? first : ids[r];
     if (e >= 0 && e < E) atomicAdd(&cnt[e], 1);
   }
   __syncthreads();
-  if (tid == 0) {
+  if (wave == 0) {
     int acc = 0;
-    off[0] = 0;
-    for (int e = 0; e < E; ++e) {
-      acc += (cnt[e] + B - 1) / B * B;
-      off[e + 1] = acc;
+    if (lane == 0) off[0] = 0;
+    for (int e0 = 0; e0 < E; e0 += 64) {
+      const int e = e0 + lane;
+      int v = e < E ? (cnt[e] + B - 1) / B * B : 0;
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {
+        const int o = __shfl_up(v, d);
+        if (lane >= d) v += o;
+      }
+      if (e < E) off[e + 1] = acc + v;
+      acc += __shfl(v, 63);
     }
-    total[0] = acc;
+    if (lane == 0) total[0] = acc;
   }
   __syncthreads();
   for (int e = tid; e <= E; e += kAlignThreads) offsets[e] = off[e];
@@ -220,7 +238,7 @@ __global__ __launch_bounds__(kAlignThreads) void moe_align_kernel(const int32_t*
   for (int c = 0; c < R; c += kAlignThreads) {
     for (int i = tid; i < kAlignWaves * E; i += kAlignThreads) wcnt(i / E, i % E) = 0;
     const int r = c + tid;
-    int e = r < R ? ids[r] : -1;
+    int e = c == 0 ? first : r < R ? ids[r] : -1;
     const bool valid = e >= 0 && e < E;
     if (!valid) e = -1;
     __syncthreads();
@@ -235,9 +253,10 @@ __global__ __launch_bounds__(kAlignThreads) void moe_align_kernel(const int32_t*
       remaining &= ~same;
     }
     __syncthreads();
+    const int waves = R - c < kAlignThreads ? (R - c + 63) / 64 : kAlignWaves;  // waves with a route
     for (int x = tid; x < E; x += kAlignThreads) {
       int run = base[x];
-      for (int w = 0; w < kAlignWaves; ++w) {
+      for (int w = 0; w < waves; ++w) {
         const int n = wcnt(w, x);
         wcnt(w, x) = run;
         run += n;

@@ -328,6 +328,23 @@ def test_moe_align(gpu, T, k, E, B):
         assert np.array_equal(host(got), ref), name
 
 
+# Expert counts at the edges of the router's lanes (four experts each, butterflies over as many lanes as hold
+# one) and of the alignment's 64-expert scan, routes at the edges of its waves and 1024-route chunks.
+@pytest.mark.parametrize("T,E,k,B", [(1, 1, 1, 16), (63, 4, 1, 16), (32, 5, 2, 32), (65, 9, 1, 64), (342, 17, 3, 128),
+                                     (1024, 63, 1, 16), (1025, 64, 1, 160), (205, 65, 5, 16), (1000, 129, 2, 32),
+                                     (260, 256, 8, 64)])
+def test_moe_route_align_edges(gpu, T, E, k, B):
+    rng = np.random.default_rng(T + E)
+    logits = np.round(rng.standard_normal((T, E)) * 4).astype(np.float32) / 4  # many ties
+    ids, wts = art(intent.moe_route_topk, TOP_K=k, RENORMALIZE=True).run(dev(logits))
+    rid, rw = oracle.moe_route(logits, k, True)
+    assert np.array_equal(host(ids), rid)
+    np.testing.assert_allclose(host(wts), rw, rtol=2e-6, atol=1e-7)
+    outs = art(intent.moe_align_block_size, EXPERTS=E, BLOCK_SIZE=B).run(ids)
+    for got, ref, name in zip(outs, oracle.moe_align(rid, E, B), ("sorted", "blocks", "offsets", "total")):
+        assert np.array_equal(host(got), ref), name
+
+
 @pytest.mark.parametrize("B", [128, 160])
 def test_moe_route_align_config4(gpu, B):
     """Routing and alignment of BASELINE config 4's own router logits (seed 0,
