@@ -929,8 +929,6 @@ int64_t dense_split_bytes(const DensePlan& p, int64_t M, int64_t N) {
 DensePlan dense_plan(int64_t M, int64_t N, int64_t K, int64_t unit, bool may_split, double stage_scale,
                      double* us = nullptr) {
   DensePlan best{M > 128 ? 256 : 128, 1};
-  if (us) *us = 1e30;
-  if (dense_tiles(M, N, 256) >= 512) return best;  // two rounds of the large tile: nothing idles
   const auto cost = [&](const DensePlan& p) {
     const double k = p.tile == 256 ? 1.0 : stage_scale;
     const intent::GridCost c = p.tile == 256   ? intent::GridCost{4, 0.95, 0.42}
@@ -939,6 +937,8 @@ DensePlan dense_plan(int64_t M, int64_t N, int64_t K, int64_t unit, bool may_spl
     return c.us(dense_tiles(M, N, p.tile) * p.splits, (double)K / 64 / p.splits) +
            (p.splits > 1 ? 3 + 0.27e-6 * (double)dense_split_bytes(p, M, N) : 0);
   };
+  if (us) *us = cost(best);
+  if (dense_tiles(M, N, 256) >= 512) return best;  // two rounds of the large tile: nothing idles
   const double keep = 0.95 * cost(best);  // the plain plan unless another is clearly faster
   double least = keep;
   for (int tile = 256; tile >= 64; tile /= 2)
@@ -1051,6 +1051,8 @@ int w4a16_skinny_launch(const void* x, int64_t M, int64_t K, int64_t x_ld, const
 // per round of 256 workgroups 1.6 us + 1 us per 1000 k (measured: N = 11008, K =
 // 4096 17 us, N = 14336, K = 2048 13.5, N = K = 8192 20, N = 4096, K = 14336 19..23);
 // where the dot-product GEMV (no weight rounded to f16) takes the call, it stays.
+// Very wide outputs are weighed the same way (N = 128256, K = 4096: M = 48 117 us
+// here against 145 in 128-row tiles, M = 77 188 against 143, 128 310 against 151).
 bool w4a16_wants_skinny(int64_t M, int64_t N, int64_t K, int64_t gs) {
   const double us = w4a16_skinny_us(M, N, K, gs);
   if (us == 0) return false;

@@ -96,6 +96,11 @@ struct Plan {
   int lds;
 };
 
+constexpr int64_t kMaxPartialBytes = 64 << 20;  // as the tiled kernels' split
+int64_t partial_bytes(const Plan& p, int64_t N) {
+  return p.splits * ((N + kRows - 1) / kRows) * kRows * 16 * p.tb * 4;
+}
+
 template <class F>
 auto with_rows(int tb, F&& f) {
   switch (tb) {
@@ -111,7 +116,8 @@ auto with_rows(int tb, F&& f) {
 
 // Runs of about 1024 k (the longest that still give two workgroups per CU at N =
 // 4096 were the fastest: N = 4096, K = 4096, M = 77: 4 runs 13.8 us, 2 16.9, 8 16.1),
-// shorter ones down to 512 k while there are fewer than 128 workgroups.
+// shorter ones down to 512 k while there are fewer than 128 workgroups; fewer where
+// the partial sums would pass 64 MB (wide N has workgroups enough without).
 Plan skinny_plan(int64_t M, int64_t N, int64_t K, int64_t gs) {
   Plan p{(int)((M + 15) / 16), 1, 0, 0};
   if (p.tb > 6) p.tb = 8;
@@ -122,6 +128,8 @@ Plan skinny_plan(int64_t M, int64_t N, int64_t K, int64_t gs) {
   while (K / (2 * p.splits) >= 1024 && p.splits < 16) p.splits *= 2;
   while (tiles * p.splits < 128 && K / (2 * p.splits) >= 512 && p.splits < 16) p.splits *= 2;
   while (p.splits > K / unit) p.splits /= 2;
+  while (p.splits > 1 && partial_bytes(p, N) > kMaxPartialBytes) p.splits /= 2;
+  if (partial_bytes(p, N) > kMaxPartialBytes) return p;
   const int64_t longest = (K / unit + p.splits - 1) / p.splits * unit;
   if (longest / gs > 256) return p;
   p.lds = with_rows(p.tb, [&](auto TB) {
@@ -146,8 +154,7 @@ double w4a16_skinny_us(int64_t M, int64_t N, int64_t K, int64_t gs) {
 }
 
 size_t w4a16_skinny_bytes(int64_t M, int64_t N, int64_t K, int64_t gs) {
-  const Plan p = skinny_plan(M, N, K, gs);
-  return (size_t)p.splits * ((N + kRows - 1) / kRows) * kRows * 16 * p.tb * 4;
+  return (size_t)partial_bytes(skinny_plan(M, N, K, gs), N);
 }
 
 // A w4a16_fast call whose plan exists, with 31-bit offsets checked by the caller.

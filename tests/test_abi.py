@@ -110,6 +110,20 @@ def test_moe_checks():
     assert _native.library().intent_moe_workspace_size(-1, 2, 8, 64, 64, 128) == 0
 
 
+def test_w4a16_wide_outputs_scratch():
+    # Very wide outputs (a vocabulary head): the streaming kernel is weighed against the tiles there too, and
+    # whatever takes the call keeps its partial sums within 64 MB.
+    size = _native.library().intent_w4a16_matmul_workspace_size
+    for N in (50304, 98304, 128256, 131072, 200000, 1 << 20):
+        for K in (1024, 4096, 8192, 16384):
+            for M in (2, 6, 16, 17, 33, 60, 77, 100, 128, 129, 300):
+                assert size(M, K, N, 128) <= 64 << 20, (M, K, N)
+    for M in (60, 77, 100, 128):  # 128-row tiles without K runs are the faster there
+        assert size(M, 4096, 128256, 128) == 0, M
+    for M in (6, 12, 16, 17, 33):  # the streaming kernel is
+        assert size(M, 8192, 128256, 128) > 0, M
+
+
 def test_kquant_checks():
     # Q8_K: x must be 16-byte aligned; rows of at least 256 values / 292 bytes
     assert status("intent_q8k_quantize", FAKE + 4, 3, 256, FAKE, 292, None) == errors.INTENT_ERR_ALIGNMENT

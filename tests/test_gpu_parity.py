@@ -433,12 +433,13 @@ def test_moe_ffn_few_routes(gpu, threads, T, H, E, k, F, group, skew):
 
 # The weight-streaming W4A16 kernel: every instantiated row count (16 .. 96, 128) with rows short of it, groups
 # scaled after the MFMAs (multiples of 128) and before (32, 64), runs of unequal length and of an odd number of
-# 128-k steps, columns off the 64-row workgroups, strided activations and outputs, and (M <= 16) the calls it
-# takes from the GEMV.
+# 128-k steps, columns off the 64-row workgroups, strided activations and outputs, (M <= 16) the calls it
+# takes from the GEMV, and an output so wide that the bound on the partial sums halves the runs.
 @pytest.mark.parametrize("M,K,N,group,pad", [
     (17, 1408, 1000, 128, 0), (33, 4096, 130, 128, 0), (48, 2944, 257, 64, 8), (64, 4096, 1001, 32, 0),
     (77, 3072, 640, 256, 0), (96, 5504, 200, 128, 0), (100, 4096, 129, 128, 16), (128, 4096, 4000, 64, 0),
-    (12, 4096, 11008, 128, 0), (4, 8192, 8200, 128, 0), (2, 14336, 4096, 256, 0), (16, 10240, 4100, 64, 8)])
+    (12, 4096, 11008, 128, 0), (4, 8192, 8200, 128, 0), (2, 14336, 4096, 256, 0), (16, 10240, 4100, 64, 8),
+    (33, 4096, 120001, 128, 0)])
 def test_w4a16_skinny(gpu, threads, M, K, N, group, pad):
     d = inputs.config1_w4a16_decode(M + N, M=M, K=K, N=N, group=group)
     x = torch.zeros(M, K + pad, dtype=torch.float16, device="cuda")
