@@ -1390,6 +1390,29 @@ def test_moe_expert_ffn_few_routes(gpu, threads, T, D, E, k, F, runs):
     assert_close_rms(host(y) - y0, ref - y0, what=f"moe_expert_ffn few routes {T}x{D}x{F}")
 
 
+# The launch has exactly as many row tiles as the worst split of the routes needs: one per expert with a route
+# and one more per whole tile of rows. Experts of one route beside one that overflows a 64- or 128-row tile by a
+# row, and more experts than routes with empty ones between them.
+@pytest.mark.parametrize("sizes", [[1] * 8 + [65], [65] + [1] * 8, [1, 129, 65, 1, 65], [1, 129, 129],
+                                   [257] + [1] * 3, [0] * 40 + [1] + [0] * 30 + [2] + [0] * 55 + [1], [0, 0, 1]])
+def test_moe_expert_ffn_worst_tiles(gpu, threads, sizes):
+    E, R, D, F = len(sizes), sum(sizes), 128, 192
+    rng = np.random.default_rng(E + R)
+    offsets = np.r_[0, np.cumsum(sizes)].astype(np.int32)
+    members, tokens = rng.permutation(R).astype(np.int32), rng.permutation(R).astype(np.int32)
+    weights = rng.random(R, dtype=np.float32)
+    x = inputs.normal_f16(rng, (R, D))
+    w1 = (rng.standard_normal((E, D, F), dtype=np.float32) / np.sqrt(D)).astype(np.float16)
+    w2 = (rng.standard_normal((E, F, D), dtype=np.float32) / np.sqrt(F)).astype(np.float16)
+    y = torch.zeros(R, D, device="cuda")
+    art(intent.moe_expert_ffn)(dev(x), dev(offsets), dev(members), dev(tokens), dev(weights), dev(w1), dev(w2), y)
+    ref = oracle.moe_expert_ffn(x, offsets, members, tokens, weights, w1, w2, y=np.zeros((R, D), np.float32),
+                                threads=threads)
+    got = host(y)
+    for t in range(R):  # every token has one route, so a missing tile shows in its rows
+        assert_close_rms(got[t], ref[t], what=f"token {t} of {sizes}")
+
+
 @pytest.mark.parametrize("T", [512, 4096])
 def test_moe_expert_ffn_reference_size(gpu, threads, T):
     # moe.py:6-10 (T = 4096, D = 4096, F = 14336, E = 8, top-2) and the config-4 token count,
