@@ -629,11 +629,14 @@ int intent_grouped_gemm_kn(const void* x, int64_t rows, int64_t K, int64_t x_ld,
  * with f32 accumulation; a token's contributions are added in member order
  * (deterministic). Out-of-range routing entries are clamped, never
  * dereferenced. D and F multiples of 64. workspace: at least
- * intent_moe_expert_ffn_workspace_size(T, R, D, F) bytes, 16-byte aligned (the
- * last 12 R D bytes of it, present for R <= 4096, only let the second projection
- * split K: a call with less runs without).
+ * intent_moe_expert_ffn_workspace_size_for(T, R, D, F, E) bytes, 16-byte aligned:
+ * what a call with E experts uses. intent_moe_expert_ffn_workspace_size, which does
+ * not know E, is enough for every E: its last 12 R D bytes, present for R <= 4096,
+ * hold the results of K runs of the second projection, which only calls of few
+ * routes per expert take. A call with less runs without them.
  */
 size_t intent_moe_expert_ffn_workspace_size(int64_t T, int64_t R, int64_t D, int64_t F);
+size_t intent_moe_expert_ffn_workspace_size_for(int64_t T, int64_t R, int64_t D, int64_t F, int64_t E);
 int intent_moe_expert_ffn(const void* x, int64_t T, int64_t D, int64_t x_ld, const int32_t* route_offsets,
                           int64_t E, const int32_t* member_routes, int64_t R, const int32_t* route_token,
                           const float* route_weights, int64_t NR, const void* w1, const void* w2, int64_t F,

@@ -235,7 +235,7 @@ __global__ __launch_bounds__(256) void token_combine_kernel(const float* __restr
 size_t round256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 constexpr int kFfnParts = 4;        // K runs of the second projection, at most
-constexpr int64_t kFewRows = 4096;  // routes up to which the workspace has room for them
+constexpr int64_t kFewRows = 4096;  // routes up to which they are taken: bounds their results
 
 // Tiles of both projections for R routes over E experts. Few routes per expert:
 // the time is the experts' weights, and a 256 x 256 tile at one workgroup per CU
@@ -265,10 +265,11 @@ FfnPlan ffn_plan(int64_t E, int64_t R, int64_t D, int64_t F) {
 }
 
 struct FfnLayout {
-  size_t hidden, contrib, count, start, list, base, parts, bytes;
+  size_t hidden, contrib, count, start, list, parts, bytes;
 };
 
-FfnLayout ffn_layout(int64_t T, int64_t R, int64_t D, int64_t F) {
+// parts: K runs of the second projection (the results of the runs after the first come last).
+FfnLayout ffn_layout(int64_t T, int64_t R, int64_t D, int64_t F, int parts) {
   FfnLayout L{};
   size_t o = 0;
   L.hidden = o;  o = round256(o + sizeof(uint16_t) * (size_t)R * F);
@@ -276,9 +277,7 @@ FfnLayout ffn_layout(int64_t T, int64_t R, int64_t D, int64_t F) {
   L.count = o;   o = round256(o + sizeof(int32_t) * (size_t)T);
   L.start = o;   o = round256(o + sizeof(int32_t) * (size_t)(T + 1));
   L.list = o;    o = round256(o + sizeof(int32_t) * (size_t)R);
-  L.base = o;  // enough for a call without K runs
-  L.parts = o;
-  if (R <= kFewRows) o = round256(o + sizeof(float) * (size_t)R * D * (kFfnParts - 1));
+  L.parts = o;   o = round256(o + sizeof(float) * (size_t)R * D * (parts - 1));
   L.bytes = o;
   return L;
 }
@@ -287,7 +286,12 @@ FfnLayout ffn_layout(int64_t T, int64_t R, int64_t D, int64_t F) {
 
 extern "C" size_t intent_moe_expert_ffn_workspace_size(int64_t T, int64_t R, int64_t D, int64_t F) {
   if (T < 0 || R < 0 || D < 0 || F < 0) return 0;
-  return ffn_layout(T, R, D, F).bytes;
+  return ffn_layout(T, R, D, F, R <= kFewRows ? kFfnParts : 1).bytes;
+}
+
+extern "C" size_t intent_moe_expert_ffn_workspace_size_for(int64_t T, int64_t R, int64_t D, int64_t F, int64_t E) {
+  if (T < 0 || R < 0 || D < 0 || F < 0 || E < 1) return 0;
+  return ffn_layout(T, R, D, F, ffn_plan(E, R, D, F).parts).bytes;
 }
 
 extern "C" int intent_moe_expert_ffn(const void* x, int64_t T, int64_t D, int64_t x_ld, const int32_t* route_offsets,
@@ -311,9 +315,11 @@ extern "C" int intent_moe_expert_ffn(const void* x, int64_t T, int64_t D, int64_
                  "x must be 16-byte aligned with 16-byte row strides");
   INTENT_REQUIRE(intent::fits_offset(T, x_ld * 2) && intent::fits_offset(R, F * 2) && intent::fits_offset(R, D * 4),
                  INTENT_ERR_UNSUPPORTED, "moe_expert_ffn: operands exceed 31-bit buffer offsets");
-  const FfnLayout L = ffn_layout(T, R, D, F);
-  INTENT_REQUIRE(workspace && workspace_bytes >= L.base, INTENT_ERR_WORKSPACE, "workspace needs %zu bytes, got %zu",
-                 L.bytes, workspace_bytes);
+  FfnPlan p = ffn_plan(E, R, D, F);
+  const FfnLayout L = ffn_layout(T, R, D, F, p.parts);
+  const size_t least_bytes = ffn_layout(T, R, D, F, 1).bytes;
+  INTENT_REQUIRE(workspace && workspace_bytes >= least_bytes, INTENT_ERR_WORKSPACE,
+                 "workspace needs %zu bytes, got %zu", least_bytes, workspace_bytes);
   INTENT_REQUIRE(intent::aligned16(workspace), INTENT_ERR_ALIGNMENT, "workspace must be 16-byte aligned");
   char* ws = (char*)workspace;
   uint16_t* hidden = (uint16_t*)(ws + L.hidden);
@@ -322,8 +328,7 @@ extern "C" int intent_moe_expert_ffn(const void* x, int64_t T, int64_t D, int64_
   int32_t* start = (int32_t*)(ws + L.start);
   int32_t* list = (int32_t*)(ws + L.list);
   hipStream_t s = (hipStream_t)stream;
-  FfnPlan p = ffn_plan(E, R, D, F);
-  if (p.parts > 1 && workspace_bytes < L.bytes) p.parts = 1;
+  if (workspace_bytes < L.bytes) p.parts = 1;
   // Row tiles: every expert with a route has at least one, and one more per whole
   // p.rows routes. With one per expert instead, E = 128 and 8 routes launched 129 rows
   // of workgroups that only walk the offsets (T = 1, top-8, D = 2048, F = 768: 314 us,

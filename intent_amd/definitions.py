@@ -416,7 +416,7 @@ def _f16ffn_check(env: dict) -> None:
 
 def _f16ffn_workspace(env: dict) -> int:
     lib = _native.library()
-    return int(lib.intent_moe_expert_ffn_workspace_size(env["T"], env["R"], env["D"], env["F"]))
+    return int(lib.intent_moe_expert_ffn_workspace_size_for(env["T"], env["R"], env["D"], env["F"], env["E"]))
 
 
 def _f16ffn_launch(v: dict, env: dict, stream: int, workspace) -> str:

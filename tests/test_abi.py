@@ -110,6 +110,21 @@ def test_moe_checks():
     assert _native.library().intent_moe_workspace_size(-1, 2, 8, 64, 64, 128) == 0
 
 
+def test_moe_expert_ffn_workspace_holds_what_the_plan_uses():
+    lib = _native.library()
+    every, exact = lib.intent_moe_expert_ffn_workspace_size, lib.intent_moe_expert_ffn_workspace_size_for
+    D, F, round256 = 4096, 14336, lambda v: (v + 255) // 256 * 256
+    for T, R, E in ((2048, 4096, 8), (512, 1024, 8), (4096, 8192, 8), (5000, 5000, 64)):  # many routes, or more than 4096
+        base = sum(round256(b) for b in (2 * R * F, 4 * R * D, 4 * T, 4 * (T + 1), 4 * R))
+        assert exact(T, R, D, F, E) == base, (T, R, E)  # no room for K runs that the plan does not take
+    for T, R, E in ((16, 32, 8), (200, 400, 8)):  # few routes per expert: up to three results beside the first
+        extra = exact(T, R, D, F, E) - sum(round256(b) for b in (2 * R * F, 4 * R * D, 4 * T, 4 * (T + 1), 4 * R))
+        assert extra in (4 * R * D, 12 * R * D), (T, R, E)
+    for T, R, E in ((1, 2, 8), (16, 32, 8), (512, 1024, 8), (2048, 4096, 8), (300, 4096, 64), (4096, 8192, 8)):
+        assert exact(T, R, D, F, E) <= every(T, R, D, F), (T, R, E)
+    assert exact(4, 8, 64, 64, 0) == 0 and exact(-1, 8, 64, 64, 2) == 0
+
+
 def test_w4a16_wide_outputs_scratch():
     # Very wide outputs (a vocabulary head): the streaming kernel is weighed against the tiles there too, and
     # whatever takes the call keeps its partial sums within 64 MB.
