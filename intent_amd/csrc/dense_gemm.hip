@@ -63,7 +63,6 @@ struct W4SymArgs {
   int64_t ldq;
   const f16* s;
   int64_t lds;
-  INTENT_DEVICE W4SymArgs at(int k0) const { return {q + (int64_t)(k0 / 8) * ldq, ldq, s + (int64_t)(k0 / 64) * lds, lds}; }
 };
 template <class T>
 struct WeightOp<T, W4SymArgs> {
@@ -915,6 +914,9 @@ struct DensePlan {
   int splits;  // K runs (1: no workspace)
 };
 constexpr int64_t kMaxSplitBytes = 64 << 20;
+constexpr intent::PlanNames kW4Names = INTENT_PLAN_NAMES("w4a16_gemm", "256x192");
+constexpr intent::PlanNames kW8Names = INTENT_PLAN_NAMES("w8a16_matmul", "256x192");
+constexpr intent::PlanNames kW4SymNames = INTENT_PLAN_NAMES("w4a16_sym_gemm", "256x192");
 
 int64_t dense_tiles(int64_t M, int64_t N, int tile) {
   const int64_t bn = tile == 256 ? 192 : 128;
@@ -992,7 +994,8 @@ int launch_split(const f16* x, int64_t ldx, int M, int N, int K, const WArgs& w,
 
 template <class WArgs, bool kColScale>
 int launch_dense(const f16* x, int64_t ldx, int M, int N, int K, const WArgs& w, f16* y, int64_t ldy,
-                 const f16* colscale, hipStream_t st, const char* name, const DensePlan& p) {
+                 const f16* colscale, hipStream_t st, const intent::PlanNames& names, const DensePlan& p) {
+  const char* name = names(p.tile, 1);
   if (p.tile == 256)
     return launch_tile<mp::Tile<256, 192, 2, 2>, WArgs, kColScale>(x, ldx, M, N, K, w, y, ldy, colscale, st, name);
   if (p.tile == 128)
@@ -1002,8 +1005,9 @@ int launch_dense(const f16* x, int64_t ldx, int M, int N, int K, const WArgs& w,
 
 template <class WArgs, bool kColScale>
 int launch_dense_split(const f16* x, int64_t ldx, int M, int N, int K, const WArgs& w, f16* y, int64_t ldy,
-                       const f16* colscale, hipStream_t st, const char* name, const DensePlan& p, int64_t unit,
-                       float* part) {
+                       const f16* colscale, hipStream_t st, const intent::PlanNames& names, const DensePlan& p,
+                       int64_t unit, float* part) {
+  const char* name = names(p.tile, p.splits);
   if (p.tile == 256)
     return launch_split<mp::Tile<256, 192, 2, 2>, WArgs, kColScale>(x, ldx, M, N, K, w, y, ldy, colscale, p.splits,
                                                                     (int)unit, part, st, name);
@@ -1088,15 +1092,15 @@ int w4a16_gemm_launch(const void* x, int64_t M, int64_t K, int64_t x_ld, const u
   if (split_ready(split, M, N, ws, ws_bytes)) {
     if (win && cut.win)
       return launch_dense_split<W4WinArgs, false>(xx, x_ld, (int)M, (int)N, (int)K, W4WinArgs{w}, yy, y_ld, nullptr, st,
-                                                  "w4a16_gemm", split, cut.unit, (float*)ws);
-    return launch_dense_split<W4Args, false>(xx, x_ld, (int)M, (int)N, (int)K, w, yy, y_ld, nullptr, st, "w4a16_gemm",
+                                                  kW4Names, split, cut.unit, (float*)ws);
+    return launch_dense_split<W4Args, false>(xx, x_ld, (int)M, (int)N, (int)K, w, yy, y_ld, nullptr, st, kW4Names,
                                              split, cut.unit, (float*)ws);
   }
   const DensePlan p = w4_plan(M, N, K, gs, false);
   if (win)
     return launch_dense<W4WinArgs, false>(xx, x_ld, (int)M, (int)N, (int)K, W4WinArgs{w}, yy, y_ld, nullptr, st,
-                                          "w4a16_gemm", p);
-  return launch_dense<W4Args, false>(xx, x_ld, (int)M, (int)N, (int)K, w, yy, y_ld, nullptr, st, "w4a16_gemm", p);
+                                          kW4Names, p);
+  return launch_dense<W4Args, false>(xx, x_ld, (int)M, (int)N, (int)K, w, yy, y_ld, nullptr, st, kW4Names, p);
 }
 
 }  // namespace intent
@@ -1261,9 +1265,9 @@ int w8a16_launch(const void* x, int64_t M, int64_t K, int64_t x_ld, const int8_t
   const DensePlan split = w8_plan(M, N, K, true);
   if (split_ready(split, M, N, workspace, workspace_bytes))
     return launch_dense_split<W8Args, true>(xx, x_ld, (int)M, (int)N, (int)K, ws, yy, y_ld, (const f16*)scales, st,
-                                            "w8a16_matmul", split, 64, (float*)workspace);
+                                            kW8Names, split, 64, (float*)workspace);
   return launch_dense<W8Args, true>(xx, x_ld, (int)M, (int)N, (int)K, ws, yy, y_ld, (const f16*)scales, st,
-                                    "w8a16_matmul", w8_plan(M, N, K, false));
+                                    kW8Names, w8_plan(M, N, K, false));
 }
 
 }  // namespace
@@ -1572,5 +1576,5 @@ extern "C" int intent_w4a16_sym_gemm(const void* x, int64_t M, int64_t K, int64_
                  INTENT_ERR_UNSUPPORTED, "w4a16_sym_gemm: operand too large for 31-bit buffer offsets");
   W4SymArgs w{packed, packed_ld, (const f16*)scales, scales_ld};
   return launch_dense<W4SymArgs, false>((const f16*)x, x_ld, (int)M, (int)N, (int)K, w, (f16*)y, y_ld, nullptr,
-                                        (hipStream_t)stream, "w4a16_sym_gemm", DensePlan{M > 128 ? 256 : 128, 1});
+                                        (hipStream_t)stream, kW4SymNames, DensePlan{M > 128 ? 256 : 128, 1});
 }

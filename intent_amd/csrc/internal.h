@@ -51,7 +51,21 @@ struct GridCost {
   }
 };
 
+// Names of the kernels of a plan (tile and runs of K), recorded by launch_status.
+struct PlanNames {
+  const char* name[3][5];  // tiles of 256, 128 and 64 rows; 1, 2, 4, 8 and 16 runs
+  const char* operator()(int rows, int runs) const {
+    return name[rows == 256 ? 0 : rows == 128 ? 1 : 2][__builtin_ctz((unsigned)runs)];
+  }
+};
+
 }  // namespace intent
+
+#define INTENT_RUN_NAMES(tile) \
+  { tile ">", tile ", 2 runs>", tile ", 4 runs>", tile ", 8 runs>", tile ", 16 runs>" }
+// big: the 256-row tile; the others are 128x128 and 64x128.
+#define INTENT_PLAN_NAMES(base, big) \
+  {{INTENT_RUN_NAMES(base "<" big), INTENT_RUN_NAMES(base "<128x128"), INTENT_RUN_NAMES(base "<64x128")}}
 
 #define INTENT_REQUIRE(cond, code, ...)            \
   do {                                             \

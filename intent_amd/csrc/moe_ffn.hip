@@ -383,5 +383,5 @@ extern "C" int intent_moe_expert_ffn(const void* x, int64_t T, int64_t D, int64_
   const int64_t items = T * ((D + 3) / 4);
   hipLaunchKernelGGL(token_combine_kernel, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, s, contrib, D, start,
                      list, (int)T, (int)D, y, y_ld, p.parts, (const float*)(ws + L.parts), R * D);
-  return intent::launch_status("token_combine");
+  return intent::launch_status_fmt("moe_expert_ffn<%d rows, %d and %d columns, %d runs>", p.rows, p.up, p.down, p.parts);
 }

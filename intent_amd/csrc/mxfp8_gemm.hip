@@ -1408,6 +1408,8 @@ struct DgPlan {
   int tile;    // rows of the tile (128 or 64; 128 columns)
   int splits;  // K runs (1: no workspace)
 };
+constexpr intent::PlanNames kDgNames = INTENT_PLAN_NAMES("deepgemm_fp8", "");
+
 int64_t dg_tiles(int64_t M, int64_t N, int tile) { return ((M + tile - 1) / tile) * ((N + 127) / 128); }
 int64_t dg_split_bytes(const DgPlan& p, int64_t M, int64_t N) {
   return p.splits > 1 ? p.splits * dg_tiles(M, N, p.tile) * p.tile * 128 * 4 : 0;
@@ -1446,20 +1448,21 @@ int dg_launch(const uint8_t* a, int64_t M, int64_t K, int64_t a_ld, const float*
   const int64_t grid = (int64_t)mblocks * ((N + T::BN - 1) / T::BN);
   const int64_t cgrid = grid * T::NW * T::TI * T::TJ;
   INTENT_REQUIRE(cgrid < (1ll << 31), INTENT_ERR_UNSUPPORTED, "deepgemm_fp8: grid too large");
+  const char* name = kDgNames(T::BM, splits);
   hipStream_t st = (hipStream_t)stream;
   if (splits == 1) {
     hipLaunchKernelGGL((deepgemm_fp8_kernel<T, false>), dim3((unsigned)grid), dim3(256), 0, st, a, a_ld, (int)M,
                        a_scales, a_scales_ld, b, b_ld, (int)N, b_scales, b_scales_ld, (int)K, out, out_ld, mblocks);
-    return intent::launch_status("deepgemm_fp8");
+    return intent::launch_status(name);
   }
   hipLaunchKernelGGL((deepgemm_fp8_kernel<T, true>), dim3((unsigned)grid, splits), dim3(256), 0, st, a, a_ld, (int)M,
                      a_scales, a_scales_ld, b, b_ld, (int)N, b_scales, b_scales_ld, (int)K, ws, 0, mblocks);
-  const int s = intent::launch_status("deepgemm_fp8");
+  const int s = intent::launch_status(name);
   if (s != INTENT_OK) return s;
   const int vec = out_ld % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & 7) == 0;
   hipLaunchKernelGGL((deepgemm_combine_kernel<T>), dim3((unsigned)cgrid), dim3(64), 0, st, (const float*)ws, splits,
                      (int)grid, (int)M, (int)N, (uint16_t*)out, out_ld, vec, mblocks);
-  return intent::launch_status("deepgemm_fp8");
+  return intent::launch_status(name);
 }
 
 int dg_entry(const uint8_t* a, int64_t M, int64_t K, int64_t a_ld, const float* a_scales, int64_t a_scales_ld,

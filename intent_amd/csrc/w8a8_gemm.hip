@@ -456,6 +456,9 @@ struct I8Plan {
   int tile;    // rows of the tile: 256 (256 x 256), 128 (128 x 128), 64 (64 x 128)
   int splits;  // K runs (1: no workspace)
 };
+constexpr intent::PlanNames kW8A8Names = INTENT_PLAN_NAMES("w8a8_gemm", "256x256");
+constexpr intent::PlanNames kI8Names = INTENT_PLAN_NAMES("i8_gemm_i32", "256x256");
+
 int64_t i8_tiles(int64_t M, int64_t N, int tile) {
   const int64_t bn = tile == 256 ? 256 : 128;
   return ((M + tile - 1) / tile) * ((N + bn - 1) / bn);
@@ -516,9 +519,9 @@ int launch_split(const int8_t* a, int64_t M, int64_t K, int64_t a_ld, const floa
 
 template <Epi E>
 int launch_i8(const int8_t* a, int64_t M, int64_t K, int64_t a_ld, const float* sa, const int8_t* w, int64_t N,
-              int64_t w_ld, const float* sw, const int32_t* bias, void* out, int64_t out_ld, void* stream,
-              const char* name) {
+              int64_t w_ld, const float* sw, const int32_t* bias, void* out, int64_t out_ld, void* stream) {
   const I8Plan p = i8_plan(M, N, K, false);
+  const char* name = (E == Epi::kBf16Scaled ? kW8A8Names : kI8Names)(p.tile, 1);
   if (p.tile == 256)
     return launch_tile<T256, E>(a, M, K, a_ld, sa, w, N, w_ld, sw, bias, out, out_ld, stream, name);
   if (p.tile == 128)
@@ -539,10 +542,10 @@ int w8a8_launch(const int8_t* a, int64_t M, int64_t K, int64_t a_ld, const float
   const I8Plan p = i8_plan(M, N, K, true);
   if (p.splits > 1 && ws && intent::aligned16(ws) && ws_bytes >= (size_t)i8_split_bytes(p, M, N)) {
     const auto launch = p.tile == 256 ? launch_split<T256> : p.tile == 128 ? launch_split<T128> : launch_split<T64>;
-    return launch(a, M, K, a_ld, a_scales, w, N, w_ld, w_scales, out, out_ld, p.splits, ws, stream, "w8a8_gemm");
+    return launch(a, M, K, a_ld, a_scales, w, N, w_ld, w_scales, out, out_ld, p.splits, ws, stream,
+                  kW8A8Names(p.tile, p.splits));
   }
-  return launch_i8<Epi::kBf16Scaled>(a, M, K, a_ld, a_scales, w, N, w_ld, w_scales, nullptr, out, out_ld, stream,
-                                     "w8a8_gemm");
+  return launch_i8<Epi::kBf16Scaled>(a, M, K, a_ld, a_scales, w, N, w_ld, w_scales, nullptr, out, out_ld, stream);
 }
 
 }  // namespace
@@ -571,7 +574,7 @@ extern "C" int intent_i8_gemm_i32(const int8_t* a, int64_t M, int64_t K, int64_t
   if (st != INTENT_OK || M == 0 || N == 0) return st;
   if (!i8_fast(a, K, a_ld, w, w_ld))
     return intent::i8_generic_launch(a, M, K, a_ld, w, N, w_ld, nullptr, nullptr, bias, c, c_ld, false, stream);
-  return launch_i8<Epi::kI32Bias>(a, M, K, a_ld, nullptr, w, N, w_ld, nullptr, bias, c, c_ld, stream, "i8_gemm_i32");
+  return launch_i8<Epi::kI32Bias>(a, M, K, a_ld, nullptr, w, N, w_ld, nullptr, bias, c, c_ld, stream);
 }
 
 namespace {

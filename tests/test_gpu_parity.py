@@ -468,6 +468,20 @@ def test_w4a16_split_k(gpu, threads, M, K, N, group, pad):
     assert_close_rms(y.cpu().numpy(), ref, what=f"w4a16 split {M}x{K}x{N} g{group}")
 
 
+# Every tile whose K is split (the kernel's name carries tile and runs), with rows and columns off it.
+@pytest.mark.parametrize("M,K,N,kernel", [(17, 896, 1534, "w8a16_matmul<64x128, 8 runs>"),
+                                          (21, 576, 65, "w8a16_matmul<128x128, 8 runs>"),
+                                          (2125, 5312, 141, "w8a16_matmul<256x192, 16 runs>")])
+def test_w8a16_split_tiles(gpu, threads, M, K, N, kernel):
+    d = inputs.config0_w8a16(M + N, M=M, K=K, N=N)
+    a = art(intent.weight_only_int8_matmul)
+    y = a.run(dev(d["x"]), dev(d["w"]), dev(d["scales"]))
+    assert a.observation.kernel == kernel
+    rows = _sample_rows(M)
+    ref = oracle.w8a16(np.ascontiguousarray(d["x"][rows]), d["w"], d["scales"], threads)
+    assert_close_rms(host(y)[rows], ref, what=f"w8a16 {kernel} {M}x{K}x{N}")
+
+
 @pytest.mark.parametrize("M,K,N", [(17, 1088, 130), (65, 4096, 129), (129, 2048, 1001), (300, 8192, 200)])
 def test_w8a16_split_k(gpu, threads, M, K, N):
     d = inputs.config0_w8a16(M + N, M=M, K=K, N=N)
@@ -478,7 +492,7 @@ def test_w8a16_split_k(gpu, threads, M, K, N):
 
 
 # W8A8 with K split over workgroups: runs of unequal length, a last stage of 64 k (K % 128 == 64), rows and
-# columns off the 64-, 128- and 256-row tiles, and an output stride that rules out the vector stores. The int32
+# columns off the 64-row tiles, and an output stride that rules out the vector stores. The int32
 # sums are exact, so every output bit is the oracle's.
 @pytest.mark.parametrize("M,K,N,pad", [(1, 4160, 130, 0), (33, 4096, 257, 1), (64, 3520, 1001, 0), (129, 8192, 128, 0),
                                        (200, 4160, 640, 2), (300, 8192, 1030, 0)])
@@ -490,6 +504,22 @@ def test_w8a8_split_k(gpu, threads, M, K, N, pad):
     ref = oracle.w8a8(d["a"], d["a_scales"], d["w"], d["w_scales"], threads)
     got = y.contiguous().view(torch.int16).cpu().numpy().view(np.uint16)
     assert np.array_equal(got, ref)
+
+
+# Every tile with and without a K split (the kernel's name carries tile and runs), each with K in whole 128-k
+# stages and with a last stage of 64 k, rows off the tiles and off their 32-row blocks, columns off the tiles.
+@pytest.mark.parametrize("M,K,N,kernel", [
+    (33, 384, 204, "64x128"), (45, 320, 205, "64x128"), (69, 256, 3226, "128x128"), (65, 320, 3226, "128x128"),
+    (69, 1408, 70, "128x128, 8 runs"), (67, 1344, 65, "128x128, 8 runs"),
+    (131, 22400, 5444, "256x256, 8 runs"), (198, 13504, 8663, "256x256, 4 runs")])
+def test_w8a8_tiles(gpu, threads, M, K, N, kernel):
+    d = inputs.config3_w8a8(M + N, M=M, K=K, N=N)
+    a = art(intent.w8a8_scaled_matmul)
+    y = a.run(dev(d["a"]), dev(d["a_scales"]), dev(d["w"]), dev(d["w_scales"]))
+    assert a.observation.kernel == f"w8a8_gemm<{kernel}>"
+    cols = np.r_[0:min(N, 300), max(0, N - 300):N]
+    ref = oracle.w8a8(d["a"], d["a_scales"], d["w"][cols], d["w_scales"][cols], threads)
+    assert np.array_equal(y.view(torch.int16).cpu().numpy().view(np.uint16)[:, cols], ref)
 
 
 # More than 64 row blocks of 160 rows (64 experts of ~128 routes): the
@@ -1035,7 +1065,7 @@ def test_deepgemm_fp8(gpu, threads, M, KB, N):
     assert np.max(np.abs(_bf16_bits_to_f64(got) - ref)) <= 1e-2 * np.abs(ref).max()
 
 
-# K split over workgroups (block scales of each run) on both tiles, off their rows and columns, with runs of
+# K split over workgroups (block scales of each run) off the 64-row tile's rows and columns, with runs of
 # unequal length and an output stride that rules out the vector stores.
 @pytest.mark.parametrize("M,KB,N,pad", [(1, 32, 4096, 0), (17, 9, 130, 0), (65, 32, 257, 3), (129, 56, 130, 0),
                                         (300, 25, 200, 0)])
@@ -1050,6 +1080,23 @@ def test_deepgemm_fp8_split_k(gpu, threads, M, KB, N, pad):
     ref = _bf16_bits_to_f64(oracle.deepgemm_fp8(a, sa, b, sb, threads))
     # bf16 output: one rounding of ~2^-8 relative on either side
     assert np.max(np.abs(out.double().cpu().numpy() - ref)) <= 1e-2 * np.abs(ref).max()
+
+
+# Both tiles with and without a K split (the kernel's name carries tile and runs), off their rows and columns.
+@pytest.mark.parametrize("M,KB,N,kernel", [(33, 2, 130, "64x128"), (131, 2, 11257, "128x128"), (17, 9, 130, "64x128, 8 runs"),
+                                           (68, 30, 2113, "128x128, 8 runs"), (2184, 15, 129, "128x128, 4 runs")])
+def test_deepgemm_fp8_tiles(gpu, threads, M, KB, N, kernel):
+    a, b = _fp8_bits(M + 3, (M, KB * 128)), _fp8_bits(N + 4, (N, KB * 128))
+    g = torch.Generator().manual_seed(M + N)
+    sa, sb = (torch.rand(M, KB, generator=g) + 0.25).numpy(), (torch.rand((N + 127) // 128, KB, generator=g) + 0.25).numpy()
+    op = art(intent.deepgemm_fp8_2xacc)
+    out = op.run(dev(a).view(torch.float8_e4m3fn).view(M, KB, 128), dev(b).view(torch.float8_e4m3fn).view(N, KB, 128),
+                 dev(sa), dev(sb))
+    assert op.observation.kernel == f"deepgemm_fp8<{kernel}>"
+    rows = _sample_rows(M)
+    ref = _bf16_bits_to_f64(oracle.deepgemm_fp8(np.ascontiguousarray(a[rows]), np.ascontiguousarray(sa[rows]), b, sb, threads))
+    # bf16 output: one rounding of ~2^-8 relative on either side
+    assert np.max(np.abs(out.double().cpu().numpy()[rows] - ref)) <= 1e-2 * np.abs(ref).max()
 
 
 def test_deepgemm_fp8_reference_inputs(gpu):
@@ -1368,8 +1415,8 @@ def test_moe_expert_ffn_member_list(gpu, T, k):
     assert np.array_equal(lst[:len(order)], order)
 
 
-# Few routes per expert: the 64- and 128-row tiles (R / E up to 52 and 115) with both column widths, widths off
-# them, K runs of the second projection of unequal length, and a workspace without room for the runs.
+# Few routes per expert: the 64- and 128-row tiles (R / E up to 52 and 115) of 128 columns, widths off them, K runs
+# of the second projection of unequal length, and a workspace without room for the runs.
 @pytest.mark.parametrize("T,D,E,k,F,runs", [(1, 64, 4, 1, 64, True), (3, 192, 8, 2, 320, True), (40, 320, 8, 2, 704, True),
                                             (90, 128, 2, 1, 1088, True), (200, 576, 4, 2, 448, True),
                                             (40, 320, 8, 2, 704, False), (300, 64, 3, 1, 1280, True)])
@@ -1388,6 +1435,22 @@ def test_moe_expert_ffn_few_routes(gpu, threads, T, D, E, k, F, runs):
     ref = oracle.moe_expert_ffn(d["x"], d["route_offsets"], d["member_routes"], d["route_token"], d["route_weights"],
                                 d["w1"], d["w2"], y=y0.copy(), threads=threads)
     assert_close_rms(host(y) - y0, ref - y0, what=f"moe_expert_ffn few routes {T}x{D}x{F}")
+
+
+# 256-column tiles of 64 rows in the first, in the second and in both projections, and the 128-row tile, with
+# columns off the tiles: they need many columns, or many K runs of the second projection, to be taken.
+@pytest.mark.parametrize("T,D,E,k,F,kernel", [
+    (40, 64, 8, 2, 10304, "64 rows, 256 and 128 columns, 4 runs"), (40, 3392, 8, 2, 256, "64 rows, 128 and 256 columns, 4 runs"),
+    (40, 1088, 32, 2, 2624, "64 rows, 256 and 256 columns, 4 runs"), (300, 192, 3, 1, 1280, "128 rows, 128 and 128 columns, 4 runs")])
+def test_moe_expert_ffn_tiles(gpu, threads, T, D, E, k, F, kernel):
+    d = inputs.moe_ffn_f16(T + D, T=T, D=D, E=E, top_k=k, F=F, kind="random")
+    y = torch.zeros(T, D, device="cuda")
+    a = art(intent.moe_expert_ffn)
+    a(*(dev(d[n]) for n in ("x", "route_offsets", "member_routes", "route_token", "route_weights", "w1", "w2")), y)
+    assert a.observation.kernel == f"moe_expert_ffn<{kernel}>"
+    ref = oracle.moe_expert_ffn(d["x"], d["route_offsets"], d["member_routes"], d["route_token"], d["route_weights"],
+                                d["w1"], d["w2"], y=np.zeros((T, D), np.float32), threads=threads)
+    assert_close_rms(host(y), ref, what=f"moe_expert_ffn {kernel}")
 
 
 # The launch has exactly as many row tiles as the worst split of the routes needs: one per expert with a route
