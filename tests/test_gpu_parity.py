@@ -509,7 +509,7 @@ def test_w8a8_split_k(gpu, threads, M, K, N, pad):
 # Every tile with and without a K split (the kernel's name carries tile and runs), each with K in whole 128-k
 # stages and with a last stage of 64 k, rows off the tiles and off their 32-row blocks, columns off the tiles.
 @pytest.mark.parametrize("M,K,N,kernel", [
-    (33, 384, 204, "64x128"), (45, 320, 205, "64x128"), (69, 256, 3226, "128x128"), (65, 320, 3226, "128x128"),
+    (32, 384, 204, "128x128"), (33, 384, 204, "64x128"), (45, 320, 205, "64x128"), (69, 256, 3226, "128x128"), (65, 320, 3226, "128x128"),
     (69, 1408, 70, "128x128, 8 runs"), (67, 1344, 65, "128x128, 8 runs"),
     (131, 22400, 5444, "256x256, 8 runs"), (198, 13504, 8663, "256x256, 4 runs")])
 def test_w8a8_tiles(gpu, threads, M, K, N, kernel):
@@ -520,6 +520,21 @@ def test_w8a8_tiles(gpu, threads, M, K, N, kernel):
     cols = np.r_[0:min(N, 300), max(0, N - 300):N]
     ref = oracle.w8a8(d["a"], d["a_scales"], d["w"][cols], d["w_scales"][cols], threads)
     assert np.array_equal(y.view(torch.int16).cpu().numpy().view(np.uint16)[:, cols], ref)
+
+
+# The same kernels with int32 output, which has no K split: 128-row tiles up to 32 rows, 64-row ones above.
+@pytest.mark.parametrize("M,K,N,kernel", [(1, 2048, 300, "128x128"), (32, 1088, 205, "128x128"), (33, 2048, 300, "64x128"),
+                                          (45, 1088, 205, "64x128"), (69, 320, 3226, "128x128")])
+def test_i8_gemm_i32_tiles(gpu, threads, M, K, N, kernel):
+    rng = np.random.default_rng(M + N)
+    x, w = rng.integers(-127, 128, size=(M, K), dtype=np.int8), rng.integers(-127, 128, size=(N, K), dtype=np.int8)
+    bias = rng.integers(-1000, 1000, size=N, dtype=np.int32)
+    c = torch.empty(M, N, dtype=torch.int32, device="cuda")
+    X, W, B = dev(x), dev(w), dev(bias)
+    _native.call("intent_i8_gemm_i32", X.data_ptr(), M, K, K, W.data_ptr(), N, K, B.data_ptr(), c.data_ptr(), N,
+                 torch.cuda.current_stream().cuda_stream)
+    assert _native.last_kernel() == f"i8_gemm_i32<{kernel}>"
+    assert np.array_equal(host(c), oracle.i8_gemm_i32(x, w, bias, threads))
 
 
 # More than 64 row blocks of 160 rows (64 experts of ~128 routes): the
