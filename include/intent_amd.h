@@ -118,7 +118,7 @@ int intent_w4a16_gemm(const void* x, int64_t M, int64_t K, int64_t x_ld,
                       const void* scales, const uint8_t* zeros, int64_t qparam_ld,
                       int64_t group_size,
                       void* y, int64_t y_ld, void* stream);
-/* The GEMM with a workspace for a K split (see intent_w8a16_matmul_ws). */
+/* The tiled GEMM with a workspace for a K split (see intent_w8a16_matmul_ws). */
 size_t intent_w4a16_gemm_workspace_size(int64_t M, int64_t K, int64_t N, int64_t group_size);
 int intent_w4a16_gemm_ws(const void* x, int64_t M, int64_t K, int64_t x_ld,
                          const uint8_t* packed, int64_t N, int64_t packed_ld,
@@ -126,8 +126,9 @@ int intent_w4a16_gemm_ws(const void* x, int64_t M, int64_t K, int64_t x_ld,
                          int64_t group_size,
                          void* y, int64_t y_ld,
                          void* workspace, size_t workspace_bytes, void* stream);
-/* The entry that picks by M, with a workspace: as intent_w4a16_gemm_ws above M =
- * 16; up to 16 rows a K split too where that beats the GEMV (size 0 elsewhere). */
+/* The entry that picks the kernel, with a workspace: from 2 to 128 rows the
+ * weight-streaming kernel with its partial sums where it is the fastest, else the
+ * GEMV up to M = 16 (no workspace) and the GEMM as intent_w4a16_gemm_ws above. */
 size_t intent_w4a16_matmul_workspace_size(int64_t M, int64_t K, int64_t N, int64_t group_size);
 int intent_w4a16_matmul_ws(const void* x, int64_t M, int64_t K, int64_t x_ld,
                            const uint8_t* packed, int64_t N, int64_t packed_ld,

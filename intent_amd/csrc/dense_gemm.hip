@@ -1043,31 +1043,31 @@ int w4a16_gemv_launch(const void* x, int64_t M, int64_t K, int64_t x_ld, const u
 int w8a16_gemv_launch(const void* x, int64_t M, int64_t K, int64_t x_ld, const int8_t* w, int64_t N, int64_t w_ld,
                       const void* scales, void* y, int64_t y_ld, void* stream);
 
-double w4a16_skinny_us(int64_t M, int64_t N, int64_t K, int64_t gs);
-size_t w4a16_skinny_bytes(int64_t M, int64_t N, int64_t K, int64_t gs);
+double w4a16_skinny_us(int64_t M, int64_t N, int64_t K, int64_t gs, size_t* bytes);
 int w4a16_skinny_launch(const void* x, int64_t M, int64_t K, int64_t x_ld, const uint8_t* packed, int64_t N,
                         int64_t packed_ld, const void* scales, const uint8_t* zeros, int64_t qparam_ld, int64_t gs,
                         void* y, int64_t y_ld, void* ws, void* stream);
 
-// Whether the weight-streaming kernel (w4a16_skinny.hip) is the fastest for the
-// call. Above M = 16 it is weighed against the tiled plan. Up to 16 rows, against
-// the MFMA GEMV, whose workgroups of 16 weight rows each read all of x: 1.2 us and
-// per round of 256 workgroups 1.6 us + 1 us per 1000 k (measured: N = 11008, K =
+// Scratch of the weight-streaming kernel (w4a16_skinny.hip) where it is the fastest
+// for the call, else 0. Above M = 16 it is weighed against the tiled plan. Up to 16
+// rows, against the MFMA GEMV, whose workgroups of 16 weight rows each read all of x:
+// 1.2 us and per round of 256 workgroups 1.6 us + 1 us per 1000 k (measured: N = 11008, K =
 // 4096 17 us, N = 14336, K = 2048 13.5, N = K = 8192 20, N = 4096, K = 14336 19..23);
 // where the dot-product GEMV (no weight rounded to f16) takes the call, it stays.
 // Very wide outputs are weighed the same way (N = 128256, K = 4096: M = 48 117 us
 // here against 145 in 128-row tiles, M = 77 188 against 143, 128 310 against 151).
-bool w4a16_wants_skinny(int64_t M, int64_t N, int64_t K, int64_t gs) {
-  const double us = w4a16_skinny_us(M, N, K, gs);
-  if (us == 0) return false;
+size_t w4a16_wants_skinny(int64_t M, int64_t N, int64_t K, int64_t gs) {
+  if (M < 2 || (M == 2 && K <= 8192) || (M <= 5 && K <= 4096)) return 0;
+  size_t bytes = 0;
+  const double us = w4a16_skinny_us(M, N, K, gs, &bytes);
+  if (us == 0) return 0;
   if (M > 16) {
     double tiled;  // the estimate is up to 0.8 of the measured time for 4 runs or more, up to 1.1 of it for fewer
     const DensePlan p = w4_plan(M, N, K, gs, true, &tiled);
-    return us < (p.splits > 2 ? 1.2 : 0.9) * tiled;
+    return us < (p.splits > 2 ? 1.2 : 0.9) * tiled ? bytes : 0;
   }
-  if (M < 2 || (M == 2 && K <= 8192) || (M <= 5 && K <= 4096)) return false;
   const double rounds = (double)((N + 4095) / 4096);
-  return us < 0.9 * (1.2 + rounds * (1.6 + 1e-3 * (double)K));
+  return us < 0.9 * (1.2 + rounds * (1.6 + 1e-3 * (double)K)) ? bytes : 0;
 }
 
 int w4a16_gemm_launch(const void* x, int64_t M, int64_t K, int64_t x_ld, const uint8_t* packed, int64_t N,
@@ -1084,9 +1084,6 @@ int w4a16_gemm_launch(const void* x, int64_t M, int64_t K, int64_t x_ld, const u
   f16* yy = (f16*)y;
   hipStream_t st = (hipStream_t)stream;
   const bool win = gs % 64 == 0 && qparam_ld % 4 == 0 && intent::aligned4(scales) && intent::aligned4(zeros);
-  if (w4a16_wants_skinny(M, N, K, gs) && ws && aligned16(ws) && ws_bytes >= w4a16_skinny_bytes(M, N, K, gs) &&
-      fits_offset(M, x_ld * 2))
-    return w4a16_skinny_launch(x, M, K, x_ld, packed, N, packed_ld, scales, zeros, qparam_ld, gs, y, y_ld, ws, stream);
   const W4Cut cut = w4_cut(K, gs);
   const DensePlan split = w4_plan(M, N, K, gs, true);
   if (split_ready(split, M, N, ws, ws_bytes)) {
@@ -1200,34 +1197,37 @@ extern "C" size_t intent_w4a16_gemm_workspace_size(int64_t M, int64_t K, int64_t
   if (M <= 0 || N <= 0 || K <= 0 || K % 128 != 0 || !(group_size == 32 || (group_size > 0 && group_size % 64 == 0)) ||
       K % group_size != 0)
     return 0;
-  if (intent::w4a16_wants_skinny(M, N, K, group_size)) return intent::w4a16_skinny_bytes(M, N, K, group_size);
   return (size_t)dense_split_bytes(w4_plan(M, N, K, group_size, true), M, N);
 }
 
 extern "C" size_t intent_w4a16_matmul_workspace_size(int64_t M, int64_t K, int64_t N, int64_t group_size) {
-  if (M > 16) return intent_w4a16_gemm_workspace_size(M, K, N, group_size);
   if (M <= 0 || N <= 0 || K <= 0 || K % 128 != 0 || group_size <= 0 || group_size % 32 != 0 || K % group_size != 0)
     return 0;
-  return intent::w4a16_wants_skinny(M, N, K, group_size) ? intent::w4a16_skinny_bytes(M, N, K, group_size) : 0;
+  const size_t skinny = intent::w4a16_wants_skinny(M, N, K, group_size);
+  return skinny > 0 || M <= 16 ? skinny : intent_w4a16_gemm_workspace_size(M, K, N, group_size);
 }
 
 extern "C" int intent_w4a16_matmul_ws(const void* x, int64_t M, int64_t K, int64_t x_ld, const uint8_t* packed,
                                       int64_t N, int64_t packed_ld, const void* scales, const uint8_t* zeros,
                                       int64_t qparam_ld, int64_t group_size, void* y, int64_t y_ld, void* workspace,
                                       size_t workspace_bytes, void* stream) {
-  if (M > 16)
-    return intent_w4a16_gemm_ws(x, M, K, x_ld, packed, N, packed_ld, scales, zeros, qparam_ld, group_size, y, y_ld,
-                                workspace, workspace_bytes, stream);
   intent::clear_error();
   int st = intent::w4a16_check(x, M, K, x_ld, packed, N, packed_ld, scales, zeros, qparam_ld, group_size, y, y_ld);
   if (st != INTENT_OK) return st;
-  if (M > 0 && N > 0 && intent::w4a16_fast(x, K, x_ld, packed, packed_ld, group_size) &&
-      intent::w4a16_wants_skinny(M, N, K, group_size) && workspace && intent::aligned16(workspace) &&
-      workspace_bytes >= intent::w4a16_skinny_bytes(M, N, K, group_size) && intent::fits_offset(N, packed_ld) &&
-      intent::fits_offset(M, x_ld * 2))
-    return intent::w4a16_skinny_launch(x, M, K, x_ld, packed, N, packed_ld, scales, zeros, qparam_ld, group_size, y,
-                                       y_ld, workspace, stream);
-  return intent_w4a16_matmul(x, M, K, x_ld, packed, N, packed_ld, scales, zeros, qparam_ld, group_size, y, y_ld, stream);
+  const bool fast = intent::w4a16_fast(x, K, x_ld, packed, packed_ld, group_size);
+  // above 16 rows the limits of the tiled kernels hold for both
+  if (M > 0 && N > 0 && fast && workspace && intent::aligned16(workspace) && intent::fits_offset(N, packed_ld) && intent::fits_offset(M, x_ld * 2) &&
+      (M <= 16 || (intent::fits_offset(N, qparam_ld * 2) && intent::fits_offset(256 + 1, x_ld * 2)))) {
+    const size_t skinny = intent::w4a16_wants_skinny(M, N, K, group_size);
+    if (skinny > 0 && workspace_bytes >= skinny)
+      return intent::w4a16_skinny_launch(x, M, K, x_ld, packed, N, packed_ld, scales, zeros, qparam_ld, group_size, y,
+                                         y_ld, workspace, stream);
+  }
+  if (M <= 16 && fast)
+    return intent::w4a16_gemv_launch(x, M, K, x_ld, packed, N, packed_ld, scales, zeros, qparam_ld, group_size, y,
+                                     y_ld, stream);
+  return intent::w4a16_gemm_launch(x, M, K, x_ld, packed, N, packed_ld, scales, zeros, qparam_ld, group_size, y, y_ld,
+                                   workspace, workspace_bytes, stream);
 }
 
 extern "C" int intent_w4a16_gemm_ws(const void* x, int64_t M, int64_t K, int64_t x_ld, const uint8_t* packed, int64_t N,

@@ -145,16 +145,13 @@ Plan skinny_plan(int64_t M, int64_t N, int64_t K, int64_t gs) {
 namespace intent {
 
 // Microseconds the kernel takes, fitted to 60 shapes (M 2..128, N 1024..14336, K
-// 2048..14336) within about 10%; 0 where it does not take the call.
-double w4a16_skinny_us(int64_t M, int64_t N, int64_t K, int64_t gs) {
+// 2048..14336) within about 10%; 0 where it does not take the call. bytes: its scratch.
+double w4a16_skinny_us(int64_t M, int64_t N, int64_t K, int64_t gs, size_t* bytes) {
   const Plan p = skinny_plan(M, N, K, gs);
   if (p.unit == 0) return 0;
+  *bytes = (size_t)partial_bytes(p, N);
   const double work = (double)((N + kRows - 1) / kRows) * (double)(K / 128) / 8;
   return 5.2 + 0.6 * p.tb + work * (0.0046 + 0.0034 * p.tb);
-}
-
-size_t w4a16_skinny_bytes(int64_t M, int64_t N, int64_t K, int64_t gs) {
-  return (size_t)partial_bytes(skinny_plan(M, N, K, gs), N);
 }
 
 // A w4a16_fast call whose plan exists, with 31-bit offsets checked by the caller.

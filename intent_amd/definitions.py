@@ -141,13 +141,14 @@ def _w4_launch(v: dict, env: dict, stream: int, workspace) -> str:
         scratch = _split_scratch(_native.library().intent_w4a16_gemm_workspace_size(*size), y)
     else:
         scratch = _split_scratch(_native.library().intent_w4a16_matmul_workspace_size(*size), y)
+    if scratch is not None:
+        entry = "intent_w4a16_gemm_ws" if kernel == "gemm" else "intent_w4a16_matmul_ws"
+        _native.call(entry, _ptr(x), env["M"], env["K"], _ld(x), _ptr(q), env["N"], _ld(q), _ptr(s), _ptr(z), s.stride(0),
+                     env["GROUP"], _ptr(y), _ld(y), _ptr(scratch), scratch.numel(), stream)
+        return entry
+    if kernel == "auto":
         kernel = "gemv" if env["M"] <= 16 else "gemm"
     entry = {"gemv": "intent_w4a16_gemv", "gemm": "intent_w4a16_gemm"}[kernel]
-    if scratch is not None:
-        split = "intent_w4a16_gemm_ws" if kernel == "gemm" else "intent_w4a16_matmul_ws"
-        _native.call(split, _ptr(x), env["M"], env["K"], _ld(x), _ptr(q), env["N"], _ld(q), _ptr(s), _ptr(z), s.stride(0),
-                     env["GROUP"], _ptr(y), _ld(y), _ptr(scratch), scratch.numel(), stream)
-        return entry if kernel == "gemm" else split
     _native.call(entry, _ptr(x), env["M"], env["K"], _ld(x), _ptr(q), env["N"], _ld(q), _ptr(s), _ptr(z),
                  s.stride(0), env["GROUP"], _ptr(y), _ld(y), stream)
     return entry

@@ -453,9 +453,28 @@ def test_w4a16_skinny(gpu, threads, M, K, N, group, pad):
     assert_close_rms(host(y)[:, cols], ref, what=f"w4a16 skinny {M}x{K}x{N} g{group}")
 
 
-# K split over workgroups (partial sums through scratch) and the 64-, 128- and 256-row tiles: rows and
-# columns off the tiles, runs of unequal length (11 or 43 units over 8 runs), every group form the cut takes
-# (windowed, whole groups, 32), and an output whose row stride rules out the vector stores.
+# KERNEL = "gemm" forces the tiled kernels, also at the rows where the weight-streaming one is the faster: every
+# tile whose K is split (the kernel's name carries tile and runs) with windowed and with per-stage group parameters,
+# rows and columns off the tiles.
+@pytest.mark.parametrize("M,K,N,group,kernel", [
+    (17, 7168, 66, 128, "64x128, 8 runs"), (17, 896, 1534, 64, "64x128, 8 runs"), (19, 2048, 73, 64, "128x128, 8 runs"),
+    (18, 640, 66, 128, "128x128, 4 runs"), (17, 512, 65, 32, "128x128, 8 runs"),
+    (2136, 5376, 148, 64, "256x192, 16 runs"), (2118, 4352, 133, 128, "256x192, 16 runs"), (77, 4096, 4096, 128, ""),
+    (12, 4096, 11008, 128, "")])
+def test_w4a16_gemm_forced(gpu, threads, M, K, N, group, kernel):
+    d = inputs.config1_w4a16_decode(M + N, M=M, K=K, N=N, group=group)
+    a = art(intent.weight_only_int4_asym_matmul, KERNEL="gemm")
+    y = a.run(dev(d["x"]), dev(d["packed"]), dev(d["scales"]), dev(d["zeros"]))
+    name = a.observation.kernel
+    assert name == f"w4a16_gemm<{kernel}>" if kernel else name.startswith("w4a16_gemm<"), name
+    rows, cols = _sample_rows(M), np.r_[0:min(N, 700), max(0, N - 70):N]
+    ref = oracle.w4a16(np.ascontiguousarray(d["x"][rows]), d["packed"][cols], d["scales"][cols], d["zeros"][cols], threads)
+    assert_close_rms(host(y)[np.ix_(rows, cols)], ref, what=f"w4a16 {name} {M}x{K}x{N} g{group}")
+
+
+# K split over workgroups (partial sums through scratch): rows and columns off the 64- and 128-row tiles, runs of
+# unequal length (11 or 43 units over 8 runs), every group form the cut takes (windowed, whole groups, 32), and an
+# output whose row stride rules out the vector stores.
 @pytest.mark.parametrize("M,K,N,group,pad", [
     (17, 1408, 130, 128, 0), (64, 2048, 257, 64, 0), (65, 4096, 128, 128, 3), (129, 5504, 193, 128, 0),
     (200, 3072, 1001, 32, 0), (300, 8192, 129, 256, 0), (256, 4096, 640, 128, 1), (513, 4096, 200, 64, 0)])
@@ -463,7 +482,9 @@ def test_w4a16_split_k(gpu, threads, M, K, N, group, pad):
     d = inputs.config1_w4a16_decode(M + N, M=M, K=K, N=N, group=group)
     assert _native.library().intent_w4a16_gemm_workspace_size(M, K, N, group) > 0
     y = torch.zeros(M, N + pad, dtype=torch.float16, device="cuda")[:, :N]
-    art(intent.weight_only_int4_asym_matmul)(dev(d["x"]), dev(d["packed"]), dev(d["scales"]), dev(d["zeros"]), y)
+    a = art(intent.weight_only_int4_asym_matmul, KERNEL="gemm")
+    a(dev(d["x"]), dev(d["packed"]), dev(d["scales"]), dev(d["zeros"]), y)
+    assert a.observation.kernel.startswith("w4a16_gemm<") and "runs" in a.observation.kernel, a.observation.kernel
     ref = oracle.w4a16(d["x"], d["packed"], d["scales"], d["zeros"], threads)
     assert_close_rms(y.cpu().numpy(), ref, what=f"w4a16 split {M}x{K}x{N} g{group}")
 
