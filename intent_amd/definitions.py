@@ -47,6 +47,9 @@ class KernelDefinition:
     workspace: Callable[[dict], int] | None = None
     reference: str = ""
     doc: str = ""
+    # bytes of a launch's own scratch (never shared between launches that may overlap; 0: none).
+    # The launch gets it in the place of the workspace, or None where it could not be allocated.
+    scratch: Callable[[dict], int] | None = None
 
     @property
     def __name__(self) -> str:  # the reference uses definition.__name__ as the entry name
@@ -103,17 +106,6 @@ def _ld(t) -> int:
     return t.stride(0) if t.dim() >= 2 else t.shape[0]
 
 
-def _split_scratch(nbytes: int, like):
-    """Scratch of a K split for one launch: from torch's allocator on the launch stream (which
-    reuses it only after that stream has passed the launch), so that calls of one artifact on
-    several streams or threads never share it. None when the call needs none."""
-    if nbytes == 0:
-        return None
-    import torch
-
-    return torch.empty(nbytes, dtype=torch.uint8, device=like.device)
-
-
 # ---- W4A16 ------------------------------------------------------------------------
 
 def _w4_check(env: dict) -> None:
@@ -129,18 +121,20 @@ def _w4_check(env: dict) -> None:
         raise ValueError("KERNEL must be 'auto', 'gemv' or 'gemm'")
 
 
-def _w4_launch(v: dict, env: dict, stream: int, workspace) -> str:
+def _w4_scratch(env: dict) -> int:
+    size = (env["M"], env["K"], env["N"], env["GROUP"])
+    if env["KERNEL"] == "gemv":
+        return 0
+    if env["KERNEL"] == "gemm":
+        return _native.library().intent_w4a16_gemm_workspace_size(*size)
+    return _native.library().intent_w4a16_matmul_workspace_size(*size)
+
+
+def _w4_launch(v: dict, env: dict, stream: int, scratch) -> str:
     x, q, s, z, y = v["activation"], v["packed_weight"], v["scales"], v["zeros"], v["output"]
     if s.stride(0) != z.stride(0):
         raise ValueError("scales and zeros must share a row stride")
     kernel = env["KERNEL"]
-    size = (env["M"], env["K"], env["N"], env["GROUP"])
-    if kernel == "gemv":
-        scratch = None
-    elif kernel == "gemm":
-        scratch = _split_scratch(_native.library().intent_w4a16_gemm_workspace_size(*size), y)
-    else:
-        scratch = _split_scratch(_native.library().intent_w4a16_matmul_workspace_size(*size), y)
     if scratch is not None:
         entry = "intent_w4a16_gemm_ws" if kernel == "gemm" else "intent_w4a16_matmul_ws"
         _native.call(entry, _ptr(x), env["M"], env["K"], _ld(x), _ptr(q), env["N"], _ld(q), _ptr(s), _ptr(z), s.stride(0),
@@ -164,6 +158,7 @@ weight_only_int4_asym_matmul = KernelDefinition(
         Param("output", "f16", ("M", "N"), OUT, leading_stride=True),
     ),
     launch=_w4_launch,
+    scratch=_w4_scratch,
     constexprs={"KERNEL": "auto"},
     check=_w4_check,
     reference="examples/kernels/contraction/weight_only_int4.py:18-51",
@@ -173,11 +168,12 @@ weight_only_int4_asym_matmul = KernelDefinition(
 
 # ---- W8A16 ------------------------------------------------------------------------
 
-def _w8a16_launch(v: dict, env: dict, stream: int, workspace) -> str:
+def _w8a16_scratch(env: dict) -> int:
+    return _native.library().intent_w8a16_matmul_workspace_size(env["M"], env["K"], env["N"])
+
+
+def _w8a16_launch(v: dict, env: dict, stream: int, scratch) -> str:
     x, w, s, y = v["activation"], v["weight"], v["scales"], v["output"]
-    scratch = None
-    if env["M"] > 16:
-        scratch = _split_scratch(_native.library().intent_w8a16_matmul_workspace_size(env["M"], env["K"], env["N"]), y)
     if scratch is not None:
         _native.call("intent_w8a16_matmul_ws", _ptr(x), env["M"], env["K"], _ld(x), _ptr(w), env["N"], _ld(w), _ptr(s),
                      _ptr(y), _ld(y), _ptr(scratch), scratch.numel(), stream)
@@ -196,6 +192,7 @@ weight_only_int8_matmul = KernelDefinition(
         Param("output", "f16", ("M", "N"), OUT, leading_stride=True),
     ),
     launch=_w8a16_launch,
+    scratch=_w8a16_scratch,
     reference="doc/dsl/core.en.md:246 (I.cast(W_i8, f16) -> I.matmul(acc f32) -> scale)",
     doc="y = f16(scale[n] * (x @ w.T)), per-channel int8 weights",
 )
@@ -203,9 +200,12 @@ weight_only_int8_matmul = KernelDefinition(
 
 # ---- W8A8 -------------------------------------------------------------------------
 
-def _w8a8_launch(v: dict, env: dict, stream: int, workspace) -> str:
+def _w8a8_scratch(env: dict) -> int:
+    return _native.library().intent_w8a8_gemm_workspace_size(env["M"], env["K"], env["N"])
+
+
+def _w8a8_launch(v: dict, env: dict, stream: int, scratch) -> str:
     a, sa, w, sw, out = v["activation"], v["activation_scales"], v["weight"], v["weight_scales"], v["output"]
-    scratch = _split_scratch(_native.library().intent_w8a8_gemm_workspace_size(env["M"], env["K"], env["N"]), out)
     if scratch is not None:
         _native.call("intent_w8a8_gemm_ws", _ptr(a), env["M"], env["K"], _ld(a), _ptr(sa), _ptr(w), env["N"], _ld(w),
                      _ptr(sw), _ptr(out), _ld(out), _ptr(scratch), scratch.numel(), stream)
@@ -225,6 +225,7 @@ w8a8_scaled_matmul = KernelDefinition(
         Param("output", "bf16", ("M", "N"), OUT, leading_stride=True),
     ),
     launch=_w8a8_launch,
+    scratch=_w8a8_scratch,
     reference="lib/Conversion/KIRToCPU/Contractions.cpp:30-35 + examples/kernels/contraction/gemm.py:83-106",
     doc="out = bf16(f32(int32 acc) * sa[m] * sw[n])",
 )
@@ -875,10 +876,13 @@ def _deepgemm_check(env: dict) -> None:
         raise ValueError(f"rhs_scale has {env['NB']} row blocks; N = {env['N']} needs {(env['N'] + 127) // 128}")
 
 
-def _deepgemm_launch(v: dict, env: dict, stream: int, workspace) -> str:
+def _deepgemm_scratch(env: dict) -> int:
+    return _native.library().intent_deepgemm_fp8_workspace_size(env["M"], env["KB"] * 128, env["N"])
+
+
+def _deepgemm_launch(v: dict, env: dict, stream: int, scratch) -> str:
     lhs, rhs, ls, rs, out = v["lhs"], v["rhs"], v["lhs_scale"], v["rhs_scale"], v["output"]
     M, KB, N = env["M"], env["KB"], env["N"]
-    scratch = _split_scratch(_native.library().intent_deepgemm_fp8_workspace_size(M, KB * 128, N), out)
     if scratch is not None:
         _native.call("intent_deepgemm_fp8_ws", _ptr(lhs), M, KB * 128, KB * 128, _ptr(ls), KB, _ptr(rhs), N, KB * 128,
                      _ptr(rs), KB, _ptr(out), _ld(out), _ptr(scratch), scratch.numel(), stream)
@@ -898,6 +902,7 @@ deepgemm_fp8_2xacc = KernelDefinition(
         Param("output", "bf16", ("M", "N"), OUT, leading_stride=True),
     ),
     launch=_deepgemm_launch,
+    scratch=_deepgemm_scratch,
     check=_deepgemm_check,
     reference="examples/kernels/contraction/block_scaled.py:101-122",
     doc="output = bf16(sum over k-blocks of (lhs . rhs) * lhs_scale[m, kb] * rhs_scale[n // 128, kb])",

@@ -58,6 +58,7 @@ class _Layout:
     spans: tuple
     pairs: tuple
     workspace: int      # bytes, -1 without one
+    scratch: int        # bytes of a launch's own scratch
 
 
 MAX_LAYOUTS = 256  # layouts kept per artifact and calling form; the oldest go first
@@ -154,13 +155,13 @@ class HIPRuntime:
                 t = torch.empty(shape, dtype=dt, device=self._home_device())
                 views[name] = t
                 outputs.append(t)
-            return Binding(views, env, tuple(outputs), self._workspace_of(known.workspace))
+            return Binding(views, env, tuple(outputs), self._buffer_of(known.workspace, known.scratch))
         outputs = ()
         if supplied_outputs:
             outputs = tuple(views[p.name] for p in params if p.name not in self._scalars and p.access is ViewKind.OUT)
-        return Binding(views, env, outputs, self._workspace_of(known.workspace))
+        return Binding(views, env, outputs, self._buffer_of(known.workspace, known.scratch))
 
-    def _remember(self, arguments: tuple, supplied_outputs: bool, binding: Binding) -> None:
+    def _remember(self, arguments: tuple, supplied_outputs: bool, binding: Binding, workspace: int, scratch: int) -> None:
         params = self.definition.params if supplied_outputs else self._supplied
         key = self._layout_key(params, arguments)
         if key is None:
@@ -177,8 +178,7 @@ class HIPRuntime:
         if len(known) >= MAX_LAYOUTS:
             for old in list(known)[:MAX_LAYOUTS // 2]:
                 known.pop(old, None)
-        need = -1 if self.definition.workspace is None else int(self.definition.workspace(binding.env))
-        known[key] = _Layout(dict(binding.env), tuple(p.name for p, _ in views), made, spans, pairs, need)
+        known[key] = _Layout(dict(binding.env), tuple(p.name for p, _ in views), made, spans, pairs, workspace, scratch)
 
     # ---- binding ------------------------------------------------------------
     def _bind(self, arguments: tuple, explicit_outputs: tuple | None, abstract: bool = False) -> Binding:
@@ -290,8 +290,24 @@ class HIPRuntime:
                 if s0 < e1 and s1 < e0:
                     raise ValueError(f"{self.definition.name}: {a} and {b} overlap; writable views must not alias")
 
-    def _workspace_for(self, env: dict):
-        return self._workspace_of(-1 if self.definition.workspace is None else self.definition.workspace(env))
+    def _needs(self, env: dict) -> tuple[int, int]:
+        """Bytes of the workspace (-1 without one) and of a launch's own scratch."""
+        d = self.definition
+        return (-1 if d.workspace is None else int(d.workspace(env)), 0 if d.scratch is None else int(d.scratch(env)))
+
+    def _buffer_of(self, workspace: int, scratch: int):
+        return self._scratch_of(scratch) if scratch > 0 else self._workspace_of(workspace)
+
+    def _scratch_of(self, need: int):
+        """Scratch of one launch: from torch's allocator on the launch stream (which reuses it only
+        after that stream has passed the launch), so that calls of one artifact on several streams or
+        threads never share it. None when memory is short: the call then runs without it."""
+        import torch
+
+        try:
+            return torch.empty(need, dtype=torch.uint8, device=self._home_device())
+        except torch.OutOfMemoryError:
+            return None
 
     def _workspace_of(self, need: int):
         if need < 0:
@@ -313,8 +329,9 @@ class HIPRuntime:
 
     def run(self, *arguments):
         binding = self._bind(arguments, None)
-        self._remember(arguments, False, binding)
-        binding.workspace = self._workspace_for(binding.env)
+        needs = self._needs(binding.env)
+        self._remember(arguments, False, binding, *needs)
+        binding.workspace = self._buffer_of(*needs)
         return self.launch_bound(binding)
 
     def launch(self, *arguments):
@@ -327,15 +344,17 @@ class HIPRuntime:
         outs = tuple(a for a, p in zip(arguments, interface.parameters) if getattr(p, "output", False))
         assert len(ins) == n_in
         binding = self._bind(ins, outs)
-        self._remember(arguments, True, binding)
-        binding.workspace = self._workspace_for(binding.env)
+        needs = self._needs(binding.env)
+        self._remember(arguments, True, binding, *needs)
+        binding.workspace = self._buffer_of(*needs)
         self._launch(binding)
         return None
 
     def prepare_call(self, arguments: tuple, *, outputs: tuple | None = None) -> "HIPPreparedCall":
         binding = self._bind(tuple(arguments), outputs)
-        binding.workspace = self._workspace_for(binding.env)
-        return HIPPreparedCall(self, binding)
+        workspace, scratch = self._needs(binding.env)
+        binding.workspace = self._buffer_of(workspace, scratch)
+        return HIPPreparedCall(self, binding, owns_scratch=scratch > 0)
 
     def infer_outputs(self, arguments: tuple):
         binding = self._bind(tuple(arguments), None, abstract=True)
@@ -359,16 +378,25 @@ def _result(outputs: tuple):
 
 
 class HIPPreparedCall:
-    """Invocation-owned arguments and outputs; launch() runs on torch's current stream."""
+    """Invocation-owned arguments, outputs and scratch; launch() runs on torch's current stream.
 
-    def __init__(self, runtime: HIPRuntime, binding: Binding):
+    launch() allocates nothing, so a capture of it (torch.cuda.graph or a plain stream capture) holds
+    only addresses that the prepared call keeps: it must outlive the graph."""
+
+    def __init__(self, runtime: HIPRuntime, binding: Binding, owns_scratch: bool = False):
         self._runtime = runtime
         self._binding = binding
+        # the stream whose order the allocator follows when the scratch is given back
+        self._stream = _current_stream(runtime.device) if owns_scratch and binding.workspace is not None else None
 
     def compile(self) -> None:
         _native.library()  # the code objects are prebuilt; this validates the library and ABI
 
     def launch(self) -> None:
+        if self._stream is not None and _current_stream(self._runtime.device) != self._stream:
+            import torch
+
+            self._binding.workspace.record_stream(torch.cuda.current_stream(self._runtime.device))
         self._runtime._launch(self._binding)
 
     def result(self):

@@ -228,3 +228,63 @@ def test_known_layouts_scalars_and_bound(monkeypatch):
         rt.run(torch.zeros(m, 128, dtype=torch.float8_e4m3fn), rhs, 1.0, 1.0)
         assert len(rt._layouts[0]) <= 4
     assert rt.rebind((torch.zeros(11, 128, dtype=torch.float8_e4m3fn), rhs, 1.0, 1.0), False) is not None
+
+
+def _split_call(monkeypatch):
+    """A W8A8 call whose plan has K runs, on CPU tensors, with the library's calls recorded."""
+    from intent_amd import _native
+    from intent_amd import runtime as runtime_module
+
+    rt = runtime_for(intent.w8a8_scaled_matmul)
+    rt._home = torch.device("cpu")
+    calls = []
+    monkeypatch.setattr(_native, "call", lambda entry, *a: calls.append((entry, a)))
+    monkeypatch.setattr(runtime_module, "_current_stream", lambda device: 0)
+    M, K, N = 32, 4096, 512
+    size = _native.library().intent_w8a8_gemm_workspace_size(M, K, N)
+    assert size > 0
+    args = (torch.zeros(M, K, dtype=torch.int8), torch.zeros(M), torch.zeros(N, K, dtype=torch.int8), torch.zeros(N))
+    return rt, args, size, calls
+
+
+def test_prepared_call_owns_its_scratch(monkeypatch):
+    rt, args, size, calls = _split_call(monkeypatch)
+    prepared = rt.prepare_call(args)
+    other = rt.prepare_call(args)
+    with monkeypatch.context() as m:
+        m.setattr(torch, "empty", lambda *a, **k: pytest.fail("a prepared launch allocated"))
+        prepared.launch()
+        other.launch()
+        prepared.launch()
+    assert [entry for entry, _ in calls] == ["intent_w8a8_gemm_ws"] * 3
+    first, second, third = (a[-3:-1] for _, a in calls)  # scratch address and bytes
+    assert first == third and first[1] == second[1] == size and first[0] != second[0]
+    assert first[0] == prepared._binding.workspace.data_ptr()
+
+
+def test_split_call_without_memory_for_its_scratch(monkeypatch):
+    rt, args, size, calls = _split_call(monkeypatch)
+    empty = torch.empty
+
+    def short(*shape, **kw):
+        if kw.get("dtype") is torch.uint8:
+            raise torch.OutOfMemoryError("no memory for scratch")
+        return empty(*shape, **kw)
+
+    monkeypatch.setattr(torch, "empty", short)
+    rt.run(*args)
+    rt.launch_bound(rt.rebind(args, False))
+    rt.prepare_call(args).launch()
+    assert [entry for entry, _ in calls] == ["intent_w8a8_gemm"] * 3  # the best plan without runs
+
+
+def test_split_calls_do_not_share_scratch(monkeypatch):
+    # calls that may overlap (streams, threads): each launch has its own, on a known layout too
+    rt, args, size, calls = _split_call(monkeypatch)
+    held = []
+    launch = rt._launch
+    monkeypatch.setattr(rt, "_launch", lambda b: (held.append(b.workspace), launch(b)))
+    rt.run(*args)
+    rt.launch_bound(rt.rebind(args, False))
+    rt.launch_bound(rt.rebind(args, False))
+    assert len({t.data_ptr() for t in held}) == 3 and all(t.numel() == size for t in held)
