@@ -50,6 +50,10 @@ class KernelDefinition:
     # bytes of a launch's own scratch (never shared between launches that may overlap; 0: none).
     # The launch gets it in the place of the workspace, or None where it could not be allocated.
     scratch: Callable[[dict], int] | None = None
+    # (entry, what it covers, largest M or None) of a definition with several, and the one that a
+    # launch calls, from its extents and whether it has scratch.
+    entries: tuple = ()
+    entry: Callable[[dict, bool], str] | None = None
 
     @property
     def __name__(self) -> str:  # the reference uses definition.__name__ as the entry name
@@ -106,6 +110,12 @@ def _ld(t) -> int:
     return t.stride(0) if t.dim() >= 2 else t.shape[0]
 
 
+def _with_runs(base: str):
+    """Entry rule and entries of a contraction with a form that splits K."""
+    return (lambda env, scratch: base + "_ws" if scratch else base,
+            ((base, "without K runs", None), (base + "_ws", "K runs, partial sums through scratch", None)))
+
+
 # ---- W4A16 ------------------------------------------------------------------------
 
 def _w4_check(env: dict) -> None:
@@ -130,19 +140,24 @@ def _w4_scratch(env: dict) -> int:
     return _native.library().intent_w4a16_matmul_workspace_size(*size)
 
 
+def _w4_entry(env: dict, scratch: bool) -> str:
+    kernel = env["KERNEL"]
+    if scratch:
+        return "intent_w4a16_gemm_ws" if kernel == "gemm" else "intent_w4a16_matmul_ws"
+    if kernel == "auto":
+        kernel = "gemv" if env["M"] <= 16 else "gemm"
+    return "intent_w4a16_gemv" if kernel == "gemv" else "intent_w4a16_gemm"
+
+
 def _w4_launch(v: dict, env: dict, stream: int, scratch) -> str:
     x, q, s, z, y = v["activation"], v["packed_weight"], v["scales"], v["zeros"], v["output"]
     if s.stride(0) != z.stride(0):
         raise ValueError("scales and zeros must share a row stride")
-    kernel = env["KERNEL"]
+    entry = _w4_entry(env, scratch is not None)
     if scratch is not None:
-        entry = "intent_w4a16_gemm_ws" if kernel == "gemm" else "intent_w4a16_matmul_ws"
         _native.call(entry, _ptr(x), env["M"], env["K"], _ld(x), _ptr(q), env["N"], _ld(q), _ptr(s), _ptr(z), s.stride(0),
                      env["GROUP"], _ptr(y), _ld(y), _ptr(scratch), scratch.numel(), stream)
         return entry
-    if kernel == "auto":
-        kernel = "gemv" if env["M"] <= 16 else "gemm"
-    entry = {"gemv": "intent_w4a16_gemv", "gemm": "intent_w4a16_gemm"}[kernel]
     _native.call(entry, _ptr(x), env["M"], env["K"], _ld(x), _ptr(q), env["N"], _ld(q), _ptr(s), _ptr(z),
                  s.stride(0), env["GROUP"], _ptr(y), _ld(y), stream)
     return entry
@@ -159,6 +174,11 @@ weight_only_int4_asym_matmul = KernelDefinition(
     ),
     launch=_w4_launch,
     scratch=_w4_scratch,
+    entries=(("intent_w4a16_gemv", "GEMV, M <= 16", 16),
+             ("intent_w4a16_gemm", "tiled MFMA GEMM without K runs", None),
+             ("intent_w4a16_gemm_ws", "tiled MFMA GEMM with K runs through scratch (KERNEL = 'gemm')", None),
+             ("intent_w4a16_matmul_ws", "weight-streaming kernel or tiled GEMM with K runs, through scratch", None)),
+    entry=_w4_entry,
     constexprs={"KERNEL": "auto"},
     check=_w4_check,
     reference="examples/kernels/contraction/weight_only_int4.py:18-51",
@@ -172,15 +192,19 @@ def _w8a16_scratch(env: dict) -> int:
     return _native.library().intent_w8a16_matmul_workspace_size(env["M"], env["K"], env["N"])
 
 
+_w8a16_entry, _w8a16_entries = _with_runs("intent_w8a16_matmul")
+
+
 def _w8a16_launch(v: dict, env: dict, stream: int, scratch) -> str:
     x, w, s, y = v["activation"], v["weight"], v["scales"], v["output"]
+    entry = _w8a16_entry(env, scratch is not None)
     if scratch is not None:
-        _native.call("intent_w8a16_matmul_ws", _ptr(x), env["M"], env["K"], _ld(x), _ptr(w), env["N"], _ld(w), _ptr(s),
+        _native.call(entry, _ptr(x), env["M"], env["K"], _ld(x), _ptr(w), env["N"], _ld(w), _ptr(s),
                      _ptr(y), _ld(y), _ptr(scratch), scratch.numel(), stream)
     else:
-        _native.call("intent_w8a16_matmul", _ptr(x), env["M"], env["K"], _ld(x), _ptr(w), env["N"], _ld(w), _ptr(s),
+        _native.call(entry, _ptr(x), env["M"], env["K"], _ld(x), _ptr(w), env["N"], _ld(w), _ptr(s),
                      _ptr(y), _ld(y), stream)
-    return "intent_w8a16_matmul"
+    return entry
 
 
 weight_only_int8_matmul = KernelDefinition(
@@ -193,6 +217,8 @@ weight_only_int8_matmul = KernelDefinition(
     ),
     launch=_w8a16_launch,
     scratch=_w8a16_scratch,
+    entries=_w8a16_entries,
+    entry=_w8a16_entry,
     reference="doc/dsl/core.en.md:246 (I.cast(W_i8, f16) -> I.matmul(acc f32) -> scale)",
     doc="y = f16(scale[n] * (x @ w.T)), per-channel int8 weights",
 )
@@ -204,15 +230,19 @@ def _w8a8_scratch(env: dict) -> int:
     return _native.library().intent_w8a8_gemm_workspace_size(env["M"], env["K"], env["N"])
 
 
+_w8a8_entry, _w8a8_entries = _with_runs("intent_w8a8_gemm")
+
+
 def _w8a8_launch(v: dict, env: dict, stream: int, scratch) -> str:
     a, sa, w, sw, out = v["activation"], v["activation_scales"], v["weight"], v["weight_scales"], v["output"]
+    entry = _w8a8_entry(env, scratch is not None)
     if scratch is not None:
-        _native.call("intent_w8a8_gemm_ws", _ptr(a), env["M"], env["K"], _ld(a), _ptr(sa), _ptr(w), env["N"], _ld(w),
+        _native.call(entry, _ptr(a), env["M"], env["K"], _ld(a), _ptr(sa), _ptr(w), env["N"], _ld(w),
                      _ptr(sw), _ptr(out), _ld(out), _ptr(scratch), scratch.numel(), stream)
     else:
-        _native.call("intent_w8a8_gemm", _ptr(a), env["M"], env["K"], _ld(a), _ptr(sa), _ptr(w), env["N"], _ld(w),
+        _native.call(entry, _ptr(a), env["M"], env["K"], _ld(a), _ptr(sa), _ptr(w), env["N"], _ld(w),
                      _ptr(sw), _ptr(out), _ld(out), stream)
-    return "intent_w8a8_gemm"
+    return entry
 
 
 w8a8_scaled_matmul = KernelDefinition(
@@ -226,6 +256,8 @@ w8a8_scaled_matmul = KernelDefinition(
     ),
     launch=_w8a8_launch,
     scratch=_w8a8_scratch,
+    entries=_w8a8_entries,
+    entry=_w8a8_entry,
     reference="lib/Conversion/KIRToCPU/Contractions.cpp:30-35 + examples/kernels/contraction/gemm.py:83-106",
     doc="out = bf16(f32(int32 acc) * sa[m] * sw[n])",
 )
@@ -880,16 +912,20 @@ def _deepgemm_scratch(env: dict) -> int:
     return _native.library().intent_deepgemm_fp8_workspace_size(env["M"], env["KB"] * 128, env["N"])
 
 
+_deepgemm_entry, _deepgemm_entries = _with_runs("intent_deepgemm_fp8")
+
+
 def _deepgemm_launch(v: dict, env: dict, stream: int, scratch) -> str:
     lhs, rhs, ls, rs, out = v["lhs"], v["rhs"], v["lhs_scale"], v["rhs_scale"], v["output"]
     M, KB, N = env["M"], env["KB"], env["N"]
+    entry = _deepgemm_entry(env, scratch is not None)
     if scratch is not None:
-        _native.call("intent_deepgemm_fp8_ws", _ptr(lhs), M, KB * 128, KB * 128, _ptr(ls), KB, _ptr(rhs), N, KB * 128,
+        _native.call(entry, _ptr(lhs), M, KB * 128, KB * 128, _ptr(ls), KB, _ptr(rhs), N, KB * 128,
                      _ptr(rs), KB, _ptr(out), _ld(out), _ptr(scratch), scratch.numel(), stream)
     else:
-        _native.call("intent_deepgemm_fp8", _ptr(lhs), M, KB * 128, KB * 128, _ptr(ls), KB, _ptr(rhs), N, KB * 128,
+        _native.call(entry, _ptr(lhs), M, KB * 128, KB * 128, _ptr(ls), KB, _ptr(rhs), N, KB * 128,
                      _ptr(rs), KB, _ptr(out), _ld(out), stream)
-    return "intent_deepgemm_fp8"
+    return entry
 
 
 deepgemm_fp8_2xacc = KernelDefinition(
@@ -903,6 +939,8 @@ deepgemm_fp8_2xacc = KernelDefinition(
     ),
     launch=_deepgemm_launch,
     scratch=_deepgemm_scratch,
+    entries=_deepgemm_entries,
+    entry=_deepgemm_entry,
     check=_deepgemm_check,
     reference="examples/kernels/contraction/block_scaled.py:101-122",
     doc="output = bf16(sum over k-blocks of (lhs . rhs) * lhs_scale[m, kb] * rhs_scale[n // 128, kb])",

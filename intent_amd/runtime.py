@@ -408,14 +408,9 @@ class HIPPreparedCall:
 
     def inspect_configurations(self) -> tuple[ConfigurationAssessment, ...]:
         d = self._runtime.definition
+        if d.entry is None:
+            return (ConfigurationAssessment(d.name, True, "single fixed kernel"),)
         env = self._binding.env
-        if d.name == "weight_only_int4_asym_matmul":
-            m = env["M"]
-            choice = env["KERNEL"]
-            return (
-                ConfigurationAssessment("intent_w4a16_gemv", m <= 16 and choice in ("auto", "gemv"),
-                                        "decode GEMV covers M <= 16"),
-                ConfigurationAssessment("intent_w4a16_gemm", (m > 16 and choice == "auto") or choice == "gemm",
-                                        "MFMA tile GEMM for M > 16"),
-            )
-        return (ConfigurationAssessment(d.name, True, "single fixed kernel"),)
+        chosen = d.entry(env, self._binding.workspace is not None)
+        return tuple(ConfigurationAssessment(name, name == chosen and (limit is None or env["M"] <= limit), covers)
+                     for name, covers, limit in d.entries)

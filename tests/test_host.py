@@ -288,3 +288,38 @@ def test_split_calls_do_not_share_scratch(monkeypatch):
     rt.launch_bound(rt.rebind(args, False))
     rt.launch_bound(rt.rebind(args, False))
     assert len({t.data_ptr() for t in held}) == 3 and all(t.numel() == size for t in held)
+
+
+@pytest.mark.parametrize("M,K,N,kernel,entry", [
+    (1, 4096, 4096, "auto", "intent_w4a16_gemv"), (12, 4096, 11008, "auto", "intent_w4a16_matmul_ws"),
+    (12, 4096, 11008, "gemv", "intent_w4a16_gemv"), (77, 4096, 4096, "auto", "intent_w4a16_matmul_ws"),
+    (77, 4096, 4096, "gemm", "intent_w4a16_gemm_ws"), (2048, 4096, 11008, "auto", "intent_w4a16_gemm"),
+    (2048, 4096, 11008, "gemm", "intent_w4a16_gemm"), (20, 4096, 128, "gemv", None)])
+def test_configurations_name_the_entry_that_runs(monkeypatch, M, K, N, kernel, entry):
+    from intent_amd import _native
+    from intent_amd import runtime as runtime_module
+
+    rt = runtime_for(intent.weight_only_int4_asym_matmul, KERNEL=kernel)
+    rt._home = torch.device("cpu")
+    calls = []
+    monkeypatch.setattr(_native, "call", lambda name, *a: calls.append(name))
+    monkeypatch.setattr(runtime_module, "_current_stream", lambda device: 0)
+    call = rt.prepare_call((torch.empty(M, K, dtype=torch.float16), torch.empty(N, K // 2, dtype=torch.uint8),
+                            torch.empty(N, K // 128, dtype=torch.float16), torch.empty(N, K // 128, dtype=torch.uint8)))
+    eligible = [c.entry for c in call.inspect_configurations() if c.eligible]
+    if entry is None:  # the GEMV covers M <= 16: nothing takes the call, and the library refuses it
+        assert not eligible
+        return
+    call.launch()
+    assert eligible == calls == [call.observation.entry] == [entry]
+
+
+def test_split_entries_are_named(monkeypatch):
+    rt, args, size, calls = _split_call(monkeypatch)
+    call = rt.prepare_call(args)
+    call.launch()
+    assert [c.entry for c in call.inspect_configurations() if c.eligible] == ["intent_w8a8_gemm_ws"]
+    assert call.observation.entry == calls[0][0] == "intent_w8a8_gemm_ws"
+    rt.run(torch.zeros(4096, 256, dtype=torch.int8), torch.zeros(4096), torch.zeros(8192, 256, dtype=torch.int8),
+           torch.zeros(8192))
+    assert rt.observation.entry == calls[1][0] == "intent_w8a8_gemm"  # no K runs
