@@ -21,8 +21,19 @@ and, in every kernel that contains an LDS DMA,
   (buffer resource or offset).
 
 The wait states are the gfx9 hazard table's (an instruction counts one,
-``s_nop N`` counts N + 1). The input is a code object built here from this
-repository's own sources.
+``s_nop N`` counts N + 1).
+
+In every kernel with MFMAs it also rejects an MFMA whose A, B or scale operand
+was written while lanes were masked off. MFMAs ignore EXEC and read their
+operands from all 64 lanes, but the reads and decodes that produce those operands
+obey it. The compiler may move an MFMA with no other use below a per-lane branch
+(the rows past M of an epilogue), which is harmless by itself and does happen; it
+would be wrong if the operand's own instruction moved with it, since the masked
+lanes would then leave their part of the operand stale. Nothing in the source
+rules that out everywhere, so the built code is checked, but for
+``WAVE_UNIFORM_KERNELS``.
+
+The input is a code object built here from this repository's own sources.
 """
 from __future__ import annotations
 
@@ -38,9 +49,15 @@ TARGET = "hipv4-amdgcn-amd-amdhsa--gfx950"
 # does not see it). Substrings of the mangled names.
 UNTRACKED_DMA_KERNELS = ("moe_gate_up_pk_kernel", "moe_down_pk_kernel")
 
+# Kernels whose K loop the compiler takes for divergent (its bounds come from threadIdx.x >> 6), though
+# every lane of a wave agrees: the loads and MFMAs of a step are masked as a whole or not at all.
+# Substrings of the mangled names.
+WAVE_UNIFORM_KERNELS = ("_117w4a16_gemv_kernel", "_117w8a16_gemv_kernel")
+
 M0_WAIT = 1
 VALU_SGPR_WAIT = 5
 
+_TARGET = re.compile(r"<[^>+]+(?:\+0x([0-9a-f]+))?>")
 _LABEL = re.compile(r"^[0-9a-f]+ <(?P<name>[^>]+)>:\s*$")
 _DMA = re.compile(r"^buffer_load_(dword|dwordx4|ubyte|ushort|sbyte|sshort)\b.*\blds\b")
 _SREG = re.compile(r"\bs\[(\d+):(\d+)\]|\bs(\d+)\b|\b(vcc)\b|\b(m0)\b")
@@ -191,6 +208,128 @@ def _check_kernel(name: str, insts: list, meta: dict) -> KernelReport:
     return rep
 
 
+_BRANCH = ("s_cbranch", "s_branch", "s_endpgm", "s_setpc")
+_VREG = re.compile(r"^([va])(?:(\d+)|\[(\d+):(\d+)\])$")
+# Vector instructions whose first operand is not a destination.
+_NO_DEST = re.compile(r"^(ds_write|ds_store|global_store|buffer_store|flat_store|scratch_store|global_atomic|"
+                      r"buffer_atomic|ds_add|v_cmp|v_readfirstlane|v_readlane|v_nop)")
+
+
+def _vregs(operand: str) -> set:
+    m = _VREG.match(operand)
+    if not m:
+        return set()
+    lo, hi = (m.group(2), m.group(2)) if m.group(2) else (m.group(3), m.group(4))
+    return {m.group(1) + str(i) for i in range(int(lo), int(hi) + 1)}
+
+
+class _Masked:
+    """Lanes masked off on some path to a point: the SGPR pairs that hold the EXEC to restore, each
+    with those outstanding when it was saved, and the vector registers written since."""
+
+    def __init__(self, saved=None, written=()):
+        self.saved = dict(saved or {})
+        self.written = set(written)
+
+    def merge(self, other) -> bool:
+        before = ({k: set(v) for k, v in self.saved.items()}, len(self.written))
+        for reg, outer in other.saved.items():
+            self.saved[reg] = self.saved.get(reg, frozenset()) | outer
+        self.written |= other.written
+        return before != ({k: set(v) for k, v in self.saved.items()}, len(self.written))
+
+    def _restore(self, reg: str) -> None:
+        if reg not in self.saved:
+            return
+        for inner in [k for k, outer in self.saved.items() if k == reg or reg in outer]:
+            del self.saved[inner]
+
+    def _save(self, reg: str) -> None:
+        self._restore(reg)
+        self.saved[reg] = frozenset(self.saved)
+
+    def step(self, inst: str):
+        """Applies one instruction; the operands an MFMA reads that were written under a mask."""
+        op, _, rest = inst.partition(" ")
+        if op.startswith("s_") and "exec" in inst:
+            ops = _operands(inst)
+            if "saveexec" in op:
+                if not op.startswith("s_and_saveexec"):  # the other side of a branch: EXEC is whole between
+                    self._restore(ops[1])
+                self._save(ops[0])
+            elif op == "s_xor_b64" and ops[1] == "exec" and ops[0] != "exec" and ops[2] in self.saved:
+                self.saved[ops[0]] = self.saved.pop(ops[2])  # the lanes of the other side, kept for its saveexec
+            elif ops[0] == "exec" and op in ("s_or_b64", "s_mov_b64"):
+                for reg in ops[1:]:
+                    self._restore(reg)
+                self._restore("exec")
+            elif ops[0] == "exec" and op == "s_andn2_b64":  # lanes that left a loop
+                self.saved.setdefault(ops[2], frozenset(self.saved))
+            elif ops[0] == "exec" and op == "s_and_b64" and not self.saved:
+                self._save("exec")
+            if not self.saved:
+                self.written.clear()
+            return set()
+        if not self.saved or not op.startswith(("v_", "ds_", "global_", "buffer_", "flat_", "scratch_")):
+            return set()
+        ops = _operands(inst)
+        if op.startswith("v_mfma"):
+            reads = set()
+            for o in ops[1:3] + ops[4:]:
+                reads |= _vregs(o.split(" ")[0])
+            stale = reads & self.written
+            self.written -= _vregs(ops[0])  # written in every lane
+            return stale
+        if ops and not _NO_DEST.match(op) and " lds" not in inst:
+            self.written |= _vregs(ops[0])
+        return set()
+
+
+def masked_mfma_operands(insts: list) -> list:
+    """The MFMAs of a kernel, (address, text, branch target address or None) per instruction, that
+    read an A, B or scale operand written while lanes were masked off."""
+    if not any(text.startswith("v_mfma") for _, text, _ in insts):
+        return []
+    index = {addr: i for i, (addr, _, _) in enumerate(insts)}
+    starts = {0}
+    for i, (_, text, target) in enumerate(insts):
+        if text.startswith(_BRANCH):
+            starts.add(i + 1)
+            if target in index:
+                starts.add(index[target])
+    order = sorted(x for x in starts if x < len(insts))
+    ends = dict(zip(order, order[1:] + [len(insts)]))
+    state = {0: _Masked()}
+    work = [0]
+    while work:
+        first = work.pop()
+        cur = _Masked(state[first].saved, state[first].written)
+        for i in range(first, ends[first]):
+            cur.step(insts[i][1])
+        _, last, target = insts[ends[first] - 1]
+        following = []
+        if not last.startswith(("s_branch", "s_endpgm", "s_setpc")) and ends[first] < len(insts):
+            following.append(ends[first])
+        if last.startswith(("s_branch", "s_cbranch")) and target in index:
+            following.append(index[target])
+        for nxt in following:
+            if nxt not in state:
+                state[nxt] = _Masked(cur.saved, cur.written)
+                work.append(nxt)
+            elif state[nxt].merge(cur):
+                work.append(nxt)
+    problems = []
+    for first in order:
+        if first not in state:
+            continue  # padding
+        cur = _Masked(state[first].saved, state[first].written)
+        for i in range(first, ends[first]):
+            stale = cur.step(insts[i][1])
+            if stale:
+                problems.append(f"operand {sorted(stale)} was written with lanes masked off: {insts[i][1]!r}")
+    return problems
+
+
 def _metadata(code_object: Path) -> dict:
     notes = _run([_tool("llvm-readelf"), "--notes", str(code_object)])
     meta, cur = {}, None
@@ -208,30 +347,36 @@ def _metadata(code_object: Path) -> dict:
 
 def check_code_object(code_object: Path) -> list:
     """Reports for every kernel of a gfx950 code object; raises CodeObjectError
-    listing every kernel with an LDS DMA that breaks a rule above."""
+    listing every kernel that breaks a rule above."""
     meta = _metadata(code_object)
     dis = _run([_tool("llvm-objdump"), "-d", "--no-show-raw-insn", str(code_object)])
-    kernels, name, insts = [], None, []
+    kernels, name, insts, base = [], None, [], 0
     for line in dis.splitlines():
         m = _LABEL.match(line)
         if m:
             if name is not None:
                 kernels.append((name, insts))
-            name, insts = m.group("name"), []
+            name, insts, base = m.group("name"), [], int(line.split(" ", 1)[0], 16)
             continue
-        s = line.split("//")[0].strip()
+        s, _, comment = (part.strip() for part in line.partition("//"))
         if name is not None and s:
-            insts.append(s)
+            addr = int(comment.split(":")[0], 16) if ":" in comment else -1
+            to = _TARGET.search(comment)
+            insts.append((addr, s, base + int(to.group(1) or "0", 16) if to else None))
     if name is not None:
         kernels.append((name, insts))
-    reports = [_check_kernel(n, ins, meta.get(n, {})) for n, ins in kernels]
+    reports = []
+    for n, ins in kernels:
+        reports.append(_check_kernel(n, [text for _, text, _ in ins], meta.get(n, {})))
+        if not any(k in n for k in WAVE_UNIFORM_KERNELS):
+            reports[-1].problems.extend(masked_mfma_operands(ins))
     bad = [r for r in reports if r.problems]
     if bad:
         lines = []
         for r in bad:
             lines.append(f"{r.name}:")
             lines.extend(f"  {p}" for p in r.problems[:8])
-        raise CodeObjectError("kernels with LDS DMA break their scratch/hazard rules:\n" + "\n".join(lines))
+        raise CodeObjectError("kernels break their scratch, hazard or mask rules:\n" + "\n".join(lines))
     return reports
 
 

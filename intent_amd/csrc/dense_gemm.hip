@@ -820,7 +820,7 @@ __global__ __launch_bounds__(T::NT_WS, 1) void dense_split_kernel(const f16* __r
   float* out = part + (((int64_t)p * gridDim.x + blockIdx.x) * T::NW + T::wave()) * (BLK * 256) + (threadIdx.x & 63) * 4;
 #pragma unroll
   for (int i = 0; i < T::TI; ++i) {
-    if (m0 + T::wave_m() * T::WTM + i * 32 >= M) continue;  // wave-uniform: a per-lane test lets the last MFMAs' operand reads sink under it
+    if (m0 + T::wave_m() * T::WTM + i * 32 >= M) continue;  // by whole blocks: no branch per lane (mp::settle)
 #pragma unroll
     for (int j = 0; j < T::TJ; ++j)
 #pragma unroll

@@ -122,6 +122,22 @@ INTENT_DEVICE void wait_vm_lgkm_barrier() {
   __builtin_amdgcn_s_barrier();
 }
 
+// Before an epilogue that branches per lane right after a main loop (rows past M):
+// the sums are complete here, under the whole wave. The compiler moves MFMAs whose
+// result only one side of a branch needs into it, and the instructions that make
+// their operands may follow. MFMAs ignore EXEC but those do not, and a fragment read
+// or shifted in only some lanes is wrong for all rows of the block. With one 32-row
+// block per wave (64-row tiles) nothing else uses an operand of either side, so
+// either can move; intent_amd/codeobj_check.py rejects a build where one has.
+// Accumulators in AGPRs only (four-wave tiles), where this costs no copy.
+template <class V, int TI, int TJ>
+INTENT_DEVICE void settle(V (&acc)[TI][TJ]) {
+#pragma unroll
+  for (int i = 0; i < TI; ++i)
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) asm volatile("" : "+a"(acc[i][j]));
+}
+
 // ds_write_b128 that the compiler does not see as an LDS access. Producer
 // waves write decoded weights into a stage buffer while LDS DMAs into other
 // buffers are in flight; a visible LDS store there would make the compiler's

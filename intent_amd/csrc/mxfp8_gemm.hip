@@ -204,6 +204,7 @@ __global__ __launch_bounds__(T::NT, 1) void mxfp8_gemm_kernel(const uint8_t* __r
   }
   compute_stage_mx<T>((kt & 1) ? buf1 : buf0, acc);
 
+  mp::settle(acc);
   store_mx<T>(acc, m0, n0, M, N, out, ldo);
 }
 
@@ -1061,7 +1062,7 @@ __global__ __launch_bounds__(256, 2) void deepgemm_fp8_kernel(
                   (threadIdx.x & 63) * 4;
 #pragma unroll
     for (int i = 0; i < T::TI; ++i) {
-      if (m0 + T::wave_m() * T::WTM + i * 32 >= M) continue;  // wave-uniform: a per-lane test lets the last MFMAs' operand reads sink under it
+      if (m0 + T::wave_m() * T::WTM + i * 32 >= M) continue;  // by whole blocks: no branch per lane (mp::settle)
 #pragma unroll
       for (int j = 0; j < T::TJ; ++j)
 #pragma unroll

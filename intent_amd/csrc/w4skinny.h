@@ -301,9 +301,9 @@ INTENT_DEVICE void w4_mainloop(char* lds, const void* x, const TRow& trow, const
 #pragma unroll
   for (int d = 0; d + 1 < D; ++d)
     if (whole + d < nst) stage(whole + d, xr[d], wr[d], false);
-  // The sums are complete here, under the whole wave: without this the compiler
-  // may move a last stage's fragment reads below a caller's per-lane branch,
-  // where masked lanes would not load their part of an MFMA operand.
+  // The sums are complete here, under the whole wave: a caller's branch per lane
+  // must not take a last stage's fragment reads with it (mp::settle; the sums are
+  // in VGPRs here).
 #pragma unroll
   for (int b = 0; b < NB; ++b)
 #pragma unroll

@@ -165,6 +165,7 @@ __global__ __launch_bounds__(T::NT, 1) void i8_gemm_kernel(const int8_t* __restr
     store_bf16_lds<T>(acc, buf0, scales, m0, n0, M, N, reinterpret_cast<uint16_t*>(out), ldo);
     return;
   }
+  if constexpr (T::NW == 4) mp::settle(acc);
   store_tile<T, E>(acc, m0, n0, M, N, a_scales, w_scales, bias, out, ldo);
 }
 
@@ -356,7 +357,7 @@ __global__ __launch_bounds__(T::NT, 1) void i8_split_kernel(const int8_t* __rest
   int32_t* out = part + (((int64_t)p * gridDim.x + blockIdx.x) * T::NW + T::wave()) * (BLK * 256) + (threadIdx.x & 63) * 4;
 #pragma unroll
   for (int i = 0; i < T::TI; ++i) {
-    if (m0 + T::wave_m() * T::WTM + i * 32 >= M) continue;  // wave-uniform: a per-lane test lets the last MFMAs' operand reads sink under it
+    if (m0 + T::wave_m() * T::WTM + i * 32 >= M) continue;  // by whole blocks: no branch per lane (mp::settle)
 #pragma unroll
     for (int j = 0; j < T::TJ; ++j)
 #pragma unroll
