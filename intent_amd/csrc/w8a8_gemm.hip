@@ -165,7 +165,7 @@ __global__ __launch_bounds__(T::NT, 1) void i8_gemm_kernel(const int8_t* __restr
     store_bf16_lds<T>(acc, buf0, scales, m0, n0, M, N, reinterpret_cast<uint16_t*>(out), ldo);
     return;
   }
-  if constexpr (T::NW == 4) mp::settle(acc);
+  if constexpr (T::TI == 1) mp::settle(acc);  // 128 x 128: 0.25 us more, the scales are loaded over the last MFMAs
   store_tile<T, E>(acc, m0, n0, M, N, a_scales, w_scales, bias, out, ldo);
 }
 
@@ -495,8 +495,10 @@ I8Plan i8_plan(int64_t M, int64_t N, int64_t K, bool may_split) {
   }
   // Up to 32 rows a wave of the 128-row tile stores one 32-row block, as one of the
   // 64-row tile does, and its main loop is the faster (int32 output, N = 2432, K =
-  // 6272, M = 32: 30.5 us against 32.0; at M = 33, two blocks, 34.0 against 32.1).
-  if (best.tile == 64 && best.splits == 1 && M <= 32) best.tile = 128;
+  // 6272, M = 32: 30.5 us against 32.0; at M = 33, two blocks, 34.0 against 32.1). It
+  // starts the slower: the lines cross at 16 stages (K = 2048 15.7 against 16.1 us,
+  // 1536 both 13.9, 512 10.1 against 9.9).
+  if (best.tile == 64 && best.splits == 1 && M <= 32 && stages >= 16) best.tile = 128;
   return best;
 }
 

@@ -530,7 +530,7 @@ def test_w8a8_split_k(gpu, threads, M, K, N, pad):
 # Every tile with and without a K split (the kernel's name carries tile and runs), each with K in whole 128-k
 # stages and with a last stage of 64 k, rows off the tiles and off their 32-row blocks, columns off the tiles.
 @pytest.mark.parametrize("M,K,N,kernel", [
-    (32, 384, 204, "128x128"), (33, 384, 204, "64x128"), (45, 320, 205, "64x128"), (69, 256, 3226, "128x128"), (65, 320, 3226, "128x128"),
+    (32, 384, 204, "64x128"), (32, 2048, 8200, "128x128"), (33, 384, 204, "64x128"), (45, 320, 205, "64x128"), (69, 256, 3226, "128x128"), (65, 320, 3226, "128x128"),
     (69, 1408, 70, "128x128, 8 runs"), (67, 1344, 65, "128x128, 8 runs"),
     (131, 22400, 5444, "256x256, 8 runs"), (198, 13504, 8663, "256x256, 4 runs")])
 def test_w8a8_tiles(gpu, threads, M, K, N, kernel):
@@ -543,9 +543,10 @@ def test_w8a8_tiles(gpu, threads, M, K, N, kernel):
     assert np.array_equal(y.view(torch.int16).cpu().numpy().view(np.uint16)[:, cols], ref)
 
 
-# The same kernels with int32 output, which has no K split: 128-row tiles up to 32 rows, 64-row ones above.
-@pytest.mark.parametrize("M,K,N,kernel", [(1, 2048, 300, "128x128"), (32, 1088, 205, "128x128"), (33, 2048, 300, "64x128"),
-                                          (45, 1088, 205, "64x128"), (69, 320, 3226, "128x128")])
+# The same kernels with int32 output, which has no K split: 128-row tiles up to 32 rows from 16 stages of 128 k on,
+# 64-row ones for less and above.
+@pytest.mark.parametrize("M,K,N,kernel", [(1, 2048, 300, "128x128"), (32, 1984, 205, "128x128"), (32, 1920, 205, "64x128"),
+                                          (33, 2048, 300, "64x128"), (45, 1088, 205, "64x128"), (69, 320, 3226, "128x128")])
 def test_i8_gemm_i32_tiles(gpu, threads, M, K, N, kernel):
     rng = np.random.default_rng(M + N)
     x, w = rng.integers(-127, 128, size=(M, K), dtype=np.int8), rng.integers(-127, 128, size=(N, K), dtype=np.int8)
