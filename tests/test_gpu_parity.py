@@ -453,6 +453,35 @@ def test_w4a16_skinny(gpu, threads, M, K, N, group, pad):
     assert_close_rms(host(y)[:, cols], ref, what=f"w4a16 skinny {M}x{K}x{N} g{group}")
 
 
+# The same kernel over the other forms it accepts: weight and parameter rows wider than the row and starting inside
+# a larger buffer (parameter rows then off the vector loads, or on them), zero points over the whole byte, an
+# activation row of zeros.
+@pytest.mark.parametrize("M,K,N,group", [(12, 8192, 8200, 128), (77, 4096, 640, 128), (40, 4096, 333, 32), (100, 2048, 200, 64)])
+@pytest.mark.parametrize("lead,extra", [(0, 4), (4, 8), (1, 6), (3, 5)])
+def test_w4a16_skinny_strided_parameters(gpu, threads, M, K, N, group, lead, extra):
+    d = inputs.config1_w4a16_decode(M + N, M=M, K=K, N=N, group=group)
+    rng = np.random.default_rng(N)
+    d["zeros"] = rng.integers(0, 256, d["zeros"].shape, dtype=np.uint8)
+    d["x"][0] = 0
+    G = K // group
+
+    def inside(a, before, after):
+        wide = torch.full((a.shape[0], before + a.shape[1] + after), 0x7F, dtype=torch.uint8).to(dev(a).dtype).cuda()
+        wide[:, before:before + a.shape[1]] = dev(a)
+        return wide[:, before:before + a.shape[1]]
+
+    args = (inside(d["x"], 8, 8), inside(d["packed"], 16, 16), inside(d["scales"], lead, extra), inside(d["zeros"], lead, extra))
+    assert args[2].stride(0) == G + lead + extra
+    a = art(intent.weight_only_int4_asym_matmul)
+    y = a.run(*args)
+    assert a.observation.kernel == "w4a16_skinny", a.observation.kernel
+    cols = np.r_[0:min(N, 300), max(0, N - 70):N]
+    ref = oracle.w4a16(d["x"], d["packed"][cols], d["scales"][cols], d["zeros"][cols], threads)
+    got = host(y)[:, cols]
+    assert not got[0].any()
+    assert_close_rms(got, ref, what=f"w4a16 skinny strided {M}x{K}x{N} g{group}")
+
+
 # KERNEL = "gemm" forces the tiled kernels, also at the rows where the weight-streaming one is the faster: every
 # tile whose K is split (the kernel's name carries tile and runs) with windowed and with per-stage group parameters,
 # rows and columns off the tiles.
