@@ -144,14 +144,24 @@ Plan skinny_plan(int64_t M, int64_t N, int64_t K, int64_t gs) {
 
 namespace intent {
 
-// Microseconds the kernel takes, fitted to 60 shapes (M 2..128, N 1024..14336, K
-// 2048..14336) within about 10%; 0 where it does not take the call. bytes: its scratch.
+// Microseconds of a fit to 60 shapes (M 2..128, N 1024..14336, K 2048..14336); over
+// 121 other ones (N 310..131072, K 256..16384) that it takes, four in five of the
+// fits are 0.80 to 1.02 of the measured time. 0 where the kernel does not take the
+// call. bytes: its scratch.
 double w4a16_skinny_us(int64_t M, int64_t N, int64_t K, int64_t gs, size_t* bytes) {
   const Plan p = skinny_plan(M, N, K, gs);
   if (p.unit == 0) return 0;
   *bytes = (size_t)partial_bytes(p, N);
   const double work = (double)((N + kRows - 1) / kRows) * (double)(K / 128) / 8;
-  return 5.2 + 0.6 * p.tb + work * (0.0046 + 0.0034 * p.tb);
+  // Runs that are not whole quads of groups load the parameters one by one: 1 to 2.5 us
+  // more. Up to 6 rows that decides against one round of the GEMV for K below 10240 (N =
+  // 2304, M = 6: K = 8320 10.6 us against 9.6, 9344 11.1 against 10.5, 10368 11.5 against
+  // 11.4), at 7 rows below 9216 (N = 3072, K = 9344 10.8 against 11.3); not at M = 8 (K =
+  // 8320 10.7 against 10.6), nor while one workgroup per CU does (M = 6, N = 2048 8.5
+  // against 9.6).
+  const bool gemv_round = N > 2048 && N <= 4096 && (M <= 6 ? K < 10240 : M == 7 && K < 9216);
+  const double singles = gemv_round && p.unit % (4 * gs) != 0 ? 3 : 0;
+  return 5.2 + 0.6 * p.tb + work * (0.0046 + 0.0034 * p.tb) + singles;
 }
 
 // A w4a16_fast call whose plan exists, with 31-bit offsets checked by the caller.

@@ -125,6 +125,18 @@ def test_moe_expert_ffn_workspace_holds_what_the_plan_uses():
     assert exact(4, 8, 64, 64, 0) == 0 and exact(-1, 8, 64, 64, 2) == 0
 
 
+def test_w4a16_streaming_kernel_against_the_gemv():
+    # Up to 7 rows and parameter rows off whole quads of groups the GEMV is the faster for K just above 8192.
+    size = _native.library().intent_w4a16_matmul_workspace_size
+    for M in (3, 4, 6):
+        for K, N in ((8320, 2304), (8320, 4096), (9344, 2304), (9344, 4096)):
+            assert size(M, K, N, 128) == 0, (M, K, N)
+    assert size(7, 8320, 2304, 128) == 0
+    for M, K, N in ((7, 9344, 3072), (8, 8320, 2304), (12, 8320, 2304), (6, 8320, 2048), (6, 10240, 2304), (6, 10368, 4096),
+                    (6, 14208, 2304), (3, 8192, 8200)):
+        assert size(M, K, N, 128) > 0, (M, K, N)
+
+
 def test_w4a16_wide_outputs_scratch():
     # Very wide outputs (a vocabulary head): the streaming kernel is weighed against the tiles there too, and
     # whatever takes the call keeps its partial sums within 64 MB.
