@@ -39,10 +39,16 @@ int fill_launch(void* out, int64_t rows, int64_t cols, int64_t ld, int elem_byte
 // query fails, which callers treat as "no round-fitting").
 int cu_count();
 
-// Time of a tiled kernel in microseconds, from measurements of it: base, plus
-// per stage of the K loop a + b L while the L = workgroups / 256 do not exceed
-// one per CU, and (a + b) times the rounds beyond (half a round's cost for a
-// partly filled one, since its workgroups share a CU with those before them).
+// By this the plans of one tiled kernel are ranked, in microseconds of a fit to
+// measurements of it: base, plus per stage of the K loop a + b L while the L =
+// workgroups / 256 do not exceed one per CU, and (a + b) times the rounds beyond
+// (half a round's cost for a partly filled one, since its workgroups share a CU with
+// those before them). It predicts no time: bandwidth, stores and how far workgroups
+// that share a CU hide each other are left out. Over 700 random shapes (M 1..4096, K
+// 256..16384, N 256..131072) the chosen plan reads 0.76 to 0.99 of its measured time
+// in the median up to one workgroup per CU and 0.68 to 0.98 up to four, 0.3 where K is
+// short and N very wide, and 47 us for the 35 of block-scaled FP8 at M = 300, N =
+// 14336, K = 4096 (two workgroups on some CUs).
 struct GridCost {
   double base, a, b;
   double us(int64_t workgroups, double stages) const {

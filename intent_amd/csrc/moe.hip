@@ -680,8 +680,8 @@ __global__ __launch_bounds__(GateUpPk::NT, 2) void moe_down_pk_kernel(
 // by the stream of expert weights. The 128-row packed core copies 128 token
 // rows per stage whatever the block holds, twice the bytes of the weights, in
 // 32-byte pieces. E = 8, top-2, H = 4096, F = 14336, whole layer on one box:
-// T = 1 110 -> 63 us, 16 270 -> 165 us (gate/up 165 -> 100, 4.9 TB/s; down
-// 98 -> 57), 40 280 -> 182, 100 290 -> 223, 160 315 -> 262 us. At 16 rows two
+// T = 1 110 -> 59 us, 16 279 -> 160 us (gate/up 91, 5.4 TB/s; down 53, 4.6
+// TB/s), 40 282 -> 178, 100 293 -> 221, 160 313 -> 240 us. At 16 rows two
 // blocks per wave beat four (186 vs 204 us: 1.2 rounds of workgroups against
 // 2.3); non-temporal weight loads took 205 us.
 template <int TB>

@@ -242,8 +242,8 @@ constexpr int64_t kFewRows = 4096;  // routes up to which they are taken: bounds
 // keeps 32 KB of them in flight and copies 256 rows for a handful of routes
 // (and the second projection has D / 256 tiles per expert: 128 workgroups at
 // E = 8, D = 4096). 64-row tiles run two or three workgroups per CU; columns and K
-// runs are chosen for about 512 workgroups. E = 8, D = 4096, F = 14336, whole layer:
-// T = 1 348 -> 152 us, 16 498 -> 320, 200 531 -> 346 (5.5 TB/s), 400 553 -> 412 us.
+// runs are chosen for about 512 workgroups. E = 8, top-2, D = 4096, F = 14336, whole
+// layer: T = 1 346 -> 122 us, 16 507 -> 323, 200 525 -> 345 (5.4 TB/s), 400 546 -> 396 us.
 // The lines: 50 routes per expert 346 us (64 rows) against 373 (128), 64 383 (128);
 // 100 412 (128) against 553 (256), 125 (E = 32) 522 against 520, 150 622 against 579.
 struct FfnPlan {

@@ -160,8 +160,13 @@ double w4a16_skinny_us(int64_t M, int64_t N, int64_t K, int64_t gs, size_t* byte
   // 8320 10.7 against 10.6), nor while one workgroup per CU does (M = 6, N = 2048 8.5
   // against 9.6).
   const bool gemv_round = N > 2048 && N <= 4096 && (M <= 6 ? K < 10240 : M == 7 && K < 9216);
-  const double singles = gemv_round && p.unit % (4 * gs) != 0 ? 3 : 0;
-  return 5.2 + 0.6 * p.tb + work * (0.0046 + 0.0034 * p.tb) + singles;
+  const bool quads = p.unit % (4 * gs) == 0 || (p.splits == 1 && K % (4 * gs) == 0);
+  const double singles = gemv_round && !quads ? 3 : 0;
+  // The partial sums' way through memory, which the fit has in its terms of K from 1024
+  // on (N = 106112, K = 256, M = 26 18.3 us against 14.6 in tiles; N = 22848, K = 768, M =
+  // 17 10.8 against 9.5; the other way round at N = 8192, K = 512: 6.6 against 6.9).
+  const double sums = M > 16 && K < 1024 && (N > 16384 || !quads) ? 0.27e-6 * (double)partial_bytes(p, N) : 0;
+  return 5.2 + 0.6 * p.tb + work * (0.0046 + 0.0034 * p.tb) + singles + sums;
 }
 
 // A w4a16_fast call whose plan exists, with 31-bit offsets checked by the caller.
