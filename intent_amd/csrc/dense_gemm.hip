@@ -967,9 +967,12 @@ W4Cut w4_cut(int64_t K, int64_t gs) {
   const bool win = gs % 64 == 0 && K % (4 * gs) == 0;
   return {win ? 4 * gs : gs % 64 == 0 ? gs : 64, win};
 }
+bool w4_brief(int64_t M, int64_t K) { return M > 80 && M <= 128 && K < 1024; }
 DensePlan w4_plan(int64_t M, int64_t N, int64_t K, int64_t gs, bool may_split, double* us = nullptr) {
   const W4Cut c = w4_cut(K, gs);
-  return dense_plan(M, N, K, c.unit, may_split, c.win ? 1.0 : 1.1, us);
+  // Under 16 stages of a well filled 128-row tile, runs do not pay for their sums
+  // (N = 2048, M = 128: K = 768 8.9 us without, 10.1 with four; 896 9.7 and 10.2).
+  return dense_plan(M, N, K, c.unit, may_split && !w4_brief(M, K), c.win ? 1.0 : 1.1, us);
 }
 DensePlan w8_plan(int64_t M, int64_t N, int64_t K, bool may_split) { return dense_plan(M, N, K, 64, may_split, 1.0); }
 
@@ -1055,7 +1058,8 @@ int w4a16_skinny_launch(const void* x, int64_t M, int64_t K, int64_t x_ld, const
 // 4096 17 us, N = 14336, K = 2048 13.5, N = K = 8192 20, N = 4096, K = 14336 19..23);
 // where the dot-product GEMV (no weight rounded to f16) takes the call, it stays.
 // Very wide outputs are weighed the same way (N = 128256, K = 4096: M = 48 117 us
-// here against 145 in 128-row tiles, M = 77 188 against 143, 128 310 against 151).
+// here against 145 in 128-row tiles, M = 77 188 against 143, 128 310 against 151). So
+// are short K (N = 2048, K = 768, M = 100: 11.3 here, 8.9 in 128-row tiles).
 size_t w4a16_wants_skinny(int64_t M, int64_t N, int64_t K, int64_t gs) {
   if (M < 2 || (M == 2 && K <= 8192) || (M <= 5 && K <= 4096)) return 0;
   size_t bytes = 0;
@@ -1064,7 +1068,7 @@ size_t w4a16_wants_skinny(int64_t M, int64_t N, int64_t K, int64_t gs) {
   if (M > 16) {
     double tiled;  // the estimate is up to 0.8 of the measured time for 4 runs or more, up to 1.1 of it for fewer
     const DensePlan p = w4_plan(M, N, K, gs, true, &tiled);
-    return us < (p.splits > 2 ? 1.2 : 0.9) * tiled ? bytes : 0;
+    return us < (p.splits > 2 ? 1.2 : w4_brief(M, K) ? 0.8 : 0.9) * tiled ? bytes : 0;
   }
   const double rounds = (double)((N + 4095) / 4096);
   return us < 0.9 * (1.2 + rounds * (1.6 + 1e-3 * (double)K)) ? bytes : 0;

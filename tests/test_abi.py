@@ -140,7 +140,7 @@ def test_w4a16_streaming_kernel_against_the_gemv():
 def test_w4a16_streaming_kernel_at_short_k():
     # Below K = 1024 its partial sums weigh as much as the weights: wide outputs go to the tiles without runs.
     size = _native.library().intent_w4a16_matmul_workspace_size
-    for M, K, N, group in ((26, 256, 106112, 128), (17, 640, 38400, 64), (17, 768, 22848, 128), (64, 896, 106112, 64)):
+    for M, K, N, group in ((100, 768, 2048, 128), (128, 896, 1024, 64), (26, 256, 106112, 128), (17, 640, 38400, 64), (17, 768, 22848, 128), (64, 896, 106112, 64)):
         assert size(M, K, N, group) == 0, (M, K, N)
     for M, K, N, group in ((17, 512, 8192, 128), (40, 768, 12288, 64), (17, 1024, 22848, 128)):
         assert size(M, K, N, group) > 0, (M, K, N)
