@@ -916,7 +916,6 @@ struct DensePlan {
 constexpr int64_t kMaxSplitBytes = 64 << 20;
 constexpr intent::PlanNames kW4Names = INTENT_PLAN_NAMES("w4a16_gemm", "256x192");
 constexpr intent::PlanNames kW8Names = INTENT_PLAN_NAMES("w8a16_matmul", "256x192");
-constexpr intent::PlanNames kW4SymNames = INTENT_PLAN_NAMES("w4a16_sym_gemm", "256x192");
 
 int64_t dense_tiles(int64_t M, int64_t N, int tile) {
   const int64_t bn = tile == 256 ? 192 : 128;
@@ -1579,6 +1578,8 @@ extern "C" int intent_w4a16_sym_gemm(const void* x, int64_t M, int64_t K, int64_
                      intent::fits_offset(256 + 1, x_ld * 2),
                  INTENT_ERR_UNSUPPORTED, "w4a16_sym_gemm: operand too large for 31-bit buffer offsets");
   W4SymArgs w{packed, packed_ld, (const f16*)scales, scales_ld};
-  return launch_dense<W4SymArgs, false>((const f16*)x, x_ld, (int)M, (int)N, (int)K, w, (f16*)y, y_ld, nullptr,
-                                        (hipStream_t)stream, kW4SymNames, DensePlan{M > 128 ? 256 : 128, 1});
+  const auto launch = M > 128 ? launch_tile<mp::Tile<256, 192, 2, 2>, W4SymArgs, false>
+                              : launch_tile<mp::Tile<128, 128, 2, 2>, W4SymArgs, false>;
+  return launch((const f16*)x, x_ld, (int)M, (int)N, (int)K, w, (f16*)y, y_ld, nullptr, (hipStream_t)stream,
+                M > 128 ? "w4a16_sym_gemm<256x192>" : "w4a16_sym_gemm<128x128>");
 }
